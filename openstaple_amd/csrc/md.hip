@@ -61,43 +61,15 @@ __global__ __launch_bounds__(kBlock) void k_mom_exp(double2* __restrict__ conf, 
     const int link = gid / sizeh, i = gid - link * sizeh;
     Thmat h;
     th_load(mom, link, sizeh, i, h);
-    // QA = -i delta P in the tamat form: the reference's -P*delta*1.0I
-    Tamat q;
-    q.ic00 = -h.rc00 * delta;
-    q.ic11 = -h.rc11 * delta;
-    q.c01 = make_double2(h.c01.y * delta, -(h.c01.x * delta));
-    q.c02 = make_double2(h.c02.y * delta, -(h.c02.x * delta));
-    q.c12 = make_double2(h.c12.y * delta, -(h.c12.x * delta));
-    Su3 E, U;
-    ch_exp_minus_qa(q, E);
+    Su3 E;
+    exp_ip(h, delta, E);
     double2* Ul = (double2*)((char*)conf + (size_t)link * su3_stride);
+    double2 u[2][3];
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+    for (int e = 0; e < 6; e++) u[e / 3][e % 3] = Ul[(size_t)e * sizeh + i];
+    move_link(E, u);
 #pragma unroll
-        for (int c = 0; c < 3; c++) U.c[r][c] = Ul[(size_t)(3 * r + c) * sizeh + i];
-    rebuild3row(U);
-    double2 o[2][3];
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            double2 s = cmul(E.c[r][0], U.c[0][c]);
-            s = cfma(E.c[r][1], U.c[1][c], s);
-            o[r][c] = cfma(E.c[r][2], U.c[2][c], s);
-        }
-    double n = 1.0 / sqrt(cnorm2(o[0][0]) + cnorm2(o[0][1]) + cnorm2(o[0][2]));
-#pragma unroll
-    for (int c = 0; c < 3; c++) o[0][c] = cscale(o[0][c], n);
-    double2 sp = cmul(cconj(o[0][0]), o[1][0]);
-    sp = cfma(cconj(o[0][1]), o[1][1], sp);
-    sp = cfma(cconj(o[0][2]), o[1][2], sp);
-#pragma unroll
-    for (int c = 0; c < 3; c++) o[1][c] = csub(o[1][c], cmul(sp, o[0][c]));
-    n = 1.0 / sqrt(cnorm2(o[1][0]) + cnorm2(o[1][1]) + cnorm2(o[1][2]));
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int c = 0; c < 3; c++) Ul[(size_t)(3 * r + c) * sizeh + i] = r == 0 ? o[0][c] : cscale(o[1][c], n);
+    for (int e = 0; e < 6; e++) Ul[(size_t)e * sizeh + i] = u[e / 3][e % 3];
 }
 
 // sum over the links [first, first + nlinks) of half_tr_thmat_squared = Tr(P^2)/2
@@ -158,20 +130,33 @@ bool launch_invert_momenta(void* mom) {
     return hip_ok(hipGetLastError(), "k_negate");
 }
 
-// one gauge sub-step of multistep_2MN_gauge_bloc (md_integrator.c:256-345):
-// P -= i deltas[idx] TA(U S) fused with the force, then U <- exp(i deltas[4] P) U
-static bool gauge_bloc(void* u, void* ipdot, void* mom, int idx) {
-    return launch_gauge_force(u, nullptr, ipdot, mom, deltas_Omelyan[idx]) && launch_mom_exp(u, mom, deltas_Omelyan[4]);
-}
+// the plane kernels of the gauge force (stout.hip)
+bool gf_planes_ready();
+bool gf_pack(const void* u);
+bool gf_unpack(void* u);
+bool gf_parts(const void* u, void* stap);
+bool gf_ipdot(void* ipdot, void* mom, double fact);
+bool gf_move(void* mom, double fact, double delta);
 
-// multistep_2MN_gauge (md_integrator.c:347-376) on device pointers
+// multistep_2MN_gauge (md_integrator.c:256-376) on device pointers.  A
+// sub-step is P -= i deltas[idx] TA(U S), then U <- exp(i deltas[4] P) U.
+// With the plane kernels the links stay in their records between the first
+// and the last force; the momentum step and the link update are one kernel.
 bool md_gauge(void* u, void* stap, void* ipdot, void* mom) {
     const int gs = md_parameters.gauge_scale;
-    if (!gauge_bloc(u, ipdot, mom, 3)) return false;
+    const bool planes = gf_planes_ready();
+    if (planes && !gf_pack(u)) return false;
+    auto bloc = [&](int idx) {
+        if (planes) return gf_parts(u, nullptr) && gf_move(mom, deltas_Omelyan[idx], deltas_Omelyan[4]);
+        return launch_gauge_force(u, nullptr, ipdot, mom, deltas_Omelyan[idx]) &&
+               launch_mom_exp(u, mom, deltas_Omelyan[4]);
+    };
+    if (!bloc(3)) return false;
     for (int md = 1; md < gs; md++)
-        if (!gauge_bloc(u, ipdot, mom, 5) || !gauge_bloc(u, ipdot, mom, 6)) return false;
-    if (!gauge_bloc(u, ipdot, mom, 5)) return false;
+        if (!bloc(5) || !bloc(6)) return false;
+    if (!bloc(5)) return false;
     // the last force also leaves its staples, as calc_ipdot_gauge_soloopenacc does
+    if (planes) return gf_unpack(u) && gf_parts(u, stap) && gf_ipdot(ipdot, mom, deltas_Omelyan[3]);
     return launch_gauge_force(u, stap, ipdot, mom, deltas_Omelyan[3]);
 }
 

@@ -85,6 +85,20 @@ inline T* resolve_as(const void* p, size_t bytes, const char* what) {
     return reinterpret_cast<T*>(resolve(p, bytes, what));
 }
 
+// Device buffer of the library that lives from call to call and is given back
+// by ostp_finalize (release_workspaces) or when another allocation of the
+// library runs out of memory.  try_get grows it, and returns null without
+// recording an error where that would take more than a quarter of the free
+// memory: the caller then takes a path without it.
+struct Workspace {
+    void* p = nullptr;
+    size_t n = 0;
+    Workspace();
+    void* try_get(size_t need);
+    void release();
+};
+void release_workspaces();
+
 // Launch geometry over sizeh half-sites.
 inline int blocks_for(long n, int nt = kBlock) { return (int)((n + nt - 1) / nt); }
 

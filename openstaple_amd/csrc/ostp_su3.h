@@ -274,16 +274,64 @@ __device__ __forceinline__ void th_store(void* base, int link, int sizeh, int i,
 
 // thm -= (i fact) tam on c01, c02, c12; rc00/rc11 += fact ic00/ic11, rounded
 // like the reference's complex product (no fused multiply-add)
-__device__ __forceinline__ void mom_step(void* mom, int link, int sizeh, int i, const Tamat& q, double fact) {
+__device__ __forceinline__ void th_step(Thmat& h, const Tamat& q, double fact) {
 #pragma clang fp contract(off)
-    Thmat h;
-    th_load(mom, link, sizeh, i, h);
     h.c01 = make_double2(h.c01.x + fact * q.c01.y, h.c01.y - fact * q.c01.x);
     h.c02 = make_double2(h.c02.x + fact * q.c02.y, h.c02.y - fact * q.c02.x);
     h.c12 = make_double2(h.c12.x + fact * q.c12.y, h.c12.y - fact * q.c12.x);
     h.rc00 = h.rc00 + fact * q.ic00;
     h.rc11 = h.rc11 + fact * q.ic11;
+}
+__device__ __forceinline__ void mom_step(void* mom, int link, int sizeh, int i, const Tamat& q, double fact) {
+    Thmat h;
+    th_load(mom, link, sizeh, i, h);
+    th_step(h, q, fact);
     th_store(mom, link, sizeh, i, h);
+}
+
+// rows 0,1 of exp(i delta P)
+__device__ __forceinline__ void exp_ip(const Thmat& h, double delta, Su3& E) {
+    // QA = -i delta P in the tamat form: the reference's -P*delta*1.0I
+    Tamat q;
+    q.ic00 = -h.rc00 * delta;
+    q.ic11 = -h.rc11 * delta;
+    q.c01 = make_double2(h.c01.y * delta, -(h.c01.x * delta));
+    q.c02 = make_double2(h.c02.y * delta, -(h.c02.x * delta));
+    q.c12 = make_double2(h.c12.y * delta, -(h.c12.x * delta));
+    ch_exp_minus_qa(q, E);
+}
+// rows 0,1 of a link: U <- E U, then re-unitarised (row 0 normalised, row 1
+// orthogonalised to it and normalised)
+__device__ __forceinline__ void move_link(const Su3& E, double2 (&u)[2][3]) {
+    Su3 U;
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) U.c[r][c] = u[r][c];
+    rebuild3row(U);
+    double2 o[2][3];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            double2 s = cmul(E.c[r][0], U.c[0][c]);
+            s = cfma(E.c[r][1], U.c[1][c], s);
+            o[r][c] = cfma(E.c[r][2], U.c[2][c], s);
+        }
+    double n = 1.0 / sqrt(cnorm2(o[0][0]) + cnorm2(o[0][1]) + cnorm2(o[0][2]));
+#pragma unroll
+    for (int c = 0; c < 3; c++) o[0][c] = cscale(o[0][c], n);
+    double2 sp = cmul(cconj(o[0][0]), o[1][0]);
+    sp = cfma(cconj(o[0][1]), o[1][1], sp);
+    sp = cfma(cconj(o[0][2]), o[1][2], sp);
+#pragma unroll
+    for (int c = 0; c < 3; c++) o[1][c] = csub(o[1][c], cmul(sp, o[0][c]));
+    n = 1.0 / sqrt(cnorm2(o[1][0]) + cnorm2(o[1][1]) + cnorm2(o[1][2]));
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        u[0][c] = o[0][c];
+        u[1][c] = cscale(o[1][c], n);
+    }
 }
 
 }  // namespace ostp

@@ -9,6 +9,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <vector>
 
 // ------------------------------------------------------- reference globals
 // Defaults of Include/setting_file_parser.c:462,490-492; a host program that
@@ -135,6 +136,46 @@ bool push_state() {
     return hip_ok(hipStreamSynchronize(g_ctx.stream), "stream synchronize");
 }
 
+static std::vector<Workspace*>& workspaces() {
+    static std::vector<Workspace*> v;
+    return v;
+}
+Workspace::Workspace() { workspaces().push_back(this); }
+void* Workspace::try_get(size_t need) {
+    if (n >= need) return p;
+    release();
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || need > free_b / 4 || hipMalloc(&p, need) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        return nullptr;
+    }
+    n = need;
+    return p;
+}
+void Workspace::release() {
+    if (p) {
+        if (g_ctx.stream) (void)hipStreamSynchronize(g_ctx.stream);
+        (void)hipFree(p);
+    }
+    p = nullptr;
+    n = 0;
+}
+void release_workspaces() {
+    for (Workspace* w : workspaces()) w->release();
+}
+
+// hipMalloc for the callers' memory; the library's workspaces make room for it
+static hipError_t malloc_for_caller(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        release_workspaces();
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 static void release_scratch() {
     if (g_ctx.partials) (void)hipFree(g_ctx.partials);
     if (g_ctx.state) (void)hipFree(g_ctx.state);
@@ -197,6 +238,7 @@ void ostp_finalize(void) {
     for (auto& kv : g_map) (void)hipFree(kv.second.dev);
     g_map.clear();
     release_scratch();
+    release_workspaces();
     for (auto& e : g_timer) {
         if (e) (void)hipEventDestroy(e);
         e = nullptr;
@@ -248,7 +290,7 @@ int ostp_acc_create(void* host, size_t bytes) {
     if (it != g_map.end() && it->first < a + bytes)
         return fail("ostp_acc_create: range overlaps a present region") ? 0 : 1;
     void* dev = nullptr;
-    hipError_t e = hipMalloc(&dev, bytes);
+    hipError_t e = malloc_for_caller(&dev, bytes);
     if (e != hipSuccess) return hip_ok(e, "ostp_acc_create hipMalloc") ? 0 : 1;
     g_map[a] = Mapping{bytes, dev, 1};
     return 0;
@@ -314,7 +356,7 @@ int ostp_acc_is_present(const void* host, size_t bytes) {
 
 void* ostp_malloc(size_t bytes) {
     void* p = nullptr;
-    if (!hip_ok(hipMalloc(&p, bytes), "ostp_malloc")) return nullptr;
+    if (!hip_ok(malloc_for_caller(&p, bytes), "ostp_malloc")) return nullptr;
     return p;
 }
 

@@ -14,6 +14,7 @@
 #include "ostp_blas.h"
 #include "ostp_su3.h"
 
+#include <algorithm>
 #include <cmath>
 
 extern "C" {
@@ -280,25 +281,6 @@ __device__ __forceinline__ void pc_link(const PlaneCtx& c, int which, int a, int
     rebuild3row(m);
 }
 
-// The plane kernel's link source: rows 0,1 and K of the links of a tile of
-// the plane (mu, nu) with a two-site halo, in LDS.  Region site (i, j) is
-// tile site (i - 2, j - 2) (i along mu, j along nu); slot d ns / 2 + j rw + i
-// holds its link along mu (d = 0) or nu (d = 1), so that lanes on
-// consecutive sites read consecutive 16-B entries.  A staple term of a link
-// along mu takes offsets a (along mu) and b (along nu) as in PlaneCtx; for a
-// link along nu (own = 1) the roles of the two directions swap.
-struct LdsTile {
-    const double2* e;  // 6 arrays of ns entries: row r, column c at (3 r + c) ns
-    const double* k;   // ns entries
-    int ns, rw;
-    int i0, j0;        // region coordinates of the link's site
-    int own;
-};
-__device__ __forceinline__ int lt_slot(const LdsTile& c, int which, int a, int b) {
-    const int di = c.own ? b : a, dj = c.own ? a : b;
-    return (c.own ? 1 - which : which) * (c.ns >> 1) + (c.j0 + dj) * c.rw + (c.i0 + di);
-}
-
 // rows 0,1 (src_link2) or all rows (src_link) of a staple term's link and its K
 __device__ __forceinline__ void src_link2(const PlaneCtx& c, int which, int a, int b, int pt, Su3& m, double& k) {
     pc_link2(c, which, a, b, pt, m, k);
@@ -306,19 +288,6 @@ __device__ __forceinline__ void src_link2(const PlaneCtx& c, int which, int a, i
 __device__ __forceinline__ void src_link(const PlaneCtx& c, int which, int a, int b, int pt, Su3& m, double& k) {
     pc_link(c, which, a, b, pt, m, k);
 }
-__device__ __forceinline__ void src_link2(const LdsTile& c, int which, int a, int b, int pt, Su3& m, double& k) {
-    const int s = lt_slot(c, which, a, b);
-#pragma unroll
-    for (int r = 0; r < 2; r++)
-#pragma unroll
-        for (int col = 0; col < 3; col++) m.c[r][col] = c.e[(3 * r + col) * c.ns + s];
-    k = pt ? c.k[s] : 1.0;
-}
-__device__ __forceinline__ void src_link(const LdsTile& c, int which, int a, int b, int pt, Su3& m, double& k) {
-    src_link2(c, which, a, b, pt, m, k);
-    rebuild3row(m);
-}
-
 // Each term is a chain of SU(3) products that carries only rows 0,1 and
 // rebuilds row 2 at the end.  MMMPP is formed as its conjugate
 // m5^+ m4^+ m3 m2 m1, a chain of the same kind, and added transposed.
@@ -616,150 +585,592 @@ __global__ __launch_bounds__(3 * kGfLinks, 2) void k_gauge_force(GaugePtrs G, do
     }
 }
 
-// Gauge force by planes: one launch per plane (mu, nu), mu < nu, in the order
-// (0,1) (0,2) (0,3) (1,2) (1,3) (2,3).  A block takes a TM x TN tile of the
-// plane at fixed coordinates along the other two directions, loads rows 0,1
-// and K of the tile's links along mu and nu with a two-site halo into LDS
-// (every staple term of the plane stays within it), and forms the plane's
-// terms for the tile's links along mu and along nu, one side of the plane
-// per thread, with every link operand read from LDS (the per-link kernel
-// above fetches 84 links per link from L2).  TA(U S) is linear, so a plane
-// adds K(x, d) TA(U S_plane) to ipdot (the first plane of a direction
-// stores it) and the last plane of a direction applies the momentum step
-// with the sum.  Blocks run over the tiles of one (other-coordinate) slice
-// fastest, so that an XCD's consecutive tiles share their halos in its L2.
+// Gauge force by planes.  TA(U S) is linear, so every plane (mu, nu) forms
+// its own part TA(U S_plane) of its two directions' links, in a buffer of
+// its own (three planes per direction), and the kernels that consume the
+// force add the three parts.
+//
+// A block takes tm x tn tiles (at most 64 sites, one lane each) of a plane at
+// fixed coordinates along the other two directions.  Within a tile every
+// product that several links need is formed once, in LDS.  With M = U_mu and
+// N = U_nu:
+//   corners            Cm(y) = M(y) N(y+mu),             Cn(y) = N(y) M(y+nu)
+//   plaquette staples  SM+(y) = N(y+mu) Cn(y)^+,         SM-(y) = Cm(y-nu)^+ N(y-nu)     (of M)
+//                      SN+(y) = M(y+nu) Cm(y)^+,         SN-(y) = Cn(y-mu)^+ M(y-mu)     (of N)
+// A rectangle's staple is a plaquette staple with one link replaced by that
+// link's own plaquette staple on the far side, so one side of a link O
+// (direction o, the plane's other direction p, links P) is four products:
+//   up:   (c0 P(x+o) + c1 SP+(x+o)^+) Cp(x)^+ + c1 P(x+o) [SO+(x+p) P(x)^+ + O(x+p)^+ SP-(x)]
+//   down: Co(x-p)^+ (c0 P(x-p) + c1 SP-(x-p)^+) + c1 [P(x+o-p)^+ SO-(x-p) + SP+(x+o-p) O(x-p)^+] P(x-p)
+// A wave takes one side of one direction's links (its roles, and so the
+// arrays, are wave-uniform).
+//
+// The links come from a copy in records (rows 0,1 of a link, 96 B), so that a
+// tile's loads use whole sectors in every plane: with the field's colour
+// planes, a plane without direction 0 fetches a 128-B line per 16-B entry
+// (67 M requests per plane at 48^3x12, 12 TB/s from the L2).  The blocks are
+// persistent and hold the next tile's links in registers while they work on
+// the current one.
+//
+// Bound by FP64 issue and the latency between a tile's phases: 1116 vector
+// instructions a wave and tile (1551 with every operand's address formed from
+// the plan, 2900 for the term-by-term sides), 52% of the issue slots at the
+// 2.1 GHz the card holds; LDS and two blocks per CU leave two waves per SIMD.
+// 48^3x12: 1.85 ms per force, 2.4 ms with the records' and the force's passes
+// (term-by-term sides, six launches: 3.1 ms); gauge sub-integrator 38.8 -> 28
+// ms.  Tried and slower: summing the sides of both directions in two waves
+// that the second staple pass spares (more exchange through LDS, 2.0 ms).
+// Entry e (of six: rows 0, 1) of the LDS arrays' record r is pool[e kGfPool +
+// r]: an operand's six reads share one address with constant offsets, and
+// sixteen lanes on consecutive sites read all 64 banks once, so that tiles
+// with rows of 16 sites meet no bank conflicts (records of 96 B: 2.2 times the
+// LDS cycles).
+struct GfArr {
+    int off, n, rw, org;  // record of site (i, j): off + j rw + i - org
+    int inv;              // 65536 / rw, rounded up: q / rw = q inv >> 16 for q < 512
+};
+enum GfRole : int { gM = 0, gN, gCm, gCn, gSMp, gSMm, gSNp, gSNm, gRoles };
+struct GfPlan {
+    int mu, nu, tm, tn, tiles_m, tiles_n, tiles, inv_tm;
+    GfArr a[gRoles];
+};
+struct GfPlans {
+    int tiles[8];  // of each plane (p[k].tiles)
+    GfPlan p[6];
+};
+// records and K values of the largest tile (16 x 4): 81,632 B with K, so that two blocks fit a CU
+constexpr int kGfPool = 826;
+constexpr int kGfPoolLinks = 292;
+constexpr int kGfFetch = 4;  // links per thread: 85 triples of lanes, two 16-B entries a lane
+// part of plane (d, other) in direction d's three buffers
+__device__ __forceinline__ int gf_slot(int d, int other) { return other - (other > d ? 1 : 0); }
+
 __device__ __forceinline__ int sel4(int k, int v0, int v1, int v2, int v3) {
     return k == 0 ? v0 : k == 1 ? v1 : k == 2 ? v2 : v3;
 }
-template <int TM, int TN>
-__global__ __launch_bounds__(4 * TM * TN, 2) void k_gf_plane(GaugePtrs G, double2* __restrict__ stap,
-                                                             size_t su3_stride, void* __restrict__ ipdot,
-                                                             void* __restrict__ mom, LinkGeom g, int mu, int nu,
-                                                             int pt, int tlsm, double c0, double fact, int flags) {
-    constexpr int RW = TM + 4, RH = TN + 4, NS = 2 * RW * RH, NT = TM * TN;
-    __shared__ double2 le[6][NS];
-    __shared__ double lk[NS];
-    __shared__ double accl[18][4 * NT];  // each thread's side sum (keeps 36 registers free)
-    const int oa = (mu != 0 && nu != 0) ? 0 : ((mu != 1 && nu != 1) ? 1 : 2);  // the other two directions
+// rows 0,1 (gf_load2) or all rows (gf_load) of a record in LDS
+__device__ __forceinline__ void gf_load2(const double2* e, Su3& m) {
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) m.c[r][c] = e[(3 * r + c) * kGfPool];
+}
+__device__ __forceinline__ void gf_load(const double2* e, Su3& m) {
+    gf_load2(e, m);
+    rebuild3row(m);
+}
+__device__ __forceinline__ void gf_store2(double2* e, const Su3& m) {
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) e[(3 * r + c) * kGfPool] = m.c[r][c];
+}
+// acc = s m, acc += s m^+
+__device__ __forceinline__ void su3_scale(double s, const Su3& m, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) acc.c[r][c] = cscale(m.c[r][c], s);
+}
+__device__ __forceinline__ void axpy3_dag(double s, const Su3& m, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            acc.c[r][c] = make_double2(fma(s, m.c[c][r].x, acc.c[r][c].x), fma(-s, m.c[c][r].y, acc.c[r][c].y));
+}
+// acc += a b ; a b^+ ; a^+ b
+__device__ __forceinline__ void su3_mul_add(const Su3& a, const Su3& b, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            acc.c[r][c] = cfma(a.c[r][2], b.c[2][c], cfma(a.c[r][1], b.c[1][c], cfma(a.c[r][0], b.c[0][c], acc.c[r][c])));
+}
+__device__ __forceinline__ void su3_mul_dag_add(const Su3& a, const Su3& b, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            acc.c[r][c] = cfma(a.c[r][2], cconj(b.c[c][2]),
+                               cfma(a.c[r][1], cconj(b.c[c][1]), cfma(a.c[r][0], cconj(b.c[c][0]), acc.c[r][c])));
+}
+__device__ __forceinline__ void su3_dag_mul_add(const Su3& a, const Su3& b, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+            acc.c[r][c] = cfmac(a.c[2][r], b.c[2][c], cfmac(a.c[1][r], b.c[1][c], cfmac(a.c[0][r], b.c[0][c], acc.c[r][c])));
+}
+
+// A plan's numbers in scalar registers.  The readfirstlane keeps the compiler
+// from turning a per-lane choice between two of them into a per-lane load
+// from the kernel arguments, a memory round trip each (3.3 -> 2.6 ms per force
+// at 48^3x12).
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ GfArr uni(const GfArr& a) {
+    return GfArr{uni(a.off), uni(a.n), uni(a.rw), uni(a.org), uni(a.inv)};
+}
+// The force parts of one plane (mu, nu) are records of four 16-B entries (c01,
+// c02, c12, (ic00, ic11)) at part[((slot 8 + link array) sizeh + site) 4].
+template <bool PT>
+__global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ rec, GaugePtrs G,
+                                                    double2* __restrict__ stap, size_t su3_stride,
+                                                    double2* __restrict__ part, LinkGeom g, GfPlans plans, int p0,
+                                                    int p1, int tlsm, double c0) {
+    __shared__ double2 pool[6 * kGfPool];
+    __shared__ double lk[PT ? kGfPoolLinks : 1];
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int w = uni(tid >> 6), dsel = w >> 1, side = w & 1;
     const int nd0 = g.nd[0], nd1 = g.nd[1], nd2 = g.nd[2], nd3 = g.nd[3];
-    const int ndm = sel4(mu, nd0, nd1, nd2, nd3), ndn = sel4(nu, nd0, nd1, nd2, nd3);
-    const int nda = sel4(oa, nd0, nd1, nd2, nd3);
-    // block -> tile.  Consecutive blocks (the same XCD) take neighbouring
-    // tiles: along mu, then nu, then the slice when the plane holds direction
-    // 0; otherwise direction 0 (which the half-site index runs along, so a
-    // 128-B line holds 16 consecutive x of one parity) fastest, so that the
-    // blocks sharing the lines of a tile's links and ipdot run together and
-    // the lines are fetched once into the XCD's L2.
-    int r = xcd_block_id();
-    const int tiles_m = ndm / TM, tiles_n = ndn / TN;
-    int tm, tn, xa, xb;
-    if (mu == 0) {
-        tm = r % tiles_m;
-        r /= tiles_m;
-        tn = r % tiles_n;
-        r /= tiles_n;
-        xa = r % nda;
-        xb = r / nda;
-    } else {
-        xa = r % nda;  // oa == 0
-        r /= nda;
-        tm = r % tiles_m;
-        r /= tiles_m;
-        tn = r % tiles_n;
-        xb = r / tiles_n;
-    }
-    int o[4];
+    const int st1 = nd0, st2 = nd0 * nd1, st3 = st2 * nd2;
+    const unsigned rec_stride = 96u * (unsigned)g.sizeh;
+    // Every XCD takes a contiguous eighth of each plane's tiles, and each of its
+    // blocks (hardware ids round-robin over the XCDs) a contiguous run of those:
+    // a block sets a plane up once and re-reads its tiles' halos from the L2.
+    const int xcd = (int)blockIdx.x & 7, nbx = ((int)gridDim.x - xcd + 7) >> 3, bx = (int)blockIdx.x >> 3;
+    auto share = [](int tiles, int x) { return (tiles >> 3) * x + ((tiles & 7) * x >> 3); };
+    int total = 0;
 #pragma unroll
-    for (int k = 0; k < 4; k++) o[k] = k == mu ? tm * TM : k == nu ? tn * TN : k == oa ? xa : xb;
-    // links of the region into LDS
-    for (int s = threadIdx.x; s < NS; s += 4 * NT) {
-        const int d = s >= NS / 2, site = s - d * (NS / 2), i = site % RW, j = site / RW;
-        int y[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int n = sel4(k, nd0, nd1, nd2, nd3);
-            int v = o[k] + (k == mu ? i - 2 : 0) + (k == nu ? j - 2 : 0);
-            v += v < 0 ? n : 0;
-            v -= v >= n ? n : 0;
-            y[k] = v;
+    for (int p = 0; p < 6; p++)
+        if (p >= p0 && p < p1) total += share(plans.tiles[p], xcd + 1) - share(plans.tiles[p], xcd);
+    const int each = total / nbx, rest = total - each * nbx;
+    int q = each * bx + min(bx, rest), left = each + (bx < rest ? 1 : 0);
+    for (int p = p0; p < p1 && left > 0; p++) {
+        const GfPlan& pl = plans.p[p];
+        const int tiles = uni(pl.tiles), base = share(tiles, xcd), count = share(tiles, xcd + 1) - base;
+        if (q >= count) {
+            q -= count;
+            continue;
         }
-        const int lex = y[0] + nd0 * (y[1] + nd1 * (y[2] + nd2 * y[3]));
-        const int arr = 2 * (d ? nu : mu) + ((y[0] + y[1] + y[2] + y[3]) & 1);
-        const double2* U = G.at(arr);
-        const size_t h = (size_t)(lex >> 1);
+        const int end = min(count, q + left);  // this plane's tiles [q, end)
+        left -= end - q;
+        const int mu = uni(pl.mu), nu = uni(pl.nu), TM = uni(pl.tm), TN = uni(pl.tn);
+        const int tiles_m = uni(pl.tiles_m), tiles_n = uni(pl.tiles_n);
+        const int oa = (mu != 0 && nu != 0) ? 0 : ((mu != 1 && nu != 1) ? 1 : 2), ob = 6 - mu - nu - oa;
+        const int nda = sel4(oa, nd0, nd1, nd2, nd3), ndm = sel4(mu, nd0, nd1, nd2, nd3), ndn = sel4(nu, nd0, nd1, nd2, nd3);
+        const int sa = sel4(oa, 1, st1, st2, st3), sb = sel4(ob, 1, st1, st2, st3);
+        const int sm = sel4(mu, 1, st1, st2, st3), sn = sel4(nu, 1, st1, st2, st3);
+        const GfArr M = uni(pl.a[gM]), N = uni(pl.a[gN]), Cm = uni(pl.a[gCm]), Cn = uni(pl.a[gCn]);
+        const GfArr SMp = uni(pl.a[gSMp]), SMm = uni(pl.a[gSMm]), SNp = uni(pl.a[gSNp]), SNm = uni(pl.a[gSNm]);
+        const int nL = M.n + N.n;
+
+        // What depends on the plane alone: this thread's links of the tile and
+        // its halo, and the records (pool indices) of its corner and staples.
+        int li[kGfFetch];  // i, j (+2) and direction of the link
+        auto link_pos = [&](int s) {
+            const bool d = s >= M.n;
+            const int r = d ? s - M.n : s;
+            const int j = (r * (d ? N.inv : M.inv)) >> 16, i = r - j * (d ? N.rw : M.rw);
+            return i | j << 8 | (d ? 1 << 16 : 0);
+        };
+        const int ltri = tid / 3, lpart = 2 * (tid - 3 * ltri);
 #pragma unroll
-        for (int q = 0; q < 6; q++) le[q][s] = U[(size_t)q * g.sizeh + h];
-        lk[s] = pt ? ((const double*)(U + (size_t)9 * g.sizeh))[h] : 1.0;
+        for (int k = 0; k < kGfFetch; k++) li[k] = link_pos(min(ltri + 85 * k, nL - 1));
+        int cA, cB, cO;
+        {
+            const int s = min(tid, Cm.n + Cn.n - 1);
+            const bool d = s >= Cm.n;
+            const int r = d ? s - Cm.n : s;
+            const int jj = (r * Cm.inv) >> 16, ii = r - jj * Cm.rw;  // Cn has Cm's shape
+            const int i = ii - (d ? 2 : 1), j = jj - (d ? 1 : 2);
+            const int rM = M.off + (j + (d ? 1 : 0)) * M.rw + i - M.org, rN = N.off + j * N.rw + i + (d ? 0 : 1) - N.org;
+            cA = (d ? rN : rM);
+            cB = (d ? rM : rN);
+            cO = ((d ? Cn.off : Cm.off) + r);
+        }
+        // staples: link x corner^+ (SM+, SN+) first, then corner^+ x link (SM-, SN-) from a whole wave on
+        const int np = SMp.n + SNp.n, p64 = (np + 63) & ~63, ns = p64 + SMm.n + SNm.n;
+        int sA[2], sC[2], sO[2];
+        auto item = [&](int k) { return tid + 256 * k; };
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const int s = item(k);
+            if (s < p64) {
+                const int e = min(s, np - 1);
+                const bool d = e >= SMp.n;
+                const int r = d ? e - SMp.n : e;
+                const int jj = (r * (d ? SNp.inv : SMp.inv)) >> 16, ii = r - jj * (d ? SNp.rw : SMp.rw);
+                const int i = ii + (d ? 1 : -1), j = jj + (d ? -1 : 1);
+                sA[k] = (d ? M.off + (j + 1) * M.rw + i - M.org : N.off + j * N.rw + i + 1 - N.org);
+                sC[k] = (d ? Cm.off + j * Cm.rw + i - Cm.org : Cn.off + j * Cn.rw + i - Cn.org);
+                sO[k] = ((d ? SNp.off : SMp.off) + r);
+            } else {
+                const int e = min(s, ns - 1) - p64;
+                const bool d = e >= SMm.n;
+                const int r = d ? e - SMm.n : e;
+                const int jj = (r * SMm.inv) >> 16, ii = r - jj * SMm.rw;  // SN- has SM-'s shape
+                const int i = ii - 1 - (d ? 1 : 0), j = jj - 1 - (d ? 0 : 1);  // the plaquette's own site
+                sA[k] = (d ? M.off + j * M.rw + i - M.org : N.off + j * N.rw + i - N.org);
+                sC[k] = (d ? Cn.off + j * Cn.rw + i - Cn.org : Cm.off + j * Cm.rw + i - Cm.org);
+                sO[k] = ((d ? SNm.off : SMm.off) + r);
+            }
+        }
+        const int inv_tm = uni(pl.inv_tm);
+        const int jn = (lane * inv_tm) >> 16, im = lane - jn * TM;
+        const bool inside = lane < TM * TN;
+
+        // tile r of the plane: its corner (om, on) and the sites' constant part.
+        // Consecutive tiles are neighbours along mu, then nu; in a plane without
+        // direction 0 the tiles of consecutive x, which share the records' lines,
+        // follow each other.
+        struct Tile {
+            int om, on, xa, xb;
+        };
+        auto place = [&](int r) {
+            int tm, tn, xa, xb;
+            if (mu == 0) {
+                tm = r % tiles_m;
+                r /= tiles_m;
+                tn = r % tiles_n;
+                r /= tiles_n;
+                xa = r % nda;
+                xb = r / nda;
+            } else {
+                xa = r % nda;
+                r /= nda;
+                tm = r % tiles_m;
+                r /= tiles_m;
+                tn = r % tiles_n;
+                xb = r / tiles_n;
+            }
+            return Tile{tm * TM, tn * TN, xa, xb};
+        };
+        auto advance = [&](Tile t) {  // the tile after t
+            auto up = [](int& v, int step, int n) {
+                v += step;
+                if (v < n) return false;
+                v = 0;
+                return true;
+            };
+            if (mu == 0) {
+                if (up(t.om, TM, ndm) && up(t.on, TN, ndn) && up(t.xa, 1, nda)) t.xb++;
+            } else {
+                if (up(t.xa, 1, nda) && up(t.om, TM, ndm) && up(t.on, TN, ndn)) t.xb++;
+            }
+            return t;
+        };
+        // link array (0..7) and half-site of a link; a tile that reaches past the lattice's end wraps (its
+        // lanes there write nothing).  The unsigned minimum picks the wrapped coordinate.
+        auto link_at = [&](const Tile& t, int l, int& arr, int& h) {
+            unsigned ym = (unsigned)(t.om - 2 + (l & 255)), yn = (unsigned)(t.on - 2 + ((l >> 8) & 255));
+            ym = min(ym, ym + (unsigned)ndm);
+            ym = min(ym, ym - (unsigned)ndm);
+            yn = min(yn, yn + (unsigned)ndn);
+            yn = min(yn, yn - (unsigned)ndn);
+            arr = 2 * (l >> 16 ? nu : mu) + (int)((unsigned)(t.xa + t.xb) + ym + yn & 1u);
+            h = (int)((unsigned)(t.xa * sa + t.xb * sb) + __umul24(ym, sm) + __umul24(yn, sn)) >> 1;
+        };
+        ostp_dvec2 pre[2 * kGfFetch];
+        double prek[kGfFetch];
+        auto fetch = [&](const Tile& t) {
+#pragma unroll
+            for (int k = 0; k < kGfFetch; k++) {
+                int arr, h;
+                link_at(t, li[k], arr, h);
+                // 32-bit offset within the link array (96 sizeh < 2^32)
+                const ostp_dvec2* R = (const ostp_dvec2*)((const char*)rec + (size_t)((unsigned)arr) * rec_stride +
+                                                          (unsigned)(h * 96 + lpart * 16));
+                pre[2 * k] = R[0];
+                pre[2 * k + 1] = R[1];
+                if (PT) prek[k] = ((const double*)(G.at(arr) + (size_t)9 * g.sizeh))[h];
+            }
+        };
+        Tile t = place(base + q);
+        fetch(t);
+        for (;;) {
+#pragma unroll
+            for (int k = 0; k < kGfFetch; k++)
+                if (tid < 255 && ltri + 85 * k < nL) {
+                    ostp_dvec2* e = (ostp_dvec2*)(pool + lpart * kGfPool + ltri + 85 * k);
+                    e[0] = pre[2 * k];
+                    e[kGfPool] = pre[2 * k + 1];
+                    if (PT && lpart == 0) lk[ltri + 85 * k] = prek[k];
+                }
+            __syncthreads();
+            if (tid < Cm.n + Cn.n) {
+                Su3 A, B;
+                gf_load2(pool + cA, A);
+                gf_load(pool + cB, B);
+                mul_r2(A, B, A);
+                gf_store2(pool + cO, A);
+            }
+            __syncthreads();
+            // the next tile's links, while this one is worked on
+            const bool more = q + 1 < end;
+            Tile tn = t;
+            if (more) {
+                tn = advance(t);
+                fetch(tn);
+            }
+            if (tlsm) {
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int s = item(k);
+                    if (s < np) {
+                        Su3 A, C;
+                        gf_load2(pool + sA[k], A);
+                        gf_load(pool + sC[k], C);
+                        mul_dag_r2(A, C, A);
+                        gf_store2(pool + sO[k], A);
+                    } else if (s >= p64 && s < ns) {
+                        Su3 A, C, X;
+                        gf_load(pool + sA[k], A);
+                        gf_load(pool + sC[k], C);
+                        dag_mul_r2(C, A, X);
+                        gf_store2(pool + sO[k], X);
+                    }
+                }
+                __syncthreads();
+            }
+            // one side of one direction's links per wave
+            const bool live = inside && t.om + im < ndm && t.on + jn < ndn;
+            auto pick = [&](const GfArr& a, const GfArr& b) {  // dsel ? b : a, in scalar registers
+                return GfArr{uni(dsel ? b.off : a.off), 0, uni(dsel ? b.rw : a.rw), uni(dsel ? b.org : a.org), 0};
+            };
+            const GfArr aO = pick(M, N), aP = pick(N, M);
+            const GfArr aC = side ? pick(Cm, Cn) : pick(Cn, Cm);  // Co down, Cp up
+            const GfArr aSO = side ? pick(SMm, SNm) : pick(SMp, SNp), aSPp = pick(SNp, SMp), aSPm = pick(SNm, SMm);
+            // record of x + do e_o + dp e_p
+            auto at = [&](const GfArr& a, int dO, int dP) {
+                const int di = dsel ? dP : dO, dj = dsel ? dO : dP;
+                return (jn * a.rw + im) + (a.off + dj * a.rw + di - a.org);
+            };
+            auto ld = [&](const GfArr& a, int dO, int dP, Su3& m) { gf_load(pool + at(a, dO, dP), m); };
+            auto ld2 = [&](const GfArr& a, int dO, int dP, Su3& m) { gf_load2(pool + at(a, dO, dP), m); };
+            auto kO = [&](int dO, int dP) { return PT ? lk[at(aO, dO, dP)] : 1.0; };
+            auto kP = [&](int dO, int dP) { return PT ? lk[at(aP, dO, dP)] : 1.0; };
+            Su3 T;
+            if (live) {
+                Su3 A, B;
+                if (side == 0) {
+                    const double ka = kP(1, 0), kc = kP(0, 0) * kO(0, 1);
+                    ld(aP, 1, 0, A);
+                    if (tlsm) {
+                        Su3 X, W;
+                        ld2(aSO, 0, 1, X);
+                        ld(aP, 0, 0, B);
+                        mul_dag_r2(X, B, X);
+                        rebuild3row(X);
+                        su3_scale(kCOne * ka * kP(1, 1) * kO(0, 2) * kP(0, 1) * kP(0, 0), X, W);
+                        ld(aO, 0, 1, B);
+                        Su3 Y;
+                        ld(aSPm, 0, 0, Y);
+                        dag_mul_r2(B, Y, X);
+                        rebuild3row(X);
+                        axpy3(kCOne * ka * kO(0, 1) * kP(-1, 0) * kO(-1, 1) * kO(-1, 0), X, W);
+                        su3_mul(A, W, T);
+                        su3_scale(c0 * ka * kc, A, A);
+                        ld(aSPp, 1, 0, B);
+                        axpy3_dag(kCOne * kc * kO(1, 1) * kP(2, 0) * kO(1, 0), B, A);
+                        ld(aC, 0, 0, B);
+                        su3_mul_dag_add(A, B, T);
+                    } else {
+                        ld(aC, 0, 0, B);
+                        su3_scale(c0 * ka * kc, A, A);
+                        su3_mul_dag(A, B, T);
+                    }
+                } else {
+                    const double kn = kP(0, -1), kc = kO(0, -1) * kP(1, -1);
+                    ld(aP, 0, -1, A);
+                    if (tlsm) {
+                        Su3 X, Y, W;
+                        ld(aP, 1, -1, B);
+                        ld(aSO, 0, -1, Y);
+                        dag_mul_r2(B, Y, X);
+                        rebuild3row(X);
+                        su3_scale(kCOne * kn * kP(1, -1) * kP(1, -2) * kO(0, -2) * kP(0, -2), X, W);
+                        ld2(aSPp, 1, -1, X);
+                        ld(aO, 0, -1, B);
+                        mul_dag_r2(X, B, X);
+                        rebuild3row(X);
+                        axpy3(kCOne * kn * kO(0, -1) * kO(1, 0) * kP(2, -1) * kO(1, -1), X, W);
+                        su3_mul(W, A, T);
+                        su3_scale(c0 * kc * kn, A, A);
+                        ld(aSPm, 0, -1, B);
+                        axpy3_dag(kCOne * kc * kP(-1, -1) * kO(-1, 0) * kO(-1, -1), B, A);
+                        ld(aC, 0, -1, B);
+                        su3_dag_mul_add(B, A, T);
+                    } else {
+                        ld(aC, 0, -1, B);
+                        su3_scale(c0 * kc * kn, A, A);
+                        su3_dag_mul(B, A, T);
+                    }
+                }
+            }
+            // the lower sides' sums go to the upper sides' threads through the pool past the links
+            // (entries 0-5 of the first 128 records, 0-2 of the next)
+            double2* xch = pool + nL + dsel * 64 + lane;
+            auto xe = [&](int e) -> double2& { return xch[e < 6 ? e * kGfPool : (e - 6) * kGfPool + 128]; };
+            __syncthreads();
+            if (side == 1 && live) {
+#pragma unroll
+                for (int e = 0; e < 9; e++) xe(e) = T.c[e / 3][e % 3];
+            }
+            __syncthreads();
+            double2* out = pool + nL + 256;  // force records of the tile's 2 x 64 links
+            auto site = [&](int i, int j, int d, int& arr, int& h) {
+                const int ym = t.om + i, yn = t.on + j;
+                arr = 2 * (d ? nu : mu) + ((t.xa + t.xb + ym + yn) & 1);
+                h = (t.xa * sa + t.xb * sb + ym * sm + yn * sn) >> 1;
+            };
+            if (side == 0 && live) {
+#pragma unroll
+                for (int e = 0; e < 9; e++) T.c[e / 3][e % 3] = cadd(T.c[e / 3][e % 3], xe(e));
+                Su3 U, X;
+                ld(aO, 0, 0, U);
+                const double ku = kO(0, 0);
+                su3_mul(U, T, X);
+                Tamat f;
+                ta_part(X, ku, f);
+                double2* o = out + dsel * 64 + lane;
+                o[0] = f.c01;
+                o[kGfPool] = f.c02;
+                o[2 * kGfPool] = f.c12;
+                o[3 * kGfPool] = make_double2(f.ic00, f.ic11);
+                if (stap) {
+                    // staples times K(x, d), summed over the planes (calc_ipdot_gauge_soloopenacc's output)
+                    int arr, h;
+                    site(im, jn, dsel, arr, h);
+                    const bool first = gf_slot(dsel ? nu : mu, dsel ? mu : nu) == 0;
+                    double2* O = (double2*)((char*)stap + (size_t)arr * su3_stride) + h;
+#pragma unroll
+                    for (int e = 0; e < 9; e++) {
+                        double2 v = make_double2(ku * T.c[e / 3][e % 3].x, ku * T.c[e / 3][e % 3].y);
+                        if (!first) v = cadd(v, O[(size_t)e * g.sizeh]);
+                        O[(size_t)e * g.sizeh] = v;
+                    }
+                }
+            }
+            __syncthreads();
+            // four lanes write one link's 64-B record
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int l = tid >> 2;
+                const int j = (l * inv_tm) >> 16, i = l - j * TM;
+                if (l < TM * TN && t.om + i < ndm && t.on + j < ndn) {
+                    int arr, h;
+                    site(i, j, k, arr, h);
+                    const int slot = gf_slot(k ? nu : mu, k ? mu : nu);
+                    part[((size_t)(slot * 8 + arr) * g.sizeh + h) * 4 + (tid & 3)] = out[(tid & 3) * kGfPool + 64 * k + l];
+                }
+            }
+            if (!more) break;
+            q++;
+            t = tn;
+        }
+        q = 0;
     }
+}
+
+// records of a block's links through LDS: the field's colour planes and the
+// force parts on one side, whole records with consecutive lanes on the other
+struct GfRecs {
+    double2 u[6 * kBlock];
+};
+// rows 0,1 of every link into records
+__global__ __launch_bounds__(kBlock) void k_gf_pack(GaugePtrs G, double2* __restrict__ rec, int sizeh) {
+    __shared__ GfRecs s;
+    const int l = (int)blockIdx.y, i0 = (int)blockIdx.x * kBlock, t = (int)threadIdx.x;
+    const int n = sizeh - i0 < kBlock ? sizeh - i0 : kBlock;
+    const double2* U = G.at(l) + i0;
+    if (t < n)
+#pragma unroll
+        for (int k = 0; k < 6; k++) s.u[6 * t + k] = U[(size_t)k * sizeh + t];
     __syncthreads();
-    // thread t = (2 dsel + side) NT + item: the link along mu (dsel 0) or nu
-    // (dsel 1) of tile site item, the terms on the upper (side 0) or lower
-    // (side 1) side of the plane
+    double2* R = rec + ((size_t)l * sizeh + i0) * 6;
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+        if (t + k * kBlock < 6 * n) R[t + k * kBlock] = s.u[t + k * kBlock];
+}
+// and back
+__global__ __launch_bounds__(kBlock) void k_gf_unpack(const double2* __restrict__ rec, GaugePtrs G, int sizeh) {
+    __shared__ GfRecs s;
+    const int l = (int)blockIdx.y, i0 = (int)blockIdx.x * kBlock, t = (int)threadIdx.x;
+    const int n = sizeh - i0 < kBlock ? sizeh - i0 : kBlock;
+    const double2* R = rec + ((size_t)l * sizeh + i0) * 6;
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+        if (t + k * kBlock < 6 * n) s.u[t + k * kBlock] = R[t + k * kBlock];
+    __syncthreads();
+    double2* U = const_cast<double2*>(G.at(l)) + i0;
+    if (t < n)
+#pragma unroll
+        for (int k = 0; k < 6; k++) U[(size_t)k * sizeh + t] = s.u[6 * t + k];
+}
+
+// sum of the three planes' parts of the block's links, a link per thread, through the block's LDS
+__device__ __forceinline__ void gf_parts_sum(const double2* __restrict__ part, int sizeh, int l, int i0, int n,
+                                             double2* lds, Tamat& q) {
     const int t = (int)threadIdx.x;
-    const int item = t % NT, w = t / NT;
-    const int dsel = w >> 1, side = w & 1;
-    const int im = item % TM, jn = item / TM;
-    LdsTile src{&le[0][0], lk, NS, RW, im + 2, jn + 2, dsel};
+    const size_t s8 = (size_t)8 * sizeh * 4;
+    const double2* P = part + ((size_t)l * sizeh + i0) * 4;
 #pragma unroll
-    for (int e = 0; e < 18; e++) accl[e][t] = 0.0;
-    plane_side(src, c_side[side], pt, tlsm, c0, [&](double sc, const Su3& T) {
-#pragma unroll
-        for (int rr = 0; rr < 3; rr++)
-#pragma unroll
-            for (int cc = 0; cc < 3; cc++) {
-                const int e = 2 * (3 * rr + cc);
-                accl[e][t] = fma(sc, T.c[rr][cc].x, accl[e][t]);
-                accl[e + 1][t] = fma(sc, T.c[rr][cc].y, accl[e + 1][t]);
-            }
-    });
+    for (int k = 0; k < 4; k++) {
+        const int c = t + k * kBlock;
+        if (c < 4 * n) lds[c] = cadd(cadd(P[c], P[s8 + c]), P[2 * s8 + c]);
+    }
     __syncthreads();
-    if (side != 0) return;
-    // the plane's staple of the link: both sides' sums (the lower side's
-    // thread is t + NT)
-    Su3 S, U, X;
-#pragma unroll
-    for (int rr = 0; rr < 3; rr++)
-#pragma unroll
-        for (int cc = 0; cc < 3; cc++) {
-            const int e = 2 * (3 * rr + cc);
-            S.c[rr][cc] = make_double2(accl[e][t] + accl[e][t + NT], accl[e + 1][t] + accl[e + 1][t + NT]);
-        }
-    double ku;
-    src_link(src, 0, 0, 0, pt, U, ku);
-    su3_mul(U, S, X);
-    Tamat q = {};
-    ta_part(X, ku, q);
-    int y[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) y[k] = o[k] + (k == mu ? im : 0) + (k == nu ? jn : 0);
-    const int lex = y[0] + nd0 * (y[1] + nd1 * (y[2] + nd2 * y[3]));
-    const int arr = 2 * (dsel ? nu : mu) + ((y[0] + y[1] + y[2] + y[3]) & 1);
-    const int idxh = lex >> 1;
-    const int first = flags & (dsel ? 4 : 1), last = flags & (dsel ? 8 : 2);
-    if (!first) {
-        Tamat prev;
-        ta_load(ipdot, arr, g.sizeh, idxh, prev);
-        q.c01 = cadd(q.c01, prev.c01);
-        q.c02 = cadd(q.c02, prev.c02);
-        q.c12 = cadd(q.c12, prev.c12);
-        q.ic00 += prev.ic00;
-        q.ic11 += prev.ic11;
+    if (t < n) {
+        q.c01 = lds[4 * t];
+        q.c02 = lds[4 * t + 1];
+        q.c12 = lds[4 * t + 2];
+        q.ic00 = lds[4 * t + 3].x;
+        q.ic11 = lds[4 * t + 3].y;
     }
-    ta_store(ipdot, arr, g.sizeh, idxh, q);
-    if (last && mom) mom_step(mom, arr, g.sizeh, idxh, q, fact);
-    if (stap) {
-        // staples times K(x, d), summed over the planes (calc_ipdot_gauge_soloopenacc's output)
-        double2* O = (double2*)((char*)stap + (size_t)arr * su3_stride) + idxh;
+}
+
+// ipdot = sum of the planes' parts; with mom, the momentum step of mom_sum_mult (su3_utilities.h:1383-1394)
+__global__ __launch_bounds__(kBlock) void k_gf_ipdot(const double2* __restrict__ part, void* __restrict__ ipdot,
+                                                     void* __restrict__ mom, int sizeh, double fact) {
+    __shared__ double2 lds[4 * kBlock];
+    const int l = (int)blockIdx.y, i0 = (int)blockIdx.x * kBlock, t = (int)threadIdx.x;
+    const int n = sizeh - i0 < kBlock ? sizeh - i0 : kBlock;
+    Tamat q;
+    gf_parts_sum(part, sizeh, l, i0, n, lds, q);
+    if (t >= n) return;
+    ta_store(ipdot, l, sizeh, i0 + t, q);
+    if (mom) mom_step(mom, l, sizeh, i0 + t, q, fact);
+}
+
+// momentum step with the sum of the planes' parts, then U <- exp(i delta P) U
+// on the records.  Memory-bound (512 B per link); every load is issued before
+// the first wait.
+__global__ __launch_bounds__(kBlock) void k_gf_move(const double2* __restrict__ part, void* __restrict__ mom,
+                                                    double2* __restrict__ rec, int sizeh, double fact, double delta) {
+    __shared__ GfRecs s;
+    __shared__ double2 lds[4 * kBlock];
+    const int l = (int)blockIdx.y, i0 = (int)blockIdx.x * kBlock, t = (int)threadIdx.x;
+    const int n = sizeh - i0 < kBlock ? sizeh - i0 : kBlock;
+    double2* R = rec + ((size_t)l * sizeh + i0) * 6;
+    ostp_dvec2 u6[6];
+    Thmat h;
 #pragma unroll
-        for (int rr = 0; rr < 3; rr++)
+    for (int k = 0; k < 6; k++) u6[k] = *(const ostp_dvec2*)(R + min(t + k * kBlock, 6 * n - 1));
+    th_load(mom, l, sizeh, i0 + min(t, n - 1), h);
+    Tamat q;
+    gf_parts_sum(part, sizeh, l, i0, n, lds, q);
 #pragma unroll
-            for (int cc = 0; cc < 3; cc++) {
-                const size_t e = (size_t)(3 * rr + cc) * g.sizeh;
-                double2 v = make_double2(ku * S.c[rr][cc].x, ku * S.c[rr][cc].y);
-                if (!first) v = cadd(v, O[e]);
-                O[e] = v;
-            }
+    for (int k = 0; k < 6; k++) *(ostp_dvec2*)(s.u + t + k * kBlock) = u6[k];
+    Su3 E;
+    if (t < n) {
+        th_step(h, q, fact);
+        th_store(mom, l, sizeh, i0 + t, h);
+        exp_ip(h, delta, E);
     }
+    __syncthreads();
+    if (t < n) {
+        double2 u[2][3];
+#pragma unroll
+        for (int e = 0; e < 6; e++) u[e / 3][e % 3] = s.u[6 * t + e];
+        move_link(E, u);
+#pragma unroll
+        for (int e = 0; e < 6; e++) s.u[6 * t + e] = u[e / 3][e % 3];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 6; k++)
+        if (t + k * kBlock < 6 * n) R[t + k * kBlock] = s.u[t + k * kBlock];
 }
 
 // per site (both parities): sum over the six planes of Re tr of the
@@ -1223,53 +1634,154 @@ bool launch_sigma_chain(void* sigma, void* lam, void* qa, const void* u, double 
     return hip_ok(hipGetLastError(), "k_sigma");
 }
 
-// tile extent of the plane kernel along a direction of extent n (0: none fits)
-static int gf_tile(int n) { return n % 8 == 0 ? 8 : (n % 4 == 0 ? 4 : 0); }
-static int g_gf_planes = 1;  // the plane kernels where the extents allow (0: the per-link kernel)
+static int g_gf_planes = 1;  // the plane kernel (0: the per-link kernel)
 
-template <int TM, int TN>
-static void launch_gf_plane(const void* u, void* stap, void* ipdot, void* mom, int mu, int nu, double fact,
-                            int flags) {
-    const Lattice& L = ctx().lat;
-    int oth = 1;
-    for (int k = 0; k < 4; k++)
-        if (k != mu && k != nu) oth *= L.nd[k];
-    const int nb = (L.nd[mu] / TM) * (L.nd[nu] / TN) * oth;
-    hipLaunchKernelGGL((k_gf_plane<TM, TN>), dim3(nb), dim3(4 * TM * TN), 0, ctx().stream, gauge_ptrs(u),
-                       (double2*)stap, L.su3_bytes(), ipdot, mom, link_geom(), mu, nu, L.par_temp, g_tlsm ? 1 : 0,
-                       g_c_zero, fact, flags);
-}
-
-static bool launch_gauge_force_planes(const void* u, void* stap, void* ipdot, void* mom, double fact) {
-    const Lattice& L = ctx().lat;
-    static const int planes[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
-    int first[4] = {-1, -1, -1, -1}, last[4] = {-1, -1, -1, -1};
-    for (int p = 0; p < 6; p++)
-        for (int e = 0; e < 2; e++) {
-            const int d = planes[p][e];
-            if (first[d] < 0) first[d] = p;
-            last[d] = p;
-        }
-    for (int p = 0; p < 6; p++) {
-        const int mu = planes[p][0], nu = planes[p][1];
-        const int flags = (first[mu] == p ? 1 : 0) | (last[mu] == p ? 2 : 0) | (first[nu] == p ? 4 : 0) |
-                          (last[nu] == p ? 8 : 0);
-        const int tm = gf_tile(L.nd[mu]), tn = gf_tile(L.nd[nu]);
-        if (tm == 8 && tn == 8) launch_gf_plane<8, 8>(u, stap, ipdot, mom, mu, nu, fact, flags);
-        else if (tm == 8) launch_gf_plane<8, 4>(u, stap, ipdot, mom, mu, nu, fact, flags);
-        else if (tn == 8) launch_gf_plane<4, 8>(u, stap, ipdot, mom, mu, nu, fact, flags);
-        else launch_gf_plane<4, 4>(u, stap, ipdot, mom, mu, nu, fact, flags);
+// the LDS arrays of a tm x tn tile; false when they exceed the pool
+static bool gf_plan(int tm, int tn, GfPlan& p) {
+    // first i, j and numbers of sites along i, j of each role (GfRole)
+    const int rng[gRoles][4] = {{-2, -2, tm + 3, tn + 4}, {-2, -2, tm + 4, tn + 3}, {-1, -2, tm + 2, tn + 2},
+                                {-2, -1, tm + 2, tn + 2}, {-1, 1, tm + 1, tn},      {-1, -1, tm + 1, tn + 1},
+                                {1, -1, tm, tn + 1},      {-1, -1, tm + 1, tn + 1}};
+    p.tm = tm;
+    p.tn = tn;
+    p.inv_tm = (65536 + tm - 1) / tm;
+    int off = 0;
+    for (int r = 0; r < gRoles; r++) {
+        GfArr& a = p.a[r];
+        a.off = off;
+        a.rw = rng[r][2];
+        a.n = rng[r][2] * rng[r][3];
+        a.org = rng[r][1] * a.rw + rng[r][0];
+        a.inv = (65536 + a.rw - 1) / a.rw;
+        off += a.n;
     }
-    return hip_ok(hipGetLastError(), "k_gf_plane");
+    // links and corners one pass each, the staples two; the sides' exchange (256 records) and the force
+    // records (128) lie past the links
+    const int nl = p.a[gM].n + p.a[gN].n, np = p.a[gSMp].n + p.a[gSNp].n;
+    return tm * tn <= 64 && off <= kGfPool && nl <= kGfPoolLinks && nl <= 85 * kGfFetch &&
+           p.a[gCm].n + p.a[gCn].n <= 256 && ((np + 63) & ~63) + p.a[gSMm].n + p.a[gSNm].n <= 512 &&
+           nl + 256 + 128 <= kGfPool;
 }
 
+// The tile for a plane of extents nm x nn: the least work per site, counted
+// in complex multiply-adds of the block's waves (corners 24, staples 30, a
+// side 140 and U S with its share of the rest 40 per wave), the links loaded
+// and a fifth on top where the rows are not whole groups of 16 lanes (bank
+// conflicts), over the sites a tile covers on average (a tile that does not
+// divide the extent wastes the lanes past it).
+static GfPlan gf_best_plan(int nm, int nn) {
+    GfPlan best{}, p;
+    double cost = 0.0;
+    for (int tm = 1; tm <= nm && tm <= 64; tm++)
+        for (int tn = 1; tn <= nn && tm * tn <= 64; tn++) {
+            if (!gf_plan(tm, tn, p)) continue;
+            auto waves = [](int n) { return (n + 63) / 64; };
+            const double c = (24.0 * waves(p.a[gCm].n + p.a[gCn].n) +
+                              30.0 * (waves(p.a[gSMp].n + p.a[gSNp].n) + waves(p.a[gSMm].n + p.a[gSNm].n)) +
+                              4.0 * 140.0 + 2.0 * 40.0 + 24.0 * (p.a[gM].n + p.a[gN].n) / 64.0) *
+                             (tm % 16 == 0 ? 1.0 : 1.2);
+            p.tiles_m = (nm + tm - 1) / tm;
+            p.tiles_n = (nn + tn - 1) / tn;
+            if (cost == 0.0 || c * p.tiles_m * p.tiles_n < cost) {
+                cost = c * p.tiles_m * p.tiles_n;
+                best = p;
+            }
+        }
+    return best;
+}
+
+// link records (96 B per link) and the three planes' force parts (3 x 64 B per link) of the current lattice
+static Workspace g_gf_rec, g_gf_part;
+
+struct GfPlanned {
+    int nd[4] = {0, 0, 0, 0};
+    GfPlans plans;
+};
+static const GfPlans& gf_plans() {
+    static const int planes[6][2] = {{0, 1}, {0, 2}, {0, 3}, {1, 2}, {1, 3}, {2, 3}};
+    static GfPlanned c;
+    const Lattice& L = ctx().lat;
+    if (!std::equal(c.nd, c.nd + 4, L.nd)) {
+        for (int p = 0; p < 6; p++) {
+            GfPlan& q = c.plans.p[p];
+            const int mu = planes[p][0], nu = planes[p][1];
+            q = gf_best_plan(L.nd[mu], L.nd[nu]);
+            q.mu = mu;
+            q.nu = nu;
+            q.tiles = q.tiles_m * q.tiles_n;
+            for (int k = 0; k < 4; k++)
+                if (k != mu && k != nu) q.tiles *= L.nd[k];
+            c.plans.tiles[p] = q.tiles;
+        }
+        std::copy(L.nd, L.nd + 4, c.nd);
+    }
+    return c.plans;
+}
+
+// lane offsets within a link array are 32-bit in the per-link kernel (up to 6 planes of 16 sizeh bytes)
+static bool gf_size_ok() { return (size_t)96 * ctx().lat.sizeh < ((size_t)1 << 32); }
+
+// the plane kernel's buffers, or false: the per-link kernel then (its halo wraps at most once along a direction)
+bool gf_planes_ready() {
+    const Lattice& L = ctx().lat;
+    if (!g_gf_planes || !gf_size_ok()) return false;
+    // even extents: a wrap keeps the site's parity
+    for (int k = 0; k < 4; k++)
+        if (L.nd[k] < 2 || (L.nd[k] & 1)) return false;
+    // 24-bit products of a coordinate and its stride
+    if ((long)L.nd[0] * L.nd[1] * L.nd[2] >= (1L << 24) || L.nd[3] >= (1 << 24)) return false;
+    const size_t links = (size_t)8 * L.sizeh;
+    return g_gf_rec.try_get(96 * links) && g_gf_part.try_get(3 * 64 * links);
+}
+static dim3 gf_grid8() { return dim3(blocks_for(ctx().lat.sizeh), 8); }
+
+bool gf_pack(const void* u) {
+    hipLaunchKernelGGL(k_gf_pack, gf_grid8(), dim3(kBlock), 0, ctx().stream, gauge_ptrs(u), (double2*)g_gf_rec.p,
+                       (int)ctx().lat.sizeh);
+    return hip_ok(hipGetLastError(), "k_gf_pack");
+}
+bool gf_unpack(void* u) {
+    hipLaunchKernelGGL(k_gf_unpack, gf_grid8(), dim3(kBlock), 0, ctx().stream, (const double2*)g_gf_rec.p,
+                       gauge_ptrs(u), (int)ctx().lat.sizeh);
+    return hip_ok(hipGetLastError(), "k_gf_unpack");
+}
+
+// the planes' force parts of the records' links (K planes from u); with stap, the staples as well
+bool gf_parts(const void* u, void* stap) {
+    const Lattice& L = ctx().lat;
+    const GfPlans& plans = gf_plans();
+    // The planes are independent unless the staples are summed: one launch, two blocks per CU (and at least
+    // a block for each XCD's share of the tiles).
+    const int step = stap ? 1 : 6;
+    for (int p = 0; p < 6; p += step) {
+        long tiles = 0;
+        for (int k = p; k < p + step; k++) tiles += plans.p[k].tiles;
+        const unsigned nb = (unsigned)std::max(8L, std::min(tiles, 512L));
+        auto go = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, ctx().stream, (const double2*)g_gf_rec.p, gauge_ptrs(u),
+                               (double2*)stap, L.su3_bytes(), (double2*)g_gf_part.p, link_geom(), plans, p, p + step,
+                               g_tlsm ? 1 : 0, g_c_zero);
+        };
+        if (L.par_temp) go(k_gf_tile<true>);
+        else go(k_gf_tile<false>);
+    }
+    return hip_ok(hipGetLastError(), "k_gf_tile");
+}
+bool gf_ipdot(void* ipdot, void* mom, double fact) {
+    hipLaunchKernelGGL(k_gf_ipdot, gf_grid8(), dim3(kBlock), 0, ctx().stream, (const double2*)g_gf_part.p, ipdot, mom,
+                       (int)ctx().lat.sizeh, fact);
+    return hip_ok(hipGetLastError(), "k_gf_ipdot");
+}
+// momentum step with the parts, then U <- exp(i delta P) U on the records
+bool gf_move(void* mom, double fact, double delta) {
+    hipLaunchKernelGGL(k_gf_move, gf_grid8(), dim3(kBlock), 0, ctx().stream, (const double2*)g_gf_part.p, mom,
+                       (double2*)g_gf_rec.p, (int)ctx().lat.sizeh, fact, delta);
+    return hip_ok(hipGetLastError(), "k_gf_move");
+}
 bool launch_gauge_force(const void* u, void* stap, void* ipdot, void* mom, double fact) {
     const Lattice& L = ctx().lat;
-    // lane offsets within a link array are 32-bit (up to 6 planes of 16 sizeh bytes)
-    if ((size_t)96 * L.sizeh >= ((size_t)1 << 32)) return fail("gauge force: lattice too large (sizeh %ld)", (long)L.sizeh);
-    // the plane kernels when every extent is a multiple of 4
-    if (g_gf_planes && gf_tile(L.nd[0]) && gf_tile(L.nd[1]) && gf_tile(L.nd[2]) && gf_tile(L.nd[3]))
-        return launch_gauge_force_planes(u, stap, ipdot, mom, fact);
+    if (!gf_size_ok()) return fail("gauge force: lattice too large (sizeh %ld)", (long)L.sizeh);
+    if (gf_planes_ready()) return gf_pack(u) && gf_parts(u, stap) && gf_ipdot(ipdot, mom, fact);
     // whole blocks per link array (the kernel takes the direction from the block)
     const int nb = 8 * (int)((L.sizeh + kGfLinks - 1) / kGfLinks);
     hipLaunchKernelGGL(k_gauge_force, dim3(nb), dim3(3 * kGfLinks), 0, ctx().stream, gauge_ptrs(u), (double2*)stap,

@@ -198,3 +198,42 @@ def test_plane_kernels_match_link_kernel(shape, tlsm, par_temp):
         assert rel(outs[k][0], outs[0][0]) < 1e-13
         assert rel(outs[k][1], outs[0][1]) < 1e-13
     assert rel(outs[1][2], outs[0][2]) < 1e-13
+
+
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (4, 4, 4, 4), (6, 10, 14, 2), (18, 14, 10, 6), (22, 2, 26, 4),
+                                   (32, 4, 16, 6), (8, 3, 4, 4)])
+@pytest.mark.parametrize("tlsm,par_temp", [(1, 0), (0, 0), (1, 1)])
+def test_plane_tiles_match_link_kernel(shape, tlsm, par_temp):
+    """The plane kernel on extents that its tiles divide and on those they
+    overhang, wrap onto themselves (extent 2) or leave to the per-link kernel
+    (an odd extent): the force with and without staples and a whole gauge
+    sub-integrator against the per-link kernel.  Both kernels round each link's
+    84-link sum differently, a few units of 2^-53 of its largest terms: 1e-13;
+    the five steps of the integrator carry that along: 1e-12."""
+    f = Field(shape, bool(par_temp), 9)
+    set_action(tlsm)
+    init_lattice(f.shape, par_temp=f.pt)
+    n = 8 * 8 * f.sizeh
+    mom0 = np.random.default_rng(3).standard_normal(n)
+    ost.ActionParam.in_dll(lib, "act_params").beta = 3.8
+    md = ost.MdParam(no_md=2, gauge_scale=2, t=0.4)
+    C.memmove(C.addressof(ost.MdParam.in_dll(lib, "md_parameters")), C.addressof(md), C.sizeof(md))
+    lib.initialize_md_global_variables(md)
+    outs = []
+    for planes in (0, 1):
+        prev = lib.ostp_set_gauge_force_kernel(planes)
+        du, dt, dm, ds = Dev(f.u), Dev(nbytes=8 * n), Dev(mom0), Dev(nbytes=8 * f.per)
+        zero = np.zeros(8 * f.per, dtype=np.uint8)
+        got = []
+        assert lib.ostp_time_gauge_force(du.p, None, dt.p, dm.p, 0.37, 1) > 0
+        got += [dt.get(mom0), dm.get(mom0)]
+        lib.calc_ipdot_gauge_soloopenacc(du.p, ds.p, dt.p)
+        got += [dt.get(mom0), staple_planes(f, ds.get(zero))]
+        lib.multistep_2MN_gauge(du.p, ds.p, dt.p, dm.p)
+        got += [du.get(f.u).view(np.float64), dt.get(mom0), dm.get(mom0), staple_planes(f, ds.get(zero))]
+        lib.ostp_set_gauge_force_kernel(prev)
+        ost.check(0, "gauge force")
+        outs.append(got)
+    assert np.abs(outs[0][0]).max() > 0.1
+    for k, (a, b) in enumerate(zip(*outs)):
+        assert rel(a, b) < (1e-13 if k < 4 else 1e-12), k

@@ -138,3 +138,49 @@ def test_dslash_workgroup_mapping_is_a_bijection(shape):
     assert len(np.unique(valid)) == sizeh and valid.min() == 0
     if tmajor:
         assert idx.max() == sizeh - 1  # no thread beyond the lattice
+
+
+def test_gauge_force_tile_arrays():
+    """The LDS arrays of the gauge force's plane tiles (gf_plan and k_gf_tile in
+    openstaple_amd/csrc/stout.hip): every record that a corner, a staple or a
+    side reads lies inside its array, for every tile the plan accepts, and the
+    multiply-shift division of item numbers is exact."""
+    M, N, Cm, Cn, SMp, SMm, SNp, SNm = range(8)
+    tiles = 0
+    for tm, tn in itertools.product(range(1, 65), repeat=2):
+        R = [(-2, -2, tm + 3, tn + 4), (-2, -2, tm + 4, tn + 3), (-1, -2, tm + 2, tn + 2), (-2, -1, tm + 2, tn + 2),
+             (-1, 1, tm + 1, tn), (-1, -1, tm + 1, tn + 1), (1, -1, tm, tn + 1), (-1, -1, tm + 1, tn + 1)]
+        n = [r[2] * r[3] for r in R]
+        np_ = n[SMp] + n[SNp]
+        links, items = n[M] + n[N], -(-np_ // 64) * 64 + n[SMm] + n[SNm]
+        if not (tm * tn <= 64 and sum(n) <= 826 and links <= 292 and links <= 340 and n[Cm] + n[Cn] <= 256 and
+                items <= 512 and links + 384 <= 826):
+            continue
+        tiles += 1
+        for r in R:
+            q = np.arange(512)
+            assert np.array_equal((q * (-(-65536 // r[2]))) >> 16, q // r[2])
+
+        def inside(role, i, j):
+            a = R[role]
+            assert a[0] <= i < a[0] + a[2] and a[1] <= j < a[1] + a[3], (tm, tn, role, i, j)
+
+        def sites(role):
+            a = R[role]
+            return itertools.product(range(a[0], a[0] + a[2]), range(a[1], a[1] + a[3]))
+
+        for role, reads in ((Cm, [(M, 0, 0), (N, 1, 0)]), (Cn, [(N, 0, 0), (M, 0, 1)]), (SMp, [(N, 1, 0), (Cn, 0, 0)]),
+                            (SNp, [(M, 0, 1), (Cm, 0, 0)]), (SMm, [(Cm, 0, -1), (N, 0, -1)]),
+                            (SNm, [(Cn, -1, 0), (M, -1, 0)])):
+            for (i, j), (r, di, dj) in itertools.product(sites(role), reads):
+                inside(r, i + di, j + dj)
+        for d in (0, 1):  # links along mu, along nu; offsets along the own and the other direction
+            O, P, Co, Cp, SOp, SOm, SPp, SPm = ((M, N, Cm, Cn, SMp, SMm, SNp, SNm), (N, M, Cn, Cm, SNp, SNm, SMp, SMm))[d]
+            reads = [(P, 1, 0), (SOp, 0, 1), (P, 0, 0), (O, 0, 1), (SPm, 0, 0), (SPp, 1, 0), (Cp, 0, 0), (P, 0, -1),
+                     (P, 1, -1), (SOm, 0, -1), (SPp, 1, -1), (O, 0, -1), (SPm, 0, -1), (Co, 0, -1), (O, 0, 0),
+                     # K of the staples' links
+                     (P, 1, 1), (O, 0, 2), (P, 0, 1), (P, -1, 0), (O, -1, 1), (O, -1, 0), (O, 1, 1), (P, 2, 0), (O, 1, 0),
+                     (P, 1, -2), (O, 0, -2), (P, 0, -2), (P, 2, -1), (O, 1, -1), (P, -1, -1), (O, -1, -1)]
+            for i, j, (r, o, p) in itertools.product((0, tm - 1), (0, tn - 1), reads):
+                inside(r, i + (p if d else o), j + (o if d else p))
+    assert tiles > 100
