@@ -152,8 +152,6 @@ bool launch_finalize(int fin, const SolverCtl& c, int nparts) {
     switch (fin) {
         case kFinStore: OSTP_F(kFinStore, 1); break;
         case kFinStore2: OSTP_F(kFinStore2, 2); break;
-        case kFinCgAlpha: OSTP_F(kFinCgAlpha, 1); break;
-        case kFinCgLambda: OSTP_F(kFinCgLambda, 1); break;
         case kFinCgRestart: OSTP_F(kFinCgRestart, 1); break;
         case kFinMsAlpha: OSTP_F(kFinMsAlpha, 1); break;
         case kFinMsLambda: OSTP_F(kFinMsLambda, 1); break;

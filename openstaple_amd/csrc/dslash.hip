@@ -139,14 +139,14 @@ bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, con
         if (eo == 0) OSTP_L(0, kMdagM); else OSTP_L(1, kMdagM);
     } else {
         if (eo != 0) return fail("fused dot epilogue only on Deo");
-        if (fin != kFinStore && fin != kFinCgAlpha && fin != kFinMsAlpha && fin != kFinMxAlpha &&
-            fin != kFinFcgAlpha && fin != kFinMxmAlpha)
+        if (fin != kFinNone && fin != kFinStore && fin != kFinMsAlpha && fin != kFinMxAlpha && fin != kFinFcgAlpha &&
+            fin != kFinMxmAlpha)
             return fail("unsupported dslash finalizer %d", fin);
         OSTP_L(0, kMdagMDot);
     }
 #undef OSTP_L
     if (!hip_ok(hipGetLastError(), "k_dslash launch")) return false;
-    return mode == kMdagMDot ? launch_finalize(fin, ctl, nb) : true;
+    return mode == kMdagMDot && fin != kFinNone ? launch_finalize(fin, ctl, nb) : true;
 }
 
 template bool launch_dslash<double>(int, int, int, const void*, const void*, const void*, void*, const void*,

@@ -18,9 +18,8 @@
 namespace ostp {
 
 enum Fin : int {
+    kFinNone = -1,      // no finalizer: the next kernel sums the partials
     kFinStore = 0,      // st->sum = total (stand-alone reduction)
-    kFinCgAlpha,        // alpha, omega = delta/alpha          (inverter_full.c:76-80)
-    kFinCgLambda,       // lambda, gammag, delta, counters, exit test (inverter_full.c:86-105)
     kFinCgRestart,      // delta = |r|^2 at a (re)start          (inverter_full.c:60-66)
     kFinMsAlpha,        // CG-M alpha + shift recurrences     (inverter_multishift_full.c:116-136)
     kFinMsLambda,       // CG-M lambda, gammas, flags          (inverter_multishift_full.c:141-171)
@@ -80,23 +79,10 @@ __device__ __forceinline__ void finalize(SolverState* st, double tot, double tot
     } else if (F == kFinStore2) {
         st->sum = tot;
         st->sum_im = tot_im;
-    } else if (F == kFinCgAlpha) {
-        st->alpha = tot;
-        st->omega = st->delta / tot;
     } else if (F == kFinCgRestart) {
         st->delta = tot;
         st->cg_restarted = 0;
         st->status = kRunning;
-    } else if (F == kFinCgLambda) {
-        const double lambda = tot;
-        st->lambda = lambda;
-        st->gammag = lambda / st->delta;
-        st->delta = lambda;
-        st->cg += 1;
-        st->cg_restarted += 1;
-        const bool cont = (sqrt(lambda / st->source_norm) > st->res * st->safety) &&
-                          st->cg_restarted < st->restart_every;
-        if (!cont) st->status = kInnerExit;
     } else if (F == kFinMsAlpha || F == kFinMxmAlpha) {
         // flags/maxiter computed at the end of the previous iteration become current
         st->flag_cur ^= 1;

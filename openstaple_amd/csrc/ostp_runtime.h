@@ -52,7 +52,7 @@ struct Context {
     unsigned dslash_launches = 0;
     // device scratch: reduction partials + solver state
     double* partials = nullptr;     // 2 * max_blocks
-    SolverState* state = nullptr;   // device
+    SolverState* state = nullptr;   // device: two copies (the fused iterations alternate between them)
     SolverState* state_host = nullptr;  // pinned mirror
     int max_blocks = 0;
     // extents for the host-only entry points (field files) set by

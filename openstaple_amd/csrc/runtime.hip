@@ -221,8 +221,8 @@ int ostp_init(int nd0, int nd1, int nd2, int nd3, int par_temp) {
     if (!c.partials || blocks > c.max_blocks) {
         release_scratch();
         if (!hip_ok(hipMalloc(&c.partials, sizeof(double) * 4 * (size_t)blocks), "hipMalloc partials")) return 1;
-        if (!hip_ok(hipMalloc(&c.state, sizeof(SolverState)), "hipMalloc state")) return 1;
-        if (!hip_ok(hipHostMalloc(&c.state_host, sizeof(SolverState), hipHostMallocDefault), "hipHostMalloc"))
+        if (!hip_ok(hipMalloc(&c.state, 2 * sizeof(SolverState)), "hipMalloc state")) return 1;
+        if (!hip_ok(hipHostMalloc(&c.state_host, 2 * sizeof(SolverState), hipHostMallocDefault), "hipHostMalloc"))
             return 1;
         c.max_blocks = blocks;
     }

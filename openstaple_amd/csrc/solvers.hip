@@ -15,7 +15,7 @@
 // updates are fused (x and r together; the multishift x_k and p_k together
 // with p) without changing what each element computes.
 #include "ostp_blas.h"
-#include "ostp_dslash.h"
+#include "ostp_krylov.h"
 
 #include <algorithm>
 #include <cmath>
@@ -145,14 +145,6 @@ __global__ __launch_bounds__(kBlock) void k_ms_update(const C* __restrict__ r, C
 // are kept (W x 48 B per half-site) and one pass per window updates x_k and
 // p_k: per iteration that is about 2 vectors of traffic instead of 4 per
 // active shift.
-constexpr int kMsWinMax = 64;
-struct MsWin {
-    int t;                                  // iterations in the current window
-    int active[kMaxShifts];                 // shift moved in this window
-    double a[kMaxShifts], B[kMaxShifts];
-    double c[kMaxShifts][kMsWinMax], D[kMaxShifts][kMsWinMax];
-};
-
 // r_new = r_old + omega s ; lambda = |r_new|^2
 template <typename C>
 __global__ __launch_bounds__(kBlock) void k_msw_r(const C* __restrict__ r_old, C* __restrict__ r_new,
@@ -223,10 +215,10 @@ constexpr int kMswGroup = 8;
 template <typename CX, typename C>
 __global__ __launch_bounds__(kBlock) void k_msw_flush(CX* __restrict__ xs, C* __restrict__ ps,
                                                       const C* __restrict__ hist, long n3, int order,
-                                                      const MsWin* __restrict__ w, SolverCtl ctl) {
+                                                      const MsWin* __restrict__ w, SolverCtl ctl, int full = 0) {
     if (!pred_pass(ctl)) return;
     const int t = w->t;
-    if (t == 0) return;
+    if (t == 0 || t < full) return;  // full: only a window of that many iterations
     const long i = (long)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n3) return;
     for (int k0 = 0; k0 < order; k0 += kMswGroup) {
@@ -271,9 +263,12 @@ __global__ __launch_bounds__(kBlock) void k_msw_flush(CX* __restrict__ xs, C* __
     }
 }
 
-// a fresh window: coefficients of the identity map
-__global__ __launch_bounds__(kBlock) void k_msw_reset(MsWin* w, SolverCtl ctl) {
+// a fresh window: coefficients of the identity map (full: only when that many
+// iterations fill it; w->t is not read otherwise, new memory holds anything)
+__global__ __launch_bounds__(kBlock) void k_msw_reset(MsWin* w, SolverCtl ctl, int full = 0) {
     if (!pred_pass(ctl)) return;
+    if (full && w->t < full) return;
+    __syncthreads();  // every thread has read t before it is cleared
     for (int e = threadIdx.x; e < kMaxShifts * kMsWinMax; e += kBlock) {
         const int k = e / kMsWinMax, j = e - k * kMsWinMax;
         w->c[k][j] = 0.0;
@@ -550,6 +545,184 @@ static void init_state(double res, double safety, int max_cg, int restart_every)
     s.status = kRunning;
 }
 
+// ------------------------------------- CG and CG-M in three launches each
+// (ostp_krylov.h).  The states of the systems lie two by two in `st`.
+struct KrSys {
+    const void* b;
+    void *x;                     // CG: the iterate
+    void *r, *h, *s, *p;
+    double m2;
+    char* hist = nullptr;        // CG-M: window of W residuals
+    MsWin* win = nullptr;
+    void *out = nullptr, *shiftferm = nullptr;
+    int order = 0;
+};
+
+// Lattices whose hops are split over waves (half-sites).  Below, the chip is
+// not full with a site per thread and the split form's shorter chain wins; above,
+// r and p read at eight neighbours each and the exchange through LDS cost more
+// than a kernel that stores p.  One CG-M system, split against not: ahead up to
+// 24^3 x 6 (41472), even at 24^3 x 8 (55296), behind from 32^3 x 4 (65536) on.
+constexpr long kKrSplitSizeh = 49152;
+
+static bool kr_split() { return ctx().lat.sizeh <= kKrSplitSizeh; }
+static int kr_blocks_hop() { return blocks_for(ctx().lat.sizeh, kr_split() ? kKrSites : kBlock); }
+static int kr_blocks_r() { return std::min(blocks_for(ctx().lat.sizeh), 1024); }
+// partials per system: <p, s> (two doubles a block in the ordinary hop kernels) and |r|^2
+static size_t kr_partials() { return 2 * (size_t)kr_blocks_hop() + kr_blocks_r(); }
+
+static void kr_split_hop(bool doe, const KrArgs& a, int nb) {
+    auto go = [&](auto kern, int blocks) { hipLaunchKernelGGL(kern, dim3(blocks), dim3(kKrThreads), 0, S(), a); };
+    if (doe) {
+        const int blocks = a.close ? 1 : nb;
+        if (a.n == 1) go(k_kr_doe<1>, blocks);
+        else if (a.n == 2) go(k_kr_doe<2>, blocks);
+        else go(k_kr_doe<kKrSys>, blocks);
+    } else {
+        if (a.n == 1) go(k_kr_deo<1>, nb);
+        else if (a.n == 2) go(k_kr_deo<2>, nb);
+        else go(k_kr_deo<kKrSys>, nb);
+    }
+}
+
+// both hops of iteration a.j by the ordinary kernels
+static bool kr_plain_hops(const void* u, const void* ph, const KrArgs& a);
+
+// ln(residual / target) of a state the loop left (NaN when unknown)
+static double kr_dist(const SolverState& s, bool ms) {
+    double m = s.delta;
+    if (ms) {
+        m = 0.0;
+        for (int k = 0; k < s.order && k < kMaxShifts; k++)
+            if (s.flags[0][k] == 1) m = std::max(m, s.delta * s.zeta_ii[k] * s.zeta_ii[k]);
+    }
+    if (!(m > 0.0) || !(s.source_norm > 0.0) || !(s.res > 0.0)) return NAN;
+    return 0.5 * std::log(m / s.source_norm) - std::log(s.res * s.safety);
+}
+
+// Iterate n systems from the states in st (copies 0; pinned mirror st_host)
+// until none runs.  part: room for n x (hop blocks + r blocks) partials.  On
+// return st_host[2 k] holds system k's last state.
+static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bool ms, int W, SolverState* st,
+                       SolverState* st_host, double* part, size_t part_stride) {
+    const Lattice& L = ctx().lat;
+    const long sizeh = L.sizeh, n3 = 3 * sizeh;
+    const size_t vb = L.vec3_bytes();
+    const bool split = kr_split();
+    const int nb = kr_blocks_hop(), nr = kr_blocks_r(), nb3 = blocks_for(n3);
+    KrArgs a{};
+    for (int l = 0; l < 8; l++) {
+        a.u[l] = (const double2*)((const char*)u + l * L.su3_bytes());
+        a.ph[l] = (const double*)((const char*)ph + l * L.dsoa_bytes());
+    }
+    a.g.nd0 = L.nd[0];
+    a.g.nd0h = L.nd[0] / 2;
+    a.g.nd1 = L.nd[1];
+    a.g.nd2 = L.nd[2];
+    a.g.nd3 = L.nd[3];
+    a.g.sizeh = (int)sizeh;
+    a.tmajor = (sizeh / L.nd[3]) % (split ? kKrSites : kBlock) == 0;  // whole tiles per t-slice, as k_dslash
+    a.n = n;
+    a.ms = ms ? 1 : 0;
+    a.nA = nb;
+    a.nB = nr;
+    a.sA = split ? 1 : 2;
+    for (int k = 0; k < n; k++) {
+        a.p[k] = (double2*)sy[k].p;
+        a.h[k] = (double2*)sy[k].h;
+        a.s[k] = (double2*)sy[k].s;
+        a.x[k] = (double2*)sy[k].x;
+        a.m2[k] = sy[k].m2;
+        a.st[k] = st + 2 * k;
+        a.partA[k] = part + k * part_stride;
+        a.partB[k] = part + k * part_stride + 2 * nb;
+        a.win[k] = sy[k].win;
+        a.xs[k] = (double2*)sy[k].out;
+        a.ps[k] = (double2*)sy[k].shiftferm;
+    }
+    auto residual = [&](int k, int j) {  // of system k after iteration j
+        if (!W || j == 0) return (double2*)sy[k].r;
+        return (double2*)(sy[k].hist + (size_t)((j - 1) % W) * vb);
+    };
+    // the end of iteration j - 1 and the first kernel of iteration j (close: the end only)
+    auto first = [&]() {
+        if (split) {
+            a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
+            kr_split_hop(true, a, nb);
+        } else {
+            hipLaunchKernelGGL(k_kr_p, dim3(a.close ? 1 : nr, n), dim3(kBlock), 0, S(), a);
+        }
+    };
+    int j = 0, batch = 16;
+    double prev_d = NAN;
+    for (int k = 0; k < n; k++) {
+        const double d = kr_dist(st_host[2 * k], ms);
+        if (std::isfinite(d)) prev_d = std::isfinite(prev_d) ? std::max(prev_d, d) : d;
+    }
+    int prev_j = 0, last_total = -1;
+    for (;;) {
+        for (int i = 0; i < batch; i++) {
+            a.j = ++j;
+            a.close = 0;
+            for (int k = 0; k < n; k++) {
+                a.r[k] = residual(k, j - 1);
+                a.rn[k] = residual(k, j);
+            }
+            first();
+            if (ms && !W) hipLaunchKernelGGL(k_kr_shifts, dim3(nb3, n), dim3(kBlock), 0, S(), a, n3);
+            if (W && j > 1 && (j - 1) % W == 0)
+                for (int k = 0; k < n; k++) {
+                    // the windows that iteration j - 1 filled
+                    hipLaunchKernelGGL((k_msw_flush<double2, double2>), dim3(nb3), dim3(kBlock), 0, S(),
+                                       (double2*)sy[k].out, (double2*)sy[k].shiftferm, (const double2*)sy[k].hist, n3,
+                                       sy[k].order, (const MsWin*)sy[k].win, ctl_of(kAlways), W);
+                    hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), sy[k].win, ctl_of(kAlways), W);
+                }
+            if (split) {
+                a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
+                kr_split_hop(false, a, nb);
+            } else if (!kr_plain_hops(u, ph, a)) {
+                return false;
+            }
+            if (ms) hipLaunchKernelGGL((k_kr_r<1>), dim3(nr, n), dim3(kBlock), 0, S(), a);
+            else hipLaunchKernelGGL((k_kr_r<0>), dim3(nr, n), dim3(kBlock), 0, S(), a);
+        }
+        a.j = j + 1;
+        a.close = 1;
+        for (int k = 0; k < n; k++) a.r[k] = residual(k, j);
+        first();
+        if (ms && !W) hipLaunchKernelGGL(k_kr_shifts, dim3(nb3, n), dim3(kBlock), 0, S(), a, n3);
+        if (!check_launch("solver iterations") ||
+            !hip_ok(hipMemcpyAsync(st_host, st, 2 * n * sizeof(SolverState), hipMemcpyDeviceToHost, S()),
+                    "solver states") ||
+            !hip_ok(hipStreamSynchronize(S()), "solver states"))
+            return false;
+        int running = 0, total = 0;
+        double d = NAN;
+        for (int k = 0; k < n; k++) {
+            if ((j + 1) & 1) st_host[2 * k] = st_host[2 * k + 1];
+            const SolverState& s = st_host[2 * k];
+            total += s.cg;
+            if (s.status != kRunning) continue;
+            running++;
+            const double dk = kr_dist(s, ms);
+            if (std::isfinite(dk)) d = std::isfinite(d) ? std::max(d, dk) : dk;
+        }
+        if (!running) return true;
+        // a running solver's counter advances with every iteration
+        if (total == last_total) return fail("solver state did not advance (iteration %d)", j);
+        last_total = total;
+        // the iterations left at the convergence rate so far, with a margin
+        batch = std::min(2 * batch, 64);
+        if (std::isfinite(d) && std::isfinite(prev_d)) {
+            const double rate = (prev_d - d) / (double)(j - prev_j);
+            if (rate > 1e-9) batch = std::min(batch, std::max(2, (int)std::ceil(1.1 * std::max(d, 0.0) / rate) + 1));
+        }
+        prev_d = d;
+        prev_j = j;
+    }
+}
+
 // CG of ker_invert_openacc on device pointers.  Returns status, *cg_out.
 struct CgBufs {
     const void *u, *ph, *b;
@@ -562,12 +735,13 @@ int cg_solve(const CgBufs& B, double mass, double shift, double res, int max_cg,
              double* true_res) {
     const long sizeh = ctx().lat.sizeh;
     const long n3 = 3 * sizeh;
-    const int nbh = blocks_for(sizeh), nb3 = blocks_for(n3);
+    const int nbh = blocks_for(sizeh);
     const double m2 = mass * mass + shift;
     double sn = 0.0;
     if (!source_norm(B.b, &sn)) return INVERTER_FAILURE;
     init_state(res, 0.95, max_cg, restart_every);
     H().source_norm = sn;
+    H().delta = sn;  // the distance from the target at the start
     if (!push_state()) return INVERTER_FAILURE;
 
     auto restart = [&]() -> bool {
@@ -577,22 +751,21 @@ int cg_solve(const CgBufs& B, double mass, double shift, double res, int max_cg,
                            (const double2*)B.s, (double2*)B.r, (double2*)B.p, (int)sizeh, ctl_of(kAlways));
         return check_launch("k_cg_restart") && launch_finalize(kFinCgRestart, ctl_of(kAlways), nbh);
     };
-    auto iteration = [&](int j) -> bool {
-        // s = M p ; alpha = (p,s) ; omega = delta/alpha
-        if (!launch_mdagm<double>(B.u, B.ph, B.p, B.h, B.s, m2, 2, kFinCgAlpha, ctl_of(kIfRunning))) return false;
-        hipLaunchKernelGGL((k_cg_xr<double2>), dim3(nbh), dim3(kBlock), 0, S(), (double2*)B.x, (double2*)B.r,
-                           (const double2*)B.p, (const double2*)B.s, (int)sizeh, ctl_of(kIfRunning));
-        if (!launch_finalize(kFinCgLambda, ctl_of(kIfRunning), nbh)) return false;
-        hipLaunchKernelGGL((k_cg_p<double2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)B.p, (const double2*)B.r, n3,
-                           ctl_of(kIfIter, j));
-        return check_launch("cg iteration");
-    };
-
+    KrSys sys{};
+    sys.b = B.b;
+    sys.x = B.x;
+    sys.r = B.r;
+    sys.h = B.h;
+    sys.s = B.s;
+    sys.p = B.p;
+    sys.m2 = m2;
     if (!restart()) return INVERTER_FAILURE;
     for (;;) {
-        if (!run_batches(iteration, 4, dist_cg)) return INVERTER_FAILURE;
+        if (!kr_iterate(B.u, B.ph, &sys, 1, false, 0, ctx().state, ctx().state_host, ctx().partials, 0))
+            return INVERTER_FAILURE;
         const SolverState& s = H();
         if (s.status == kInnerExit && std::sqrt(s.lambda / s.source_norm) > res && s.cg < max_cg) {
+            if (!push_state()) return INVERTER_FAILURE;  // into the copy the first iteration reads
             if (!restart()) return INVERTER_FAILURE;
             continue;
         }
@@ -952,12 +1125,14 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
     s.order = order;
     s.flag_cur = 0;
     for (int k = 0; k < order; k++) {
-        s.flags[1][k] = 1;  // becomes current at the first iteration
+        s.flags[0][k] = 1;  // current in kr_iterate
+        s.flags[1][k] = 1;  // becomes current at the first iteration of the other loops
         s.zeta_i[k] = 1.0;
         s.zeta_ii[k] = 1.0;
         s.gammas[k] = 0.0;
         s.shifts[k] = shifts[k];
     }
+    s.maxiter = order;
     s.maxiter_next = order;
     if (order == 0) s.status = kDone;  // the reference's loop runs once; nothing to update without shifts
     if (!push_state()) return INVERTER_FAILURE;
@@ -977,41 +1152,57 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
         }
         hist = (char*)g_msw_hist;
         if (!g_msw && !hip_ok(hipMalloc(&g_msw, sizeof(MsWin)), "multishift window")) return INVERTER_FAILURE;
-        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kAlways));
+        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kAlways), 0);
     }
     auto slot = [&](int j) { return (C*)(hist + (size_t)((j - 1) % W) * vb); };  // residual of iteration j (1-based)
-    auto iteration = [&](int j) -> bool {
-        if (!launch_mdagm<R>(B.u, B.ph, B.p, B.h, B.s, m2, 2, kFinMsAlpha, ctl_of(kIfRunning))) return false;
-        if (!hist) {
-            hipLaunchKernelGGL((k_ms_r<C>), dim3(nbh), dim3(kBlock), 0, S(), (C*)B.r, (const C*)B.s, (int)sizeh,
+    if constexpr (sizeof(R) == 8) {
+        KrSys sys{};
+        sys.r = B.r;
+        sys.h = B.h;
+        sys.s = B.s;
+        sys.p = B.p;
+        sys.m2 = m2;
+        sys.hist = hist;
+        sys.win = hist ? g_msw : nullptr;
+        sys.out = B.out;
+        sys.shiftferm = B.shiftferm;
+        sys.order = order;
+        if (!kr_iterate(B.u, B.ph, &sys, 1, true, hist ? W : 0, ctx().state, ctx().state_host, ctx().partials, 0))
+            return INVERTER_FAILURE;
+    } else {
+        auto iteration = [&](int j) -> bool {
+            if (!launch_mdagm<R>(B.u, B.ph, B.p, B.h, B.s, m2, 2, kFinMsAlpha, ctl_of(kIfRunning))) return false;
+            if (!hist) {
+                hipLaunchKernelGGL((k_ms_r<C>), dim3(nbh), dim3(kBlock), 0, S(), (C*)B.r, (const C*)B.s, (int)sizeh,
+                                   ctl_of(kIfRunning));
+                if (!launch_finalize(kFinMsLambda, ctl_of(kIfRunning), nbh)) return false;
+                hipLaunchKernelGGL((k_ms_update<C>), dim3(nb3), dim3(kBlock), 0, S(), (const C*)B.r, (C*)B.p,
+                                   (C*)B.out, (C*)B.shiftferm, vstride, n3, ctl_of(kIfIter, j));
+                return check_launch("multishift iteration");
+            }
+            const C* r_old = j == 1 ? (const C*)B.r : slot(j - 1);
+            C* r_new = slot(j);
+            hipLaunchKernelGGL((k_msw_r<C>), dim3(nbh), dim3(kBlock), 0, S(), r_old, r_new, (const C*)B.s, (int)sizeh,
                                ctl_of(kIfRunning));
             if (!launch_finalize(kFinMsLambda, ctl_of(kIfRunning), nbh)) return false;
-            hipLaunchKernelGGL((k_ms_update<C>), dim3(nb3), dim3(kBlock), 0, S(), (const C*)B.r, (C*)B.p,
-                               (C*)B.out, (C*)B.shiftferm, vstride, n3, ctl_of(kIfIter, j));
+            hipLaunchKernelGGL((k_msw_p<C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.p, (const C*)r_new, n3, g_msw,
+                               ctl_of(kIfIter, j), (C*)nullptr);
+            if (j % W == 0) {
+                // only when iteration j ran: a window cut short is flushed once, at the end
+                hipLaunchKernelGGL((k_msw_flush<C, C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.out, (C*)B.shiftferm,
+                                   (const C*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kIfIter, j), 0);
+                hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kIfIter, j), 0);
+            }
             return check_launch("multishift iteration");
-        }
-        const C* r_old = j == 1 ? (const C*)B.r : slot(j - 1);
-        C* r_new = slot(j);
-        hipLaunchKernelGGL((k_msw_r<C>), dim3(nbh), dim3(kBlock), 0, S(), r_old, r_new, (const C*)B.s, (int)sizeh,
-                           ctl_of(kIfRunning));
-        if (!launch_finalize(kFinMsLambda, ctl_of(kIfRunning), nbh)) return false;
-        hipLaunchKernelGGL((k_msw_p<C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.p, (const C*)r_new, n3, g_msw,
-                           ctl_of(kIfIter, j), (C*)nullptr);
-        if (j % W == 0) {
-            // only when iteration j ran: a window cut short is flushed once, at the end
-            hipLaunchKernelGGL((k_msw_flush<C, C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.out, (C*)B.shiftferm,
-                               (const C*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kIfIter, j));
-            hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kIfIter, j));
-        }
-        return check_launch("multishift iteration");
-    };
-    if (!run_batches(iteration, 4, dist_ms)) return INVERTER_FAILURE;
+        };
+        if (!run_batches(iteration, 4, dist_ms)) return INVERTER_FAILURE;
+    }
     const int cg = H().cg;
     if (hist) {
         // the partial last window, and the final residual where the per-iteration
         // version leaves it
         hipLaunchKernelGGL((k_msw_flush<C, C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.out, (C*)B.shiftferm,
-                           (const C*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kAlways));
+                           (const C*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kAlways), 0);
         if (cg > 0 && !hip_ok(hipMemcpyAsync(B.r, slot(cg), vb, hipMemcpyDeviceToDevice, S()), "final residual"))
             return INVERTER_FAILURE;
         if (!check_launch("multishift window flush")) return INVERTER_FAILURE;
@@ -1073,7 +1264,7 @@ template int multishift_solve<float>(const MsBufs&, double, int, const double*, 
 // order and reduction slots), and every other kernel of the iteration runs
 // per system on its own device state, window and partials.  Each system's
 // iterations, solutions and residuals are those of multishift_solve.
-constexpr int kMsMulti = 4;
+constexpr int kMsMulti = kKrSys;
 struct MsMultiHop {
     const double2* u[8];
     const double* ph[8];
@@ -1192,6 +1383,47 @@ static void launch_multi_hop(const MsMultiHop& a, int nbh) {
         hipLaunchKernelGGL((k_ms_multi_hop<EO, kMsMulti>), dim3(nbh), dim3(kBlock), 0, S(), a);
 }
 
+static bool kr_plain_hops(const void* u, const void* ph, const KrArgs& a) {
+    const int nb = kr_blocks_hop();
+    if (a.n == 1) {
+        SolverCtl c;
+        c.st = a.st[0] + (a.j & 1);
+        c.partials = a.partA[0];
+        c.pred = kIfRunning;
+        return launch_dslash<double>(1, kPlain, kFinStore, u, ph, a.p[0], a.h[0], nullptr, 0.0, c) &&
+               launch_dslash<double>(0, kMdagMDot, kFinNone, u, ph, a.h[0], a.s[0], a.p[0], a.m2[0], c);
+    }
+    MsMultiHop m;
+    for (int l = 0; l < 8; l++) {
+        m.u[l] = a.u[l];
+        m.ph[l] = a.ph[l];
+    }
+    m.g = a.g;
+    m.tmajor = a.tmajor;
+    m.n = a.n;
+    m.pred = kIfRunning;
+    for (int k = 0; k < kMsMulti; k++) {
+        const int q = k < a.n ? k : 0;
+        m.st[k] = a.st[q] + (a.j & 1);
+        m.part[k] = a.partA[q];
+        m.m2[k] = a.m2[q];
+        m.in[k] = a.p[q];
+        m.out[k] = a.h[q];
+        m.x[k] = nullptr;
+    }
+    m.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
+    launch_multi_hop<1>(m, nb);
+    for (int k = 0; k < kMsMulti; k++) {
+        const int q = k < a.n ? k : 0;
+        m.in[k] = a.h[q];
+        m.out[k] = a.s[q];
+        m.x[k] = a.p[q];
+    }
+    m.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
+    launch_multi_hop<0>(m, nb);
+    return check_launch("k_ms_multi_hop");
+}
+
 struct MsSys {
     const void* b;
     void *out, *shiftferm, *r, *h, *s, *p;
@@ -1206,8 +1438,18 @@ struct MsSys {
 
 static SolverState* g_mm_st = nullptr;       // device states of the systems
 static SolverState* g_mm_st_host = nullptr;  // pinned mirror
-static double* g_mm_part = nullptr;          // kMsMulti x 2 nbh partials
+static double* g_mm_part = nullptr;          // kMsMulti x g_mm_part_n partials
 static size_t g_mm_part_n = 0;
+static bool mm_partials() {
+    const size_t need = std::max((size_t)2 * blocks_for(ctx().lat.sizeh), kr_partials());
+    if (g_mm_part_n >= need) return true;
+    if (g_mm_part) (void)hipFree(g_mm_part);
+    g_mm_part = nullptr;
+    g_mm_part_n = 0;
+    if (!hip_ok(hipMalloc(&g_mm_part, sizeof(double) * need * kMsMulti), "multi partials")) return false;
+    g_mm_part_n = need;
+    return true;
+}
 static MsWin* g_mm_win = nullptr;            // kMsMulti windows
 static void* g_mm_hist = nullptr;            // kMsMulti x W residuals
 static size_t g_mm_hist_bytes = 0;
@@ -1219,7 +1461,7 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
     const Lattice& L = ctx().lat;
     const long sizeh = L.sizeh, n3 = 3 * sizeh;
     const size_t vb = L.vec3_bytes();
-    const int nbh = blocks_for(sizeh), nb3 = blocks_for(n3);
+    const int nb3 = blocks_for(n3);
     if (n < 1 || n > kMsMulti) return false;
     for (int k = 0; k < n; k++)
         if (sy[k].order < 0 || sy[k].order > kMaxShifts) return false;
@@ -1227,19 +1469,13 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
     if (W < 2) return false;
     // device resources
     if (!g_mm_st) {
-        if (!hip_ok(hipMalloc(&g_mm_st, kMsMulti * sizeof(SolverState)), "multi states") ||
-            !hip_ok(hipHostMalloc(&g_mm_st_host, kMsMulti * sizeof(SolverState), hipHostMallocDefault),
+        if (!hip_ok(hipMalloc(&g_mm_st, 2 * kMsMulti * sizeof(SolverState)), "multi states") ||
+            !hip_ok(hipHostMalloc(&g_mm_st_host, 2 * kMsMulti * sizeof(SolverState), hipHostMallocDefault),
                     "multi states") ||
             !hip_ok(hipMalloc(&g_mm_win, kMsMulti * sizeof(MsWin)), "multi windows"))
             return false;
     }
-    if (g_mm_part_n < (size_t)2 * nbh) {
-        if (g_mm_part) (void)hipFree(g_mm_part);
-        g_mm_part = nullptr;
-        g_mm_part_n = 0;
-        if (!hip_ok(hipMalloc(&g_mm_part, sizeof(double) * 2 * nbh * kMsMulti), "multi partials")) return false;
-        g_mm_part_n = (size_t)2 * nbh;
-    }
+    if (!mm_partials()) return false;
     const size_t hb = (size_t)W * vb;
     if (g_mm_hist_bytes < (size_t)n * hb) {
         if (g_mm_hist) (void)hipFree(g_mm_hist);
@@ -1251,14 +1487,6 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
         }
         g_mm_hist_bytes = (size_t)n * hb;
     }
-    auto ctl_k = [&](int k, int pred, int iter = 0) {
-        SolverCtl c;
-        c.st = g_mm_st + k;
-        c.partials = g_mm_part + (size_t)k * g_mm_part_n;
-        c.pred = pred;
-        c.iter = iter;
-        return c;
-    };
     auto hist = [&](int k) { return (char*)g_mm_hist + (size_t)k * hb; };
     auto slot = [&](int k, int j) { return (double2*)(hist(k) + (size_t)((j - 1) % W) * vb); };
 
@@ -1276,8 +1504,8 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
             !hip_ok(hipMemcpyAsync(d.p, d.b, vb, hipMemcpyDeviceToDevice, S()), "p = b") ||
             !reduce_to_host(0, d.b, nullptr, 0, &sn[k], nullptr))
             return false;
-        SolverState& s = g_mm_st_host[k];
-        std::memset(&s, 0, sizeof s);
+        SolverState& s = g_mm_st_host[2 * k];
+        std::memset(&s, 0, 2 * sizeof s);
         s.res = d.residuo;
         s.safety = 0.95;
         s.max_cg = d.max_cg;
@@ -1290,124 +1518,44 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
         s.order = d.order;
         s.flag_cur = 0;
         for (int i = 0; i < d.order; i++) {
-            s.flags[1][i] = 1;
+            s.flags[0][i] = 1;
             s.zeta_i[i] = 1.0;
             s.zeta_ii[i] = 1.0;
             s.gammas[i] = 0.0;
             s.shifts[i] = d.shifts[i];
         }
-        s.maxiter_next = d.order;
+        s.maxiter = d.order;
         if (d.order == 0) s.status = kDone;
     }
-    if (!hip_ok(hipMemcpyAsync(g_mm_st, g_mm_st_host, n * sizeof(SolverState), hipMemcpyHostToDevice, S()),
-                "multi states") ||
-        !hip_ok(hipStreamSynchronize(S()), "multi states"))
+    if (!hip_ok(hipMemcpyAsync(g_mm_st, g_mm_st_host, 2 * n * sizeof(SolverState), hipMemcpyHostToDevice, S()),
+                "multi states"))
         return false;
     for (int k = 0; k < n; k++)
-        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_mm_win + k, ctl_k(k, kAlways));
+        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_mm_win + k, ctl_of(kAlways), 0);
 
-    MsMultiHop a;
-    for (int l = 0; l < 8; l++) {
-        a.u[l] = (const double2*)((const char*)u + l * L.su3_bytes());
-        a.ph[l] = (const double*)((const char*)ph + l * L.dsoa_bytes());
+    KrSys ks[kMsMulti];
+    for (int k = 0; k < n; k++) {
+        ks[k] = KrSys{};
+        ks[k].r = sy[k].r;
+        ks[k].h = sy[k].h;
+        ks[k].s = sy[k].s;
+        ks[k].p = sy[k].p;
+        ks[k].m2 = sy[k].mass * sy[k].mass;
+        ks[k].hist = hist(k);
+        ks[k].win = g_mm_win + k;
+        ks[k].out = sy[k].out;
+        ks[k].shiftferm = sy[k].shiftferm;
+        ks[k].order = sy[k].order;
     }
-    a.g.nd0 = L.nd[0];
-    a.g.nd0h = L.nd[0] / 2;
-    a.g.nd1 = L.nd[1];
-    a.g.nd2 = L.nd[2];
-    a.g.nd3 = L.nd[3];
-    a.g.sizeh = (int)sizeh;
-    a.tmajor = (sizeh / L.nd[3]) % kBlock == 0 ? 1 : 0;  // as k_dslash<double>
-    a.n = n;
-    a.pred = kIfRunning;
-    for (int k = 0; k < kMsMulti; k++) {
-        const int q = k < n ? k : 0;
-        a.st[k] = g_mm_st + q;
-        a.part[k] = g_mm_part + (size_t)q * g_mm_part_n;
-        a.m2[k] = sy[q].mass * sy[q].mass;
-    }
-    auto iteration = [&](int j) -> bool {
-        // h_k = D_oe p_k ; s_k = m2_k p_k - D_eo h_k, <p_k, s_k>
-        for (int k = 0; k < kMsMulti; k++) {
-            const int q = k < n ? k : 0;
-            a.in[k] = (const double2*)sy[q].p;
-            a.out[k] = (double2*)sy[q].h;
-            a.x[k] = nullptr;
-        }
-        a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
-        launch_multi_hop<1>(a, nbh);
-        for (int k = 0; k < kMsMulti; k++) {
-            const int q = k < n ? k : 0;
-            a.in[k] = (const double2*)sy[q].h;
-            a.out[k] = (double2*)sy[q].s;
-            a.x[k] = (const double2*)sy[q].p;
-        }
-        a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
-        launch_multi_hop<0>(a, nbh);
-        for (int k = 0; k < n; k++) {
-            if (!launch_finalize(kFinMsAlpha, ctl_k(k, kIfRunning), nbh)) return false;
-            const double2* r_old = j == 1 ? (const double2*)sy[k].r : slot(k, j - 1);
-            hipLaunchKernelGGL((k_msw_r<double2>), dim3(nbh), dim3(kBlock), 0, S(), r_old, slot(k, j),
-                               (const double2*)sy[k].s, (int)sizeh, ctl_k(k, kIfRunning));
-            if (!launch_finalize(kFinMsLambda, ctl_k(k, kIfRunning), nbh)) return false;
-            hipLaunchKernelGGL((k_msw_p<double2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)sy[k].p,
-                               (const double2*)slot(k, j), n3, g_mm_win + k, ctl_k(k, kIfIter, j),
-                               (double2*)nullptr);
-            if (j % W == 0) {
-                hipLaunchKernelGGL((k_msw_flush<double2, double2>), dim3(nb3), dim3(kBlock), 0, S(),
-                                   (double2*)sy[k].out, (double2*)sy[k].shiftferm, (const double2*)hist(k), n3,
-                                   sy[k].order, (const MsWin*)(g_mm_win + k), ctl_k(k, kIfIter, j));
-                hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_mm_win + k, ctl_k(k, kIfIter, j));
-            }
-        }
-        return check_launch("multi multishift iteration");
-    };
-    // batches as run_batches, sized by the slowest system
-    int batch = 4, last_total = -1;
-    double prev_d = NAN;
-    int last_cg = -1;
-    for (;;) {
-        if (!hip_ok(hipMemcpyAsync(g_mm_st_host, g_mm_st, n * sizeof(SolverState), hipMemcpyDeviceToHost, S()),
-                    "multi states") ||
-            !hip_ok(hipStreamSynchronize(S()), "multi states"))
-            return false;
-        int running = 0, total = 0, cg0 = 0;
-        double d = -INFINITY;
-        for (int k = 0; k < n; k++) {
-            const SolverState& s = g_mm_st_host[k];
-            total += s.cg;
-            if (s.status == kRunning) {
-                running++;
-                cg0 = std::max(cg0, s.cg);
-                const double dk = dist_ms(s);
-                d = std::isfinite(dk) ? std::max(d, dk) : d;
-            }
-        }
-        if (!running) break;
-        if (total == last_total) return fail("multi multishift: solver states did not advance (iteration %d)", cg0);
-        last_total = total;
-        int nq = batch;
-        if (std::isfinite(d) && std::isfinite(prev_d) && last_cg >= 0 && cg0 > last_cg) {
-            const double rate = (prev_d - d) / (double)(cg0 - last_cg);
-            if (rate > 1e-9) {
-                const double left = d > 0.0 ? d / rate : 0.0;
-                nq = std::min(nq, std::max(2, (int)std::ceil(1.1 * left) + 1));
-            }
-        }
-        prev_d = std::isfinite(d) ? d : NAN;
-        last_cg = cg0;
-        for (int j = 1; j <= nq; j++)
-            if (!iteration(cg0 + j)) return false;
-        batch = std::min(2 * batch, 64);
-    }
+    if (!kr_iterate(u, ph, ks, n, true, W, g_mm_st, g_mm_st_host, g_mm_part, g_mm_part_n)) return false;
     // the partial last windows, final residuals, the per-shift check
     for (int k = 0; k < n; k++) {
         MsSys& d = sy[k];
-        const int cg = g_mm_st_host[k].cg;
+        const int cg = g_mm_st_host[2 * k].cg;
         d.cg = cg;
         hipLaunchKernelGGL((k_msw_flush<double2, double2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)d.out,
                            (double2*)d.shiftferm, (const double2*)hist(k), n3, d.order,
-                           (const MsWin*)(g_mm_win + k), ctl_k(k, kAlways));
+                           (const MsWin*)(g_mm_win + k), ctl_of(kAlways), 0);
         if (cg > 0 && !hip_ok(hipMemcpyAsync(d.r, slot(k, cg), vb, hipMemcpyDeviceToDevice, S()), "final residual"))
             return false;
         if (!check_launch("multi multishift window flush")) return false;
@@ -1475,7 +1623,7 @@ static void* grow_buffer(void*& p, size_t& have, size_t need) {
 // ostp_init with the device current) and is kept in g_scratch_dev.
 constexpr long kNoAllocMaxSizeh = 1L << 23;  // half-sites: a 64^4 lattice
 constexpr size_t kNoAllocPartialBytes = sizeof(double) * 4 * (size_t)((kNoAllocMaxSizeh + 63) / 64 + 64);
-constexpr size_t kNoAllocBytes = kNoAllocPartialBytes + ((sizeof(SolverState) + 255) / 256) * 256;
+constexpr size_t kNoAllocBytes = kNoAllocPartialBytes + ((2 * sizeof(SolverState) + 255) / 256) * 256;
 static_assert(kNoAllocPartialBytes % 256 == 0, "state offset alignment");
 static __device__ __align__(256) char scratch[kNoAllocBytes];
 constexpr int kNoAllocMaxDevices = 64;
@@ -1520,19 +1668,13 @@ static bool power_method_multi(const void* u, const void* ph, const double* coef
     const int nbh = blocks_for(sizeh);
     if (n < 1 || n > kMsMulti) return false;
     if (!g_mm_st) {
-        if (!hip_ok(hipMalloc(&g_mm_st, kMsMulti * sizeof(SolverState)), "multi states") ||
-            !hip_ok(hipHostMalloc(&g_mm_st_host, kMsMulti * sizeof(SolverState), hipHostMallocDefault),
+        if (!hip_ok(hipMalloc(&g_mm_st, 2 * kMsMulti * sizeof(SolverState)), "multi states") ||
+            !hip_ok(hipHostMalloc(&g_mm_st_host, 2 * kMsMulti * sizeof(SolverState), hipHostMallocDefault),
                     "multi states") ||
             !hip_ok(hipMalloc(&g_mm_win, kMsMulti * sizeof(MsWin)), "multi windows"))
             return false;
     }
-    if (g_mm_part_n < (size_t)2 * nbh) {
-        if (g_mm_part) (void)hipFree(g_mm_part);
-        g_mm_part = nullptr;
-        g_mm_part_n = 0;
-        if (!hip_ok(hipMalloc(&g_mm_part, sizeof(double) * 2 * nbh * kMsMulti), "multi partials")) return false;
-        g_mm_part_n = (size_t)2 * nbh;
-    }
+    if (!mm_partials()) return false;
     auto ctl_k = [&](int k, int pred) {
         SolverCtl c;
         c.st = g_mm_st + k;
@@ -2201,7 +2343,7 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
         }
         hist = (float2*)g_msw_hist;
         if (!g_msw && !hip_ok(hipMalloc(&g_msw, sizeof(MsWin)), "multishift window")) return 0;
-        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kAlways));
+        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kAlways), 0);
     }
     // Reliable updates are taken at every kMsxRuEvery-th iteration (when the
     // FP32 residual has fallen by mixed_delta since the last one): the other
@@ -2233,8 +2375,8 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
         if (j % W == 0) {
             // only when iteration j ran: a window cut short is flushed once, at the end
             hipLaunchKernelGGL((k_msw_flush<double2, float2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)dout,
-                               (float2*)pk, (const float2*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kIfIter, j));
-            hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kIfIter, j));
+                               (float2*)pk, (const float2*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kIfIter, j), 0);
+            hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kIfIter, j), 0);
         }
         return check_launch("mixed multishift iteration");
     };
@@ -2243,7 +2385,7 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
     if (cg_multishift) *cg_multishift = cg;
     if (hist)
         hipLaunchKernelGGL((k_msw_flush<double2, float2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)dout,
-                           (float2*)pk, (const float2*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kAlways));
+                           (float2*)pk, (const float2*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kAlways), 0);
     hipLaunchKernelGGL(k_msx_flush, dim3(nb3), dim3(kBlock), 0, S(), fl, n3, ctl_of(kAlways));
     if (!check_launch("flush")) return 0;
     if (verbosity_lv > 1 && !hip_ok(hipStreamSynchronize(S()), "timing")) return 0;

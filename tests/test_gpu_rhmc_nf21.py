@@ -329,6 +329,36 @@ def test_nf21_rhmc_update_second_order():
             set_ptr(name, None)
 
 
+
+@pytest.mark.parametrize("shape, ps", [((2, 2, 2, 2), (1, 1)), ((6, 4, 4, 10), (2, 1)), ((4, 4, 4, 8), (2, 2)),
+                                       ((16, 16, 16, 26), (2, 1))])
+def test_systems_iterated_together_match_one_by_one(shape, ps):
+    """Two, three and four systems in one CG-M iteration stream, on lattices
+    with blocks that are not full and on one too large for split hops: the
+    force is that of the one-by-one solves bit for bit."""
+    F = Nf21(shape)
+    vb = F.lat.vec3_bytes
+    F.chi = Dev(nbytes=sum(ps) * vb)
+    for k in range(sum(ps)):
+        lib.ostp_generate_vec3_soa_gauss(F.chi.p + k * vb, 77, 10 + k)
+    for f in range(2):
+        F.fps[f].ferm_mass = 0.1 + 0.1 * f
+        F.fps[f].number_of_ps, F.fps[f].index_of_the_first_ps = ps[f], f * ps[0]
+    du = Dev(F.u0)
+    forces = []
+    for batch in (1, 0):
+        prev = lib.ostp_set_multishift_batching(batch)
+        try:
+            ipd = Dev(nbytes=F.tb)
+            lib.fermion_force_soloopenacc(du.p, F.arr.p, F.gl3.p, ipd.p, F.fps, 2, F.chi.p, F.res, F.taux.p, F.xs.p,
+                                          F.ip(du.p), 50000)
+            ost.check(0, "fermion_force_soloopenacc")
+        finally:
+            lib.ostp_set_multishift_batching(prev)
+        forces.append(ipd.get(np.zeros(F.tb // 8)))
+    assert np.abs(forces[0]).max() > 1e-3 and np.array_equal(forces[0], forces[1]), rel(forces[0], forces[1])
+
+
 def test_config5_trajectory_reversible_48x48x48x12():
     F = Nf21((48, 48, 48, 12), eps=0.5, seed=7, res=1e-10)
     moved, back_u, back_m = forward_back(F, 10, 5, 1.0, 2026)

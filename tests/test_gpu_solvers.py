@@ -560,3 +560,38 @@ def test_config2_full_shape():
     lib.ostp_set_inverter_tricks(0, 0, 0.1, 10000)
     ost.check(0, "inverter_multishift_wrapper")
     assert worst_true_residual(out) <= 1e-10 and worst_rel_err(out, x64) < 1e-6
+
+
+# 8 and 480 half-sites (less than a block, a last block that is not full), the
+# last lattice whose hops are split over waves (49152 half-sites) and one above it
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (6, 4, 4, 10), (16, 16, 16, 24), (16, 16, 16, 26)])
+def test_solver_iterations_at_block_edges(shape):
+    """CG (with restarts) and CG-M (three shifts, windows and per-iteration
+    updates) against the oracle: the solutions differ by at most both
+    residuals times the condition number (bounded by 1 + 4 * 16 / m^2)."""
+    mass = 0.4
+    s = Sys(shape, seed=9, kind="cold", param=0.4, mass=mass)
+    cond = 1 + 64 / mass ** 2
+    st, cg, x, tr = s.cg(1e-10, restart=12)
+    ost_, ocg, ox = s.o.cg(s.u, s.ph, mass, s.b, 1e-10, restart=12)
+    assert st == 1 and ost_ == 1 and tr <= 1e-10 and iters_close(cg, ocg), (st, ost_, cg, ocg)
+    assert rel(x, ox) < 2e-10 * cond
+    ra = remez19(mass)
+    ra.approx_order = 3
+    vb = s.b.nbytes
+    b = np.array([ra.RA_b[k] for k in range(3)])
+    _, mcg, mx = s.o.multishift(s.u, s.ph, mass, b, s.b, 1e-10)[:3]
+    for w in (1, 8):
+        prev = lib.ostp_set_multishift_window(w)
+        try:
+            out, sf = Dev(nbytes=3 * vb), Dev(nbytes=3 * vb)
+            cg = C.c_int(0)
+            st = lib.multishift_invert(s.du.p, C.byref(s.fp), C.byref(ra), out.p, s.db.p, 1e-10,
+                                       *(d.p for d in s.scratch), sf.p, 10000, C.byref(cg))
+            ost.check(0, "multishift_invert")
+        finally:
+            lib.ostp_set_multishift_window(prev)
+        assert st == 1 and iters_close(cg.value, mcg), (w, cg.value, mcg)
+        got = out.get(np.zeros((3, 3, s.o.sizeh), dtype=np.complex128))
+        for k in range(3):
+            assert rel(got[k], mx[k]) < 2e-10 * cond, (w, k)
