@@ -158,8 +158,6 @@ bool launch_finalize(int fin, const SolverCtl& c, int nparts) {
         case kFinMxmAlpha: OSTP_F(kFinMxmAlpha, 1); break;
         case kFinPower: OSTP_F(kFinPower, 1); break;
         case kFinMxmLambda: OSTP_F(kFinMxmLambda, 1); break;
-        case kFinMxAlpha: OSTP_F(kFinMxAlpha, 1); break;
-        case kFinMxLambda: OSTP_F(kFinMxLambda, 1); break;
         case kFinFcgAlpha: OSTP_F(kFinFcgAlpha, 1); break;
         case kFinFcgRes: OSTP_F(kFinFcgRes, 1); break;
         case kFinFcgBeta: OSTP_F(kFinFcgBeta, 2); break;

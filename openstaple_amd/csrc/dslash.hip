@@ -29,6 +29,8 @@ struct DslashArgs {
     C* out;
     const C* x;         // epilogue input: out = m2*x - D in
     double m2;
+    const double2* b;   // kMdagMResid
+    float2* rf;
     SiteGeom g;
     int tmajor;         // workgroup order: t-slices fastest (see k_dslash)
     int rev;            // each XCD walks its slab backwards
@@ -68,6 +70,19 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<R> a) {
                 a.out[a.g.sizeh + idx] = o1;
                 a.out[2 * a.g.sizeh + idx] = o2;
             }
+        } else if constexpr (MODE == kMdagMResid) {
+            // r_f = (float)(b - (x*m2 - D in)), |r_f|^2; the FP64 product itself is not stored
+            const C o[3] = {o0, o1, o2};
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const long k = (long)c * a.g.sizeh + idx;
+                const C xx = a.x[k];
+                const double2 bb = a.b[k];
+                const double sx = (double)xx.x * a.m2 - (double)o[c].x, sy = (double)xx.y * a.m2 - (double)o[c].y;
+                const float2 f = make_float2((float)(bb.x - sx), (float)(bb.y - sy));
+                a.rf[k] = f;
+                dot += (double)f.x * f.x + (double)f.y * f.y;
+            }
         } else {
             // combine_in1xferm_mass_minus_in2: out = x*m2 - D in  (promoted to double)
             const C x0 = a.x[idx], x1 = a.x[a.g.sizeh + idx], x2 = a.x[2 * a.g.sizeh + idx];
@@ -88,7 +103,7 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<R> a) {
         }
     }
     // partial slot = logical tile, so the reduction order is the same in both walk directions
-    if (MODE == kMdagMDot) block_partial_at<kBlock>(dot, 0.0, a.ctl.partials, blk);
+    if (MODE >= kMdagMDot) block_partial_at<kBlock>(dot, 0.0, a.ctl.partials, blk);
 }
 
 // ---------------------------------------------------------------- launchers
@@ -107,6 +122,8 @@ static bool fill_args(DslashArgs<R>& a, const void* u_dev, const void* ph_dev, c
     a.out = (C*)out_dev;
     a.x = nullptr;
     a.m2 = 0.0;
+    a.b = nullptr;
+    a.rf = nullptr;
     a.g.nd0 = L.nd[0];
     a.g.nd0h = L.nd[0] / 2;
     a.g.nd1 = L.nd[1];
@@ -139,8 +156,7 @@ bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, con
         if (eo == 0) OSTP_L(0, kMdagM); else OSTP_L(1, kMdagM);
     } else {
         if (eo != 0) return fail("fused dot epilogue only on Deo");
-        if (fin != kFinNone && fin != kFinStore && fin != kFinMsAlpha && fin != kFinMxAlpha && fin != kFinFcgAlpha &&
-            fin != kFinMxmAlpha)
+        if (fin != kFinNone && fin != kFinStore && fin != kFinMsAlpha && fin != kFinFcgAlpha && fin != kFinMxmAlpha)
             return fail("unsupported dslash finalizer %d", fin);
         OSTP_L(0, kMdagMDot);
     }
@@ -153,6 +169,24 @@ template bool launch_dslash<double>(int, int, int, const void*, const void*, con
                                     double, const SolverCtl&);
 template bool launch_dslash<float>(int, int, int, const void*, const void*, const void*, void*, const void*,
                                    double, const SolverCtl&);
+
+// The two hops of a reliable update: temp = Doe x, then r_f = (float)(b - M x)
+// with the block partials of |r_f|^2.
+bool launch_mdagm_resid(const void* u, const void* ph, const void* x, void* temp, const void* b, void* rf, double m2,
+                        const SolverCtl& ctl) {
+    if (!launch_dslash<double>(1, kPlain, kFinStore, u, ph, x, temp, nullptr, 0.0, ctl)) return false;
+    DslashArgs<double> a;
+    fill_args<double>(a, u, ph, temp, nullptr);
+    a.x = (const double2*)x;
+    a.m2 = m2;
+    a.b = (const double2*)b;
+    a.rf = (float2*)rf;
+    a.ctl = ctl;
+    a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
+    hipLaunchKernelGGL((k_dslash<double, 0, kMdagMResid>), dim3(blocks_for(ctx().lat.sizeh)), dim3(kBlock), 0,
+                       ctx().stream, a);
+    return hip_ok(hipGetLastError(), "k_dslash launch");
+}
 
 // M = (m^2+shift) - Deo Doe on device pointers; temp receives Doe in.
 template <typename R>

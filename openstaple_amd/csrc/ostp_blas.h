@@ -22,6 +22,9 @@ bool launch_doe_multi(const void* u, const void* ph, const void* xs, void* hs, i
 template <typename R>
 bool launch_mdagm(const void* u, const void* ph, const void* in, void* temp, void* out, double m2, int mode,
                   int fin, const SolverCtl& ctl);
+// temp = Doe x, r_f = (float)(b - M x), block partials of |r_f|^2 (two doubles a block)
+bool launch_mdagm_resid(const void* u, const void* ph, const void* x, void* temp, const void* b, void* rf, double m2,
+                        const SolverCtl& ctl);
 
 // BLAS (blas.hip)
 template <typename C>

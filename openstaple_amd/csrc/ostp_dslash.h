@@ -13,7 +13,7 @@ template <typename R> struct Cplx;
 template <> struct Cplx<double> { using T = double2; };
 template <> struct Cplx<float> { using T = float2; };
 
-enum DslashMode : int { kPlain = 0, kMdagM = 1, kMdagMDot = 2 };
+enum DslashMode : int { kPlain = 0, kMdagM = 1, kMdagMDot = 2, kMdagMResid = 3 };
 
 
 // FP32 phases are evaluated in double (eight per site; the kernel is

@@ -602,4 +602,181 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
     if (tid == 0) a.partB[k][blockIdx.x] = t;
 }
 
+// ---- mixed-precision CG with reliable updates (inverter_mixedp.c:54-155) ----
+// FP32 iterations in four launches: k_mx_p ends iteration j - 1 and forms p,
+// the two ordinary FP32 hops follow, k_mx_xr takes the step.  Whether iteration
+// j is a reliable update is known when it starts (delta against the largest
+// since the last one), so its k_mx_xr adds the step to x instead and the FP64
+// residual comes from two predicated launches, queued after every
+// kMxTailEvery-th iteration only: an update that falls between two of them
+// pauses the solver (hold) until the next.  79 iterations on 32^3 x 8: 4370
+// us with nine launches each, four of them for an update that seldom came, 3747
+// so (21 us an iteration in the FP32 hops, 10 in these two kernels).
+constexpr int kMxTailEvery = 2;
+struct MxArgs {
+    float2 *pf, *rf, *outf;
+    const float2* sf;
+    double2* x;
+    SolverState* st;      // two copies, as KrArgs
+    const double* partA;  // <p, s>, two doubles a block
+    double* partB;        // |r|^2 of k_mx_xr
+    const double* partT;  // |r|^2 of a reliable update, two doubles a block
+    int nA, nB, nT, sizeh;
+    int j, close;
+    int tail;             // the update's launches were queued after iteration j - 1
+};
+
+// p = r + gamma p in the precision of k_cg_p<float2>
+__device__ __forceinline__ float2 mx_p(float2 r, float2 p, double g) {
+    return make_float2((float)((double)p.x * g + (double)r.x), (float)((double)p.y * g + (double)r.y));
+}
+
+__global__ __launch_bounds__(kBlock) void k_mx_p(MxArgs a) {
+    __shared__ double sh_gamma;
+    __shared__ int sh_run;
+    const int tid = (int)threadIdx.x, sh = a.sizeh;
+    const int i0 = (int)blockIdx.x * kBlock + tid, step = (int)gridDim.x * kBlock;
+    float2 rr[kKrAhead][3], pp[kKrAhead][3];
+#pragma unroll
+    for (int q = 0; q < kKrAhead; q++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const long e = (long)c * sh + (i0 + q * step < sh ? i0 + q * step : 0);
+            rr[q][c] = a.rf[e];
+            pp[q][c] = a.pf[e];
+        }
+    if (tid < 64) {
+        const SolverState* prev = a.st + ((a.j - 1) & 1);
+        SolverState* next = a.st + (a.j & 1);
+        double sum = 0.0, sumt = 0.0;
+        if (a.j > 1) sum = kr_part(a.partB, a.nB, 1, tid);
+        if (a.tail) sumt = kr_part(a.partT, a.nT, 2, tid);
+        double delta = prev->delta, lambda = prev->lambda, g = 0.0, last = prev->last_max_res;
+        int status = prev->status, cg = prev->cg, rus = prev->ru_count, ru = prev->ru;
+        const bool hold = a.j > 1 && status == kRunning && ru && !a.tail;
+        if (a.j > 1 && status == kRunning && !hold) {
+            lambda = kr_wave(ru ? sumt : sum);
+            g = lambda / delta;
+            delta = lambda;
+            cg += 1;
+            if (ru) {
+                last = 0.0;
+                rus += 1;
+            }
+            const bool cont = (sqrt(lambda / prev->source_norm) > prev->res * prev->safety) && cg < prev->max_cg;
+            if (!cont) status = kDone;
+        }
+        if (status == kRunning && !hold) {
+            if (last < delta) last = delta;
+            ru = (delta < prev->mixed_delta * last) ? 1 : 0;
+        }
+        if (tid == 0) {
+            sh_gamma = g;
+            sh_run = status == kRunning && !hold;
+            if (blockIdx.x == 0) {
+                next->delta = delta;
+                next->lambda = lambda;
+                next->gammag = g;
+                next->alpha = prev->alpha;
+                next->omega = prev->omega;
+                next->source_norm = prev->source_norm;
+                next->res = prev->res;
+                next->safety = prev->safety;
+                next->last_max_res = last;
+                next->mixed_delta = prev->mixed_delta;
+                next->cg = cg;
+                next->max_cg = prev->max_cg;
+                next->status = status;
+                next->ru = ru;
+                next->hold = hold;
+                next->ru_count = rus;
+            }
+        }
+    }
+    __syncthreads();
+    if (!sh_run || a.close) return;
+    const double g = sh_gamma;
+#pragma unroll
+    for (int q = 0; q < kKrAhead; q++)
+        if (i0 + q * step < sh)
+#pragma unroll
+            for (int c = 0; c < 3; c++) a.pf[(long)c * sh + i0 + q * step] = mx_p(rr[q][c], pp[q][c], g);
+    for (int i = i0 + kKrAhead * step; i < sh; i += step)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const long e = (long)c * sh + i;
+            a.pf[e] = mx_p(a.rf[e], a.pf[e], g);
+        }
+}
+
+// out_f += omega p_f; then either r_f -= omega s_f with |r_f|^2, or (reliable
+// update) x += out_f, out_f = 0   (inverter_mixedp.c:107-134)
+__global__ __launch_bounds__(kBlock) void k_mx_xr(MxArgs a) {
+    SolverState* st = a.st + (a.j & 1);
+    __shared__ double lds[kBlock / 64];
+    __shared__ double sh_om;
+    __shared__ int sh_go, sh_ru;
+    const int tid = (int)threadIdx.x, sh = a.sizeh;
+    const int i0 = (int)blockIdx.x * kBlock + tid, step = (int)gridDim.x * kBlock;
+    float2 pa[kKrAhead][3], oa[kKrAhead][3], ra[kKrAhead][3], sa[kKrAhead][3];
+#pragma unroll
+    for (int q = 0; q < kKrAhead; q++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const long e = (long)c * sh + (i0 + q * step < sh ? i0 + q * step : 0);
+            pa[q][c] = a.pf[e];
+            oa[q][c] = a.outf[e];
+            ra[q][c] = a.rf[e];
+            sa[q][c] = a.sf[e];
+        }
+    if (tid < 64) {
+        const double part = kr_part(a.partA, a.nA, 2, tid);
+        const int go = st->status == kRunning && !st->hold, ru = st->ru;
+        const double tot = kr_wave(part), om = st->delta / tot;
+        if (tid == 0) {
+            sh_om = om;
+            sh_go = go;
+            sh_ru = ru;
+            if (blockIdx.x == 0 && go) {
+                st->alpha = tot;
+                st->omega = om;
+            }
+        }
+    }
+    __syncthreads();
+    if (!sh_go) return;
+    const double om = sh_om;
+    const int ru = sh_ru;
+    double v = 0.0;
+    auto one = [&](long e, float2 pp, float2 oo, float2 rr, float2 ss) {
+        const float2 on =
+            make_float2((float)((double)pp.x * om + (double)oo.x), (float)((double)pp.y * om + (double)oo.y));
+        if (ru) {
+            const double2 xx = a.x[e];
+            a.x[e] = make_double2(xx.x + (double)on.x, xx.y + (double)on.y);
+            a.outf[e] = make_float2(0.f, 0.f);
+            return;
+        }
+        const float2 rn =
+            make_float2((float)((double)ss.x * (-om) + (double)rr.x), (float)((double)ss.y * (-om) + (double)rr.y));
+        a.outf[e] = on;
+        a.rf[e] = rn;
+        v += (double)rn.x * rn.x + (double)rn.y * rn.y;
+    };
+#pragma unroll
+    for (int q = 0; q < kKrAhead; q++)
+        if (i0 + q * step < sh)
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+                one((long)c * sh + i0 + q * step, pa[q][c], oa[q][c], ra[q][c], sa[q][c]);
+    for (int i = i0 + kKrAhead * step; i < sh; i += step)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const long e = (long)c * sh + i;
+            one(e, a.pf[e], a.outf[e], a.rf[e], a.sf[e]);
+        }
+    const double t = block_sum<kBlock>(v, lds);
+    if (tid == 0) a.partB[blockIdx.x] = t;
+}
+
 }  // namespace ostp

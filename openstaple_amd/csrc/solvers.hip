@@ -402,61 +402,6 @@ __global__ __launch_bounds__(kBlock) void k_mx_init(const double2* __restrict__ 
     block_partial<1>(v, 0.0, ctl);
 }
 
-// out_f += omega p_f; then either r_f -= omega s_f with lambda = |r_f|^2, or
-// (reliable update) x += out_f, out_f = 0   (inverter_mixedp.c:107-134)
-__global__ __launch_bounds__(kBlock) void k_mx_xr(float2* __restrict__ outf, const float2* __restrict__ pf,
-                                                  float2* __restrict__ rf, const float2* __restrict__ sf,
-                                                  double2* __restrict__ x, int sizeh, SolverCtl ctl) {
-    if (!pred_pass(ctl)) return;
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    const double om = ctl.st->omega;
-    const int ru = ctl.st->ru;
-    double v = 0.0;
-    if (i < sizeh) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const long k = (long)c * sizeh + i;
-            const float2 pp = pf[k], oo = outf[k];
-            const float2 on = make_float2((float)((double)pp.x * om + (double)oo.x), (float)((double)pp.y * om + (double)oo.y));
-            if (!ru) {
-                outf[k] = on;
-                const float2 ss = sf[k], rr = rf[k];
-                const float2 rn = make_float2((float)((double)ss.x * (-om) + (double)rr.x),
-                                              (float)((double)ss.y * (-om) + (double)rr.y));
-                rf[k] = rn;
-                v += (double)rn.x * rn.x + (double)rn.y * rn.y;
-            } else {
-                const double2 xx = x[k];
-                x[k] = make_double2(xx.x + (double)on.x, xx.y + (double)on.y);
-                outf[k] = make_float2(0.f, 0.f);
-            }
-        }
-    }
-    if (!ru) block_partial<1>(v, 0.0, ctl);
-}
-
-// reliable update tail: r = b - s (FP64), r_f = (float) r, lambda = |r_f|^2  (inverter_mixedp.c:121-124,137)
-__global__ __launch_bounds__(kBlock) void k_mx_resid(const double2* __restrict__ b, const double2* __restrict__ s,
-                                                     double2* __restrict__ r64, float2* __restrict__ rf, int sizeh,
-                                                     SolverCtl ctl) {
-    if (!pred_pass(ctl)) return;
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    double v = 0.0;
-    if (i < sizeh) {
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const long k = (long)c * sizeh + i;
-            const double2 bb = b[k], ss = s[k];
-            const double2 rr = make_double2(bb.x - ss.x, bb.y - ss.y);
-            r64[k] = rr;
-            const float2 f = make_float2((float)rr.x, (float)rr.y);
-            rf[k] = f;
-            v += (double)f.x * f.x + (double)f.y * f.y;
-        }
-    }
-    block_partial<1>(v, 0.0, ctl);
-}
-
 // x += (double) out_f   (combine_add_in2_into_in1_mixed_precision, inverter_mixedp.c:24-34)
 __global__ __launch_bounds__(kBlock) void k_add_f_to_d(double2* __restrict__ x, const float2* __restrict__ f, long n3) {
     const long i = (long)blockIdx.x * kBlock + threadIdx.x;
@@ -600,6 +545,20 @@ static double kr_dist(const SolverState& s, bool ms) {
     return 0.5 * std::log(m / s.source_norm) - std::log(s.res * s.safety);
 }
 
+// The next batch after one of `batch` that ended at iteration j, a distance d
+// from the target: the iterations left at the convergence rate of that batch,
+// with a margin, at most twice as many and at most 64.
+static int kr_batch(int batch, double d, double* prev_d, int j, int* prev_j) {
+    batch = std::min(2 * batch, 64);
+    if (std::isfinite(d) && std::isfinite(*prev_d)) {
+        const double rate = (*prev_d - d) / (double)(j - *prev_j);
+        if (rate > 1e-9) batch = std::min(batch, std::max(2, (int)std::ceil(1.1 * std::max(d, 0.0) / rate) + 1));
+    }
+    *prev_d = d;
+    *prev_j = j;
+    return batch;
+}
+
 // Iterate n systems from the states in st (copies 0; pinned mirror st_host)
 // until none runs.  part: room for n x (hop blocks + r blocks) partials.  On
 // return st_host[2 k] holds system k's last state.
@@ -712,14 +671,7 @@ static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bo
         // a running solver's counter advances with every iteration
         if (total == last_total) return fail("solver state did not advance (iteration %d)", j);
         last_total = total;
-        // the iterations left at the convergence rate so far, with a margin
-        batch = std::min(2 * batch, 64);
-        if (std::isfinite(d) && std::isfinite(prev_d)) {
-            const double rate = (prev_d - d) / (double)(j - prev_j);
-            if (rate > 1e-9) batch = std::min(batch, std::max(2, (int)std::ceil(1.1 * std::max(d, 0.0) / rate) + 1));
-        }
-        prev_d = d;
-        prev_j = j;
+        batch = kr_batch(batch, d, &prev_d, j, &prev_j);
     }
 }
 
@@ -856,6 +808,7 @@ int mixed_solve(const MxBufs& B, double mass, double shift, double res, int max_
     if (!source_norm(B.b, &sn)) return INVERTER_FAILURE;
     init_state(res, 0.9, max_cg, 0);
     H().source_norm = sn;
+    H().delta = sn;  // the distance from the target at the start
     H().mixed_delta = mixed_delta;
     if (!push_state()) return INVERTER_FAILURE;
 
@@ -865,22 +818,52 @@ int mixed_solve(const MxBufs& B, double mass, double shift, double res, int max_
                        (double2*)B.r, (float2*)B.rf, (float2*)B.pf, (float2*)B.outf, (int)sizeh, ctl_of(kAlways));
     if (!check_launch("k_mx_init") || !launch_finalize(kFinCgRestart, ctl_of(kAlways), nbh)) return INVERTER_FAILURE;
 
-    auto iteration = [&](int j) -> bool {
-        if (!launch_mdagm<float>(B.u_f, B.ph_f, B.pf, B.hf, B.sf, m2f, 2, kFinMxAlpha, ctl_of(kIfRunning)))
-            return false;
-        hipLaunchKernelGGL(k_mx_xr, dim3(nbh), dim3(kBlock), 0, S(), (float2*)B.outf, (const float2*)B.pf,
-                           (float2*)B.rf, (const float2*)B.sf, (double2*)B.x, (int)sizeh, ctl_of(kIfRunning));
-        if (!launch_finalize(kFinMxLambda, ctl_of(kIfRunningNoRU), nbh)) return false;
-        // reliable update: s = M x (FP64), r = b - s, r_f = (float) r
-        if (!launch_mdagm<double>(B.u, B.ph, B.x, B.h, B.s, m2, 1, kFinStore, ctl_of(kIfRunningRU))) return false;
-        hipLaunchKernelGGL(k_mx_resid, dim3(nbh), dim3(kBlock), 0, S(), (const double2*)B.b, (const double2*)B.s,
-                           (double2*)B.r, (float2*)B.rf, (int)sizeh, ctl_of(kIfRunningRU));
-        if (!launch_finalize(kFinMxLambda, ctl_of(kIfRunningRU), nbh)) return false;
-        hipLaunchKernelGGL((k_cg_p<float2>), dim3(nb3), dim3(kBlock), 0, S(), (float2*)B.pf, (const float2*)B.rf, n3,
-                           ctl_of(kIfIter, j));
-        return check_launch("mixed iteration");
-    };
-    if (!run_batches(iteration, 4, dist_cg)) return INVERTER_FAILURE;
+    MxArgs a{};
+    a.pf = (float2*)B.pf;
+    a.rf = (float2*)B.rf;
+    a.outf = (float2*)B.outf;
+    a.sf = (const float2*)B.sf;
+    a.x = (double2*)B.x;
+    a.st = ctx().state;
+    a.nA = a.nT = nbh;
+    a.nB = kr_blocks_r();
+    a.partA = ctx().partials;
+    a.partT = ctx().partials + 2 * nbh;
+    a.partB = ctx().partials + 4 * nbh;
+    a.sizeh = (int)sizeh;
+    int j = 0, batch = 16, prev_j = 0, last_cg = -1;
+    double prev_d = kr_dist(H(), false);
+    for (;;) {
+        for (int i = 0; i < batch; i++) {
+            a.j = ++j;
+            a.close = 0;
+            hipLaunchKernelGGL(k_mx_p, dim3(a.nB), dim3(kBlock), 0, S(), a);
+            SolverCtl c = ctl_of(kIfGoing);
+            c.st = a.st + (j & 1);
+            if (!launch_dslash<float>(1, kPlain, kFinStore, B.u_f, B.ph_f, B.pf, B.hf, nullptr, 0.0, c) ||
+                !launch_dslash<float>(0, kMdagMDot, kFinNone, B.u_f, B.ph_f, B.hf, B.sf, B.pf, m2f, c))
+                return INVERTER_FAILURE;
+            hipLaunchKernelGGL(k_mx_xr, dim3(a.nB), dim3(kBlock), 0, S(), a);
+            a.tail = j % kMxTailEvery == 0;
+            if (!a.tail) continue;
+            c.pred = kIfRunningRU;
+            c.partials = ctx().partials + 2 * nbh;
+            if (!launch_mdagm_resid(B.u, B.ph, B.x, B.h, B.b, B.rf, m2, c)) return INVERTER_FAILURE;
+        }
+        a.j = j + 1;
+        a.close = 1;
+        hipLaunchKernelGGL(k_mx_p, dim3(1), dim3(kBlock), 0, S(), a);
+        if (!check_launch("mixed iterations") ||
+            !hip_ok(hipMemcpyAsync(&H(), a.st + ((j + 1) & 1), sizeof(SolverState), hipMemcpyDeviceToHost, S()),
+                    "solver state") ||
+            !hip_ok(hipStreamSynchronize(S()), "solver state"))
+            return INVERTER_FAILURE;
+        const SolverState& s = H();
+        if (s.status != kRunning) break;
+        if (s.cg == last_cg) return fail("solver state did not advance (iteration %d)", s.cg) ? 0 : INVERTER_FAILURE;
+        last_cg = s.cg;
+        batch = kr_batch(batch, kr_dist(s, false), &prev_d, j, &prev_j);
+    }
     const int cg = H().cg;
     if (ru_count) *ru_count = H().ru_count;
     hipLaunchKernelGGL(k_add_f_to_d, dim3(nb3), dim3(kBlock), 0, S(), (double2*)B.x, (const float2*)B.outf, n3);

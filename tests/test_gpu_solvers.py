@@ -595,3 +595,42 @@ def test_solver_iterations_at_block_edges(shape):
         got = out.get(np.zeros((3, 3, s.o.sizeh), dtype=np.complex128))
         for k in range(3):
             assert rel(got[k], mx[k]) < 2e-10 * cond, (w, k)
+
+
+# delta 0.9: nearly every second iteration is a reliable update, also right
+# after one another and in the last iteration of a batch
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (6, 4, 4, 10), (16, 16, 16, 8)])
+@pytest.mark.parametrize("delta", [0.1, 0.9])
+def test_mixed_iterations_at_block_edges(shape, delta):
+    """The FP32 iterations with FP64 reliable updates against the oracle's:
+    the true residual (FP64, the oracle's operator), the iterations (FP32
+    rounding moves their number by a tenth at most, one on a small count), and
+    a solve cut short by max_cg."""
+    mass = 0.2
+    s = Sys(shape, seed=4, kind="cold", param=0.4, mass=mass)
+    uf, phf = s.o.to_float_gauge(s.u), s.ph.astype(np.float32)
+    duf, dphf = Dev(uf), Dev(phf)
+    fp = ost.ferm_param(mass, s.dph.p, dphf.p)
+    vb = s.b.nbytes
+    d32 = [Dev(nbytes=vb // 2) for _ in range(5)]
+    ip = ost.InverterPackage()
+    ip.u, ip.u_f = s.du.p, duf.p
+    ip.loc_r, ip.loc_h, ip.loc_s, ip.loc_p = (d.p for d in s.scratch)
+    ip.loc_r_f, ip.loc_h_f, ip.loc_s_f, ip.loc_p_f, ip.out_f = (d.p for d in d32)
+    x = Dev(nbytes=vb)
+    cg, ru, tr = C.c_int(0), C.c_int(0), C.c_double(0)
+    args = (C.byref(cg), C.byref(ru), C.byref(tr))
+    x.put(np.zeros_like(s.b))
+    st = lib.ostp_mixed_solve(ip, C.byref(fp), x.p, s.db.p, 1e-10, 10000, 0.0, delta, *args)
+    ost.check(0, "ostp_mixed_solve")
+    r = s.b - s.o.mdagm(s.u, x.get(s.b), s.ph, mass)
+    assert st == 1 and ru.value >= 1 and np.linalg.norm(r) / np.linalg.norm(s.b) <= 1e-10
+    ost_, ocg, _ = s.o.mixed(s.u, uf, s.ph, phf, mass, s.b, 1e-10, delta=delta)
+    assert ost_ == 1 and abs(cg.value - ocg) <= max(1, 0.1 * ocg), (cg.value, ocg)
+    x.put(np.zeros_like(s.b))
+    st = lib.ostp_mixed_solve(ip, C.byref(fp), x.p, s.db.p, 1e-10, 5, 0.0, delta, *args)
+    ost.check(0, "ostp_mixed_solve")
+    assert st == 0 and cg.value == 5
+    r = s.b - s.o.mdagm(s.u, x.get(s.b), s.ph, mass)
+    # the FP64 residual of what the five FP32 steps added
+    assert abs(np.linalg.norm(r) / np.linalg.norm(s.b) - tr.value) <= 1e-6 * tr.value
