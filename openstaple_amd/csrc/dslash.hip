@@ -7,7 +7,8 @@
 // with only rows 0,1 of each link read (row 2 = conj(row0 x row1)) and the
 // U(1) phase e^{i th} = cos th + i sin th folded in at load time.
 //
-// One thread per output half-site; consecutive lanes own consecutive
+// One thread per output half-site (k_dslash; k_dslash_split spreads a site's
+// hops over eight waves where that is faster); consecutive lanes own consecutive
 // half-sites, so every SoA plane access is a fully coalesced 128-bit (FP64)
 // or 64-bit (FP32) load.  Workgroups are remapped so each XCD streams a
 // contiguous slab of the lattice and its L2 serves the neighbour-spinor
@@ -37,76 +38,150 @@ struct DslashArgs {
     SolverCtl ctl;
 };
 
+template <typename C>
+__device__ __forceinline__ void st_out(C* p, C v) {
+    if constexpr (sizeof(C) == 16) st_nt(p, v);
+    else *p = v;
+}
+
+// What a half-site's colour does with o = (D in): element k; the return value
+// is its term of the fused reduction.
+template <typename R, int MODE>
+__device__ __forceinline__ double dslash_out(const DslashArgs<R>& a, long k, typename Cplx<R>::T o,
+                                             typename Cplx<R>::T x) {
+    using C = typename Cplx<R>::T;
+    if constexpr (MODE == kPlain) {
+        st_out(a.out + k, o);
+        return 0.0;
+    }
+    // combine_in1xferm_mass_minus_in2: out = x*m2 - D in  (promoted to double)
+    const double sx = (double)x.x * a.m2 - (double)o.x, sy = (double)x.y * a.m2 - (double)o.y;
+    if constexpr (MODE == kMdagMResid) {
+        // r_f = (float)(b - (x*m2 - D in)), |r_f|^2; the FP64 product itself is not stored
+        const double2 bb = a.b[k];
+        const float2 f = make_float2((float)(bb.x - sx), (float)(bb.y - sy));
+        a.rf[k] = f;
+        return (double)f.x * f.x + (double)f.y * f.y;
+    }
+    const C sv = mk<C>(sx, sy);
+    st_out(a.out + k, sv);
+    return MODE == kMdagMDot ? re_dot(x, sv) : 0.0;
+}
+
+// Workgroup -> sites: the XCD remap gives each XCD a contiguous range of
+// logical tiles; with tmajor the logical tile index runs over t fastest,
+// so the +-t neighbour slices of a tile are streamed by the same XCD at
+// nearly the same time and its L2 serves their re-reads (FP64: 81.2 us vs
+// 85.5 us per 32^4 Dslash).
+template <typename R>
+__device__ __forceinline__ int dslash_idx(const DslashArgs<R>& a, int blk, int sites, int i) {
+    if (a.tmajor) {
+        const int s3 = a.g.sizeh / a.g.nd3;
+        const int tile = blk / a.g.nd3, tt = blk - tile * a.g.nd3;
+        return tt * s3 + tile * sites + i;
+    }
+    return blk * sites + i;
+}
+
 // EO = 0: Deo (even output, odd input); EO = 1: Doe.
 template <typename R, int EO, int MODE>
 __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<R> a) {
     using C = typename Cplx<R>::T;
     if (!pred_pass(a.ctl)) return;
-    // Workgroup -> sites: the XCD remap gives each XCD a contiguous range of
-    // logical tiles; with tmajor the logical tile index runs over t fastest,
-    // so the +-t neighbour slices of a tile are streamed by the same XCD at
-    // nearly the same time and its L2 serves their re-reads (FP64: 81.2 us vs
-    // 85.5 us per 32^4 Dslash).
     const int blk = xcd_block_id_dir(a.rev);
-    int idx;
-    if (a.tmajor) {
-        const int s3 = a.g.sizeh / a.g.nd3;
-        const int tile = blk / a.g.nd3, tt = blk - tile * a.g.nd3;
-        idx = tt * s3 + tile * kBlock + (int)threadIdx.x;
-    } else {
-        idx = blk * kBlock + (int)threadIdx.x;
-    }
+    const int idx = dslash_idx(a, blk, kBlock, (int)threadIdx.x);
     double dot = 0.0;
     if (idx < a.g.sizeh) {
-        C o0, o1, o2;
-        dslash_site<R, EO>(a.u, a.ph, a.in, a.g, idx, o0, o1, o2);
-        if (MODE == kPlain) {
-            if constexpr (sizeof(R) == 8) {
-                st_nt(a.out + idx, o0);
-                st_nt(a.out + a.g.sizeh + idx, o1);
-                st_nt(a.out + 2 * a.g.sizeh + idx, o2);
-            } else {
-                a.out[idx] = o0;
-                a.out[a.g.sizeh + idx] = o1;
-                a.out[2 * a.g.sizeh + idx] = o2;
-            }
-        } else if constexpr (MODE == kMdagMResid) {
-            // r_f = (float)(b - (x*m2 - D in)), |r_f|^2; the FP64 product itself is not stored
-            const C o[3] = {o0, o1, o2};
+        C o[3];
+        dslash_site<R, EO>(a.u, a.ph, a.in, a.g, idx, o[0], o[1], o[2]);
+        C x[3];
 #pragma unroll
-            for (int c = 0; c < 3; c++) {
-                const long k = (long)c * a.g.sizeh + idx;
-                const C xx = a.x[k];
-                const double2 bb = a.b[k];
-                const double sx = (double)xx.x * a.m2 - (double)o[c].x, sy = (double)xx.y * a.m2 - (double)o[c].y;
-                const float2 f = make_float2((float)(bb.x - sx), (float)(bb.y - sy));
-                a.rf[k] = f;
-                dot += (double)f.x * f.x + (double)f.y * f.y;
-            }
-        } else {
-            // combine_in1xferm_mass_minus_in2: out = x*m2 - D in  (promoted to double)
-            const C x0 = a.x[idx], x1 = a.x[a.g.sizeh + idx], x2 = a.x[2 * a.g.sizeh + idx];
-            const double m2 = a.m2;
-            const C s0 = mk<C>((double)x0.x * m2 - (double)o0.x, (double)x0.y * m2 - (double)o0.y);
-            const C s1v = mk<C>((double)x1.x * m2 - (double)o1.x, (double)x1.y * m2 - (double)o1.y);
-            const C s2v = mk<C>((double)x2.x * m2 - (double)o2.x, (double)x2.y * m2 - (double)o2.y);
-            if constexpr (sizeof(R) == 8) {
-                st_nt(a.out + idx, s0);
-                st_nt(a.out + a.g.sizeh + idx, s1v);
-                st_nt(a.out + 2 * a.g.sizeh + idx, s2v);
-            } else {
-                a.out[idx] = s0;
-                a.out[a.g.sizeh + idx] = s1v;
-                a.out[2 * a.g.sizeh + idx] = s2v;
-            }
-            if (MODE == kMdagMDot) dot = re_dot(x0, s0) + re_dot(x1, s1v) + re_dot(x2, s2v);
-        }
+        for (int c = 0; c < 3; c++) x[c] = MODE == kPlain ? o[c] : a.x[(long)c * a.g.sizeh + idx];
+#pragma unroll
+        for (int c = 0; c < 3; c++) dot += dslash_out<R, MODE>(a, (long)c * a.g.sizeh + idx, o[c], x[c]);
     }
     // partial slot = logical tile, so the reduction order is the same in both walk directions
     if (MODE >= kMdagMDot) block_partial_at<kBlock>(dot, 0.0, a.ctl.partials, blk);
 }
 
+// The same with a half-site's eight hops split over the waves of a block: 64
+// sites a block, wave h takes hop h of k_dslash's order, and the results are
+// added in that order, so the outputs are k_dslash's.
+constexpr int kSplitSites = 64, kSplitWaves = 8;
+template <typename R, int EO, int MODE>
+__global__ __launch_bounds__(64 * kSplitWaves) void k_dslash_split(DslashArgs<R> a) {
+    using C = typename Cplx<R>::T;
+    if (!pred_pass(a.ctl)) return;
+    constexpr int F = EO == 0 ? 0 : 1, B = 1 - F;
+    __shared__ C con[kSplitWaves][3][64];
+    const int lane = (int)threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int blk = xcd_block_id_dir(a.rev);
+    const int site = dslash_idx(a, blk, kSplitSites, lane);
+    const bool live = site < a.g.sizeh;
+    const int idx = live ? site : 0, sh = a.g.sizeh;
+    // colour c is finished by wave c; its x is loaded before the hop
+    C x = mk<C>(0, 0);
+    if (MODE != kPlain && w < 3) x = a.x[(long)w * sh + idx];
+    const Nbrs nb = site_neighbours<EO>(a.g, idx);
+    const int mu = w & 3;
+    C o0 = mk<C>(0, 0), o1 = mk<C>(0, 0), o2 = mk<C>(0, 0);
+    if (w < 4) {
+        const int im = mu == 0 ? nb.im[0] : mu == 1 ? nb.im[1] : mu == 2 ? nb.im[2] : nb.im[3];
+        hop<R, true>(a.u[2 * mu + B], a.ph[2 * mu + B], a.in, sh, im, im, o0, o1, o2);
+    } else {
+        const int ip = mu == 0 ? nb.ip[0] : mu == 1 ? nb.ip[1] : mu == 2 ? nb.ip[2] : nb.ip[3];
+        hop<R, false>(a.u[2 * mu + F], a.ph[2 * mu + F], a.in, sh, idx, ip, o0, o1, o2);
+    }
+    con[w][0][lane] = o0;
+    con[w][1][lane] = o1;
+    con[w][2][lane] = o2;
+    __syncthreads();
+    double dot = 0.0;
+    if (w < 3 && live) {
+        C o = con[0][w][lane];
+#pragma unroll
+        for (int h = 1; h < kSplitWaves; h++) o = cadd(o, con[h][w][lane]);
+        const R half = (R)0.5;
+        o.x *= half;
+        o.y *= half;
+        dot = dslash_out<R, MODE>(a, (long)w * sh + idx, o, x);
+    }
+    if (MODE >= kMdagMDot) block_partial_at<64 * kSplitWaves>(dot, 0.0, a.ctl.partials, blk);
+}
+
 // ---------------------------------------------------------------- launchers
+
+// Where the hops are split over eight waves (k_dslash_split).  Small lattices
+// leave most of the chip idle with a site per thread, and each thread waits for
+// its hops in turn.  The pair D_oe, D_eo queued back to back, whole against
+// split: FP64 11.7 -> 8.2 us at 2048 half-sites, 16.6 -> 9.4 at 16384, 23.8 ->
+// 21.4 at 65536, but 41.1 -> 43.8 at 131072 and 157 -> 181 at 524288, where the
+// exchange through LDS costs more than the shorter chain gives; the line is that of
+// the fused solver iterations, so that a solver's sums have one order on either
+// side of it.  FP32 11.7 -> 7.8
+// at 2048, 25.7 -> 23.8 at 154440 and still 78.7 -> 74.5 at 524288 (half the
+// bytes a site).  Two or four waves a site lie between.
+template <typename R>
+static bool dslash_split() {
+    return sizeof(R) == 4 || ctx().lat.sizeh <= kHopSplitSizeh;
+}
+template <typename R>
+int dslash_blocks() {
+    return blocks_for(ctx().lat.sizeh, dslash_split<R>() ? kSplitSites : kBlock);
+}
+template int dslash_blocks<double>();
+template int dslash_blocks<float>();
+
+template <typename R, int EO, int MODE>
+static void go(const DslashArgs<R>& a) {
+    const dim3 blocks(dslash_blocks<R>());
+    if constexpr (sizeof(R) == 8)
+        if (!dslash_split<R>()) {
+            hipLaunchKernelGGL((k_dslash<R, EO, MODE>), blocks, dim3(kBlock), 0, ctx().stream, a);
+            return;
+        }
+    hipLaunchKernelGGL((k_dslash_split<R, EO, MODE>), blocks, dim3(64 * kSplitWaves), 0, ctx().stream, a);
+}
 
 template <typename R>
 static bool fill_args(DslashArgs<R>& a, const void* u_dev, const void* ph_dev, const void* in_dev, void* out_dev) {
@@ -132,8 +207,8 @@ static bool fill_args(DslashArgs<R>& a, const void* u_dev, const void* ph_dev, c
     a.g.sizeh = (int)L.sizeh;
     // t-fastest tiles need whole tiles per t-slice; used for FP64 only (no gain in FP32)
     const long s3 = L.sizeh / L.nd[3];
-    a.tmajor = (sizeof(R) == 8 && s3 % kBlock == 0) ? 1 : 0;
-    a.rev = 0;
+    a.tmajor = (sizeof(R) == 8 && s3 % (dslash_split<R>() ? kSplitSites : kBlock) == 0) ? 1 : 0;
+    a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
     return true;
 }
 
@@ -146,21 +221,17 @@ bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, con
     a.x = (const typename Cplx<R>::T*)x;
     a.m2 = m2;
     a.ctl = ctl;
-    a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
-    const int nb = blocks_for(ctx().lat.sizeh);
-    hipStream_t s = ctx().stream;
-#define OSTP_L(EO, MODE) hipLaunchKernelGGL((k_dslash<R, EO, MODE>), dim3(nb), dim3(kBlock), 0, s, a)
+    const int nb = dslash_blocks<R>();
     if (mode == kPlain) {
-        if (eo == 0) OSTP_L(0, kPlain); else OSTP_L(1, kPlain);
+        if (eo == 0) go<R, 0, kPlain>(a); else go<R, 1, kPlain>(a);
     } else if (mode == kMdagM) {
-        if (eo == 0) OSTP_L(0, kMdagM); else OSTP_L(1, kMdagM);
+        if (eo == 0) go<R, 0, kMdagM>(a); else go<R, 1, kMdagM>(a);
     } else {
         if (eo != 0) return fail("fused dot epilogue only on Deo");
         if (fin != kFinNone && fin != kFinStore && fin != kFinMsAlpha && fin != kFinFcgAlpha && fin != kFinMxmAlpha)
             return fail("unsupported dslash finalizer %d", fin);
-        OSTP_L(0, kMdagMDot);
+        go<R, 0, kMdagMDot>(a);
     }
-#undef OSTP_L
     if (!hip_ok(hipGetLastError(), "k_dslash launch")) return false;
     return mode == kMdagMDot && fin != kFinNone ? launch_finalize(fin, ctl, nb) : true;
 }
@@ -182,9 +253,7 @@ bool launch_mdagm_resid(const void* u, const void* ph, const void* x, void* temp
     a.b = (const double2*)b;
     a.rf = (float2*)rf;
     a.ctl = ctl;
-    a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
-    hipLaunchKernelGGL((k_dslash<double, 0, kMdagMResid>), dim3(blocks_for(ctx().lat.sizeh)), dim3(kBlock), 0,
-                       ctx().stream, a);
+    go<double, 0, kMdagMResid>(a);
     return hip_ok(hipGetLastError(), "k_dslash launch");
 }
 

@@ -16,6 +16,9 @@ template <> __host__ __device__ __forceinline__ float2 mkc<float2>(double a, dou
 template <typename R>
 bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, const void* in, void* out,
                    const void* x, double m2, const SolverCtl& ctl);
+// blocks of a launch_dslash launch (block b's partial at partials[2 b])
+template <typename R>
+int dslash_blocks();
 // D_oe of n FP64 even fields stored one after the other (xs -> hs), the
 // fields sharing each link load (solvers.hip)
 bool launch_doe_multi(const void* u, const void* ph, const void* xs, void* hs, int n);

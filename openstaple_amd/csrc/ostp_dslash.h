@@ -13,6 +13,9 @@ template <typename R> struct Cplx;
 template <> struct Cplx<double> { using T = double2; };
 template <> struct Cplx<float> { using T = float2; };
 
+// FP64 lattices whose hops are split over eight waves a site (half-sites)
+constexpr long kHopSplitSizeh = 49152;
+
 enum DslashMode : int { kPlain = 0, kMdagM = 1, kMdagMDot = 2, kMdagMResid = 3 };
 
 

@@ -508,7 +508,7 @@ struct KrSys {
 // r and p read at eight neighbours each and the exchange through LDS cost more
 // than a kernel that stores p.  One CG-M system, split against not: ahead up to
 // 24^3 x 6 (41472), even at 24^3 x 8 (55296), behind from 32^3 x 4 (65536) on.
-constexpr long kKrSplitSizeh = 49152;
+constexpr long kKrSplitSizeh = kHopSplitSizeh;
 
 static bool kr_split() { return ctx().lat.sizeh <= kKrSplitSizeh; }
 static int kr_blocks_hop() { return blocks_for(ctx().lat.sizeh, kr_split() ? kKrSites : kBlock); }
@@ -825,11 +825,14 @@ int mixed_solve(const MxBufs& B, double mass, double shift, double res, int max_
     a.sf = (const float2*)B.sf;
     a.x = (double2*)B.x;
     a.st = ctx().state;
-    a.nA = a.nT = nbh;
+    a.nA = dslash_blocks<float>();
+    a.nT = dslash_blocks<double>();
     a.nB = kr_blocks_r();
-    a.partA = ctx().partials;
-    a.partT = ctx().partials + 2 * nbh;
-    a.partB = ctx().partials + 4 * nbh;
+    // within the 4 (sizeh / 64 + 64) doubles there are: nA, nT <= sizeh / 64, and
+    // nB <= 256 where nT is not below sizeh / 256
+    a.partB = ctx().partials;
+    a.partA = a.partB + a.nB;
+    a.partT = a.partA + 2 * a.nA;
     a.sizeh = (int)sizeh;
     int j = 0, batch = 16, prev_j = 0, last_cg = -1;
     double prev_d = kr_dist(H(), false);
@@ -840,6 +843,7 @@ int mixed_solve(const MxBufs& B, double mass, double shift, double res, int max_
             hipLaunchKernelGGL(k_mx_p, dim3(a.nB), dim3(kBlock), 0, S(), a);
             SolverCtl c = ctl_of(kIfGoing);
             c.st = a.st + (j & 1);
+            c.partials = const_cast<double*>(a.partA);
             if (!launch_dslash<float>(1, kPlain, kFinStore, B.u_f, B.ph_f, B.pf, B.hf, nullptr, 0.0, c) ||
                 !launch_dslash<float>(0, kMdagMDot, kFinNone, B.u_f, B.ph_f, B.hf, B.sf, B.pf, m2f, c))
                 return INVERTER_FAILURE;
@@ -847,7 +851,7 @@ int mixed_solve(const MxBufs& B, double mass, double shift, double res, int max_
             a.tail = j % kMxTailEvery == 0;
             if (!a.tail) continue;
             c.pred = kIfRunningRU;
-            c.partials = ctx().partials + 2 * nbh;
+            c.partials = const_cast<double*>(a.partT);
             if (!launch_mdagm_resid(B.u, B.ph, B.x, B.h, B.b, B.rf, m2, c)) return INVERTER_FAILURE;
         }
         a.j = j + 1;

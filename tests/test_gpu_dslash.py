@@ -181,3 +181,29 @@ def test_bad_pointer_is_an_error_not_a_fault():
     msg = lib.ostp_last_error()
     lib.ostp_clear_error()
     assert msg and b"overruns its allocation" in msg
+
+
+# 8 and 480 half-sites (less than a block of 64, a last block that is not
+# full), the last lattice whose FP64 hops are split over waves and one above it
+@pytest.mark.parametrize("shape", [(2, 2, 2, 2), (6, 4, 4, 10), (16, 16, 16, 24), (16, 16, 16, 26)])
+def test_hops_at_block_edges(shape):
+    o = Oracle(*shape)
+    init_lattice(shape)
+    u, psi = fields(o, 17, eps=0.7)
+    ph = o.phases()
+    du, dp, dpsi = Dev(u), Dev(ph), Dev(psi)
+    dout, dtmp = Dev(nbytes=psi.nbytes), Dev(nbytes=psi.nbytes)
+    fp = ost.ferm_param(0.05, dp.p)
+    lib.acc_Deo(du.p, dout.p, dpsi.p, dp.p)
+    check64(dout.get(psi), o.deo(u, psi, ph))
+    lib.fermion_matrix_multiplication_shifted(du.p, dout.p, dpsi.p, dtmp.p, C.byref(fp), 0.013)
+    ost.check(0, "mdagm")
+    check64(dout.get(psi), o.mdagm(u, psi, ph, 0.05, 0.013))
+    check64(dtmp.get(psi), o.doe(u, psi, ph))
+    uf, phf, psif = o.to_float_gauge(u), ph.astype(np.float32), psi.astype(np.complex64)
+    duf, dpf, dpsif, doutf = Dev(uf), Dev(phf), Dev(psif), Dev(nbytes=psif.nbytes)
+    lib.acc_Deo_f(duf.p, doutf.p, dpsif.p, dpf.p)
+    assert rel(doutf.get(psif), o.deo_f(uf, psif, phf)) < TOL32
+    lib.acc_Doe_f(duf.p, doutf.p, dpsif.p, dpf.p)
+    ost.check(0, "acc_Doe_f")
+    assert rel(doutf.get(psif), o.doe_f(uf, psif, phf)) < TOL32
