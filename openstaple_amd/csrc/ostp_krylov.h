@@ -42,6 +42,7 @@ constexpr int kKrSys = 4;
 constexpr int kMsWinMax = 64;
 struct MsWin {
     int t;                                  // iterations in the current window
+    int first;                              // a solve's first: x_k and p_k not stored yet
     int active[kMaxShifts];                 // shift moved in this window
     double a[kMaxShifts], B[kMaxShifts];
     double c[kMaxShifts][kMsWinMax], D[kMaxShifts][kMsWinMax];

@@ -207,56 +207,76 @@ __global__ __launch_bounds__(kBlock) void k_msw_p(C* __restrict__ p, const C* __
 }
 
 // x_k += a_k p_k + sum_j c_kj r_j ; p_k = B_k p_k + sum_j D_kj r_j for the
-// shifts that moved, kMswGroup shifts per pass over the residuals (eight: three
-// passes for 19 shifts instead of five with four, each shift's sums unchanged).
-// CX: the solutions' type (FP64 also when the directions and residuals C are
-// FP32: the mixed CG-M adds each window straight into its FP64 solutions).
-constexpr int kMswGroup = 8;
-template <typename CX, typename C>
-__global__ __launch_bounds__(kBlock) void k_msw_flush(CX* __restrict__ xs, C* __restrict__ ps,
-                                                      const C* __restrict__ hist, long n3, int order,
-                                                      const MsWin* __restrict__ w, SolverCtl ctl, int full = 0) {
+// shifts that moved, G shifts per pass over the residuals; a solve's first
+// window takes x_k = 0 and p_k = b without reading them (nor has anyone stored
+// them).  CX: the solutions' type (FP64 also when the directions and residuals
+// C are FP32: the mixed CG-M adds each window straight into its FP64 solutions).
+// Bound by memory: a window of 64 residuals and 19 shifts read 64 x 3 + 38
+// vectors with eight shifts a pass, 64 + 38 with all of them (160 accumulator
+// registers, two waves a SIMD, the next four residuals in flight).  With the
+// copies into x_k and p_k gone: 204 iterations with 19 shifts on 32^4 43.75 ->
+// 42.47 ms, a force of two systems on 32^3 x 8 8.04 -> 7.65, order 9 on
+// 12x14x10x6 1.196 -> 1.135.  The barrier keeps a shift's coefficients in scalar
+// registers just before their use (left to itself the compiler moves them all
+// ahead, into 450 bytes of scratch a lane).
+template <typename CX, typename C, int G>
+__global__ __launch_bounds__(kBlock, 2) void k_msw_flush(CX* __restrict__ xs, C* __restrict__ ps,
+                                                         const C* __restrict__ hist, const C* __restrict__ b,
+                                                         long n3, int order, const MsWin* __restrict__ w,
+                                                         SolverCtl ctl, int full) {
     if (!pred_pass(ctl)) return;
     const int t = w->t;
     if (t == 0 || t < full) return;  // full: only a window of that many iterations
+    const bool first = w->first;
     const long i = (long)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n3) return;
-    for (int k0 = 0; k0 < order; k0 += kMswGroup) {
-        double2 ax[kMswGroup], ap[kMswGroup];
-        bool on[kMswGroup];
-        bool any = false;
+    for (int k0 = 0; k0 < order; k0 += G) {
+        double2 ax[G], ap[G];
+        unsigned on = 0;
 #pragma unroll
-        for (int q = 0; q < kMswGroup; q++) {
+        for (int q = 0; q < G; q++) {
             const int k = k0 + q;
-            on[q] = k < order && w->active[k];
-            any = any || on[q];
             ax[q] = make_double2(0.0, 0.0);
             ap[q] = make_double2(0.0, 0.0);
-            if (on[q]) {
-                const CX xv = xs[k * n3 + i];
-                const C pv = ps[k * n3 + i];
-                const double a = w->a[k], b = w->B[k];
-                ax[q] = make_double2((double)xv.x + a * (double)pv.x, (double)xv.y + a * (double)pv.y);
-                ap[q] = make_double2(b * (double)pv.x, b * (double)pv.y);
+            if (k >= order || !(first || w->active[k])) continue;
+            on |= 1u << q;
+            const C pv = first ? b[i] : ps[k * n3 + i];
+            const CX xv = first ? mkc<CX>(0.0, 0.0) : xs[k * n3 + i];
+            const double wa = w->a[k], wb = w->B[k];
+            ax[q] = make_double2((double)xv.x + wa * (double)pv.x, (double)xv.y + wa * (double)pv.y);
+            ap[q] = make_double2(wb * (double)pv.x, wb * (double)pv.y);
+        }
+        if (!on) continue;
+        constexpr int U = 4;
+        C nx[U];
+#pragma unroll
+        for (int e = 0; e < U; e++) nx[e] = hist[(long)(e < t ? e : 0) * n3 + i];
+        for (int j = 0; j < t; j += U) {
+            double2 r[U];
+#pragma unroll
+            for (int e = 0; e < U; e++) {
+                r[e] = make_double2((double)nx[e].x, (double)nx[e].y);
+                const int jn = j + U + e;
+                nx[e] = hist[(long)(jn < t ? jn : 0) * n3 + i];
+            }
+            // the last group's coefficients beyond t are zero
+#pragma unroll
+            for (int q = 0; q < G; q++) {
+                if (!(on >> q & 1)) continue;
+#pragma unroll
+                for (int e = 0; e < U; e++) {
+                    const double c = w->c[k0 + q][j + e], d = w->D[k0 + q][j + e];
+                    ax[q].x += c * r[e].x;
+                    ax[q].y += c * r[e].y;
+                    ap[q].x += d * r[e].x;
+                    ap[q].y += d * r[e].y;
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if (!any) continue;
-        for (int j = 0; j < t; j++) {
-            const C rv = hist[(long)j * n3 + i];
-            const double rx = (double)rv.x, ry = (double)rv.y;
 #pragma unroll
-            for (int q = 0; q < kMswGroup; q++) {
-                if (!on[q]) continue;
-                const double c = w->c[k0 + q][j], d = w->D[k0 + q][j];
-                ax[q].x += c * rx;
-                ax[q].y += c * ry;
-                ap[q].x += d * rx;
-                ap[q].y += d * ry;
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < kMswGroup; q++)
-            if (on[q]) {
+        for (int q = 0; q < G; q++)
+            if (on >> q & 1) {
                 xs[(k0 + q) * n3 + i] = mkc<CX>(ax[q].x, ax[q].y);
                 ps[(k0 + q) * n3 + i] = mkc<C>(ap[q].x, ap[q].y);
             }
@@ -265,7 +285,7 @@ __global__ __launch_bounds__(kBlock) void k_msw_flush(CX* __restrict__ xs, C* __
 
 // a fresh window: coefficients of the identity map (full: only when that many
 // iterations fill it; w->t is not read otherwise, new memory holds anything)
-__global__ __launch_bounds__(kBlock) void k_msw_reset(MsWin* w, SolverCtl ctl, int full = 0) {
+__global__ __launch_bounds__(kBlock) void k_msw_reset(MsWin* w, SolverCtl ctl, int full, int first) {
     if (!pred_pass(ctl)) return;
     if (full && w->t < full) return;
     __syncthreads();  // every thread has read t before it is cleared
@@ -279,7 +299,10 @@ __global__ __launch_bounds__(kBlock) void k_msw_reset(MsWin* w, SolverCtl ctl, i
         w->B[k] = 1.0;
         w->active[k] = 0;
     }
-    if (threadIdx.x == 0) w->t = 0;
+    if (threadIdx.x == 0) {
+        w->t = 0;
+        w->first = first;
+    }
 }
 
 // FP32 CG-M with FP64 reliable updates: r += omega s and, for the base
@@ -426,6 +449,21 @@ static SolverCtl ctl_of(int pred, int iter = 0) {
 }
 
 static bool check_launch(const char* what) { return hip_ok(hipGetLastError(), what); }
+
+// apply a window (see k_msw_flush); b: the source, for a solve's first window
+template <typename CX, typename C>
+static void msw_flush(void* xs, void* ps, const void* hist, const void* b, long n3, int order, const MsWin* w,
+                      const SolverCtl& ctl, int full = 0) {
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(blocks_for(n3)), dim3(kBlock), 0, S(), (CX*)xs, (C*)ps, (const C*)hist,
+                           (const C*)b, n3, order, w, ctl, full);
+    };
+    if (order <= 10) go(k_msw_flush<CX, C, 10>);
+    else go(k_msw_flush<CX, C, 20>);
+}
+static void msw_reset(MsWin* w, const SolverCtl& ctl, int full, bool first) {
+    hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), w, ctl, full, first ? 1 : 0);
+}
 
 static int batch_next(int b) { return std::min(2 * b, 64); }
 
@@ -632,10 +670,9 @@ static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bo
             if (W && j > 1 && (j - 1) % W == 0)
                 for (int k = 0; k < n; k++) {
                     // the windows that iteration j - 1 filled
-                    hipLaunchKernelGGL((k_msw_flush<double2, double2>), dim3(nb3), dim3(kBlock), 0, S(),
-                                       (double2*)sy[k].out, (double2*)sy[k].shiftferm, (const double2*)sy[k].hist, n3,
-                                       sy[k].order, (const MsWin*)sy[k].win, ctl_of(kAlways), W);
-                    hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), sy[k].win, ctl_of(kAlways), W);
+                    msw_flush<double2, double2>(sy[k].out, sy[k].shiftferm, sy[k].hist, sy[k].b, n3, sy[k].order,
+                                                sy[k].win, ctl_of(kAlways), W);
+                    msw_reset(sy[k].win, ctl_of(kAlways), W, false);
                 }
             if (split) {
                 a.rev = ctx().dslash_serpentine ? (int)(ctx().dslash_launches++ & 1u) : 0;
@@ -1090,8 +1127,9 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
     const double m2 = mass * mass;
     if (order < 0 || order > kMaxShifts) return fail("multishift: order %d out of range", order) ? 0 : INVERTER_FAILURE;
 
-    // x_k = 0 ; r = p = b ; p_k = b
-    for (int k = 0; k < order; k++) {
+    // r = p = b ; x_k = 0 ; p_k = b (with windows the first one starts from those, see k_msw_flush)
+    const int W = msw_window(vb);
+    for (int k = 0; W < 2 && k < order; k++) {
         if (!hip_ok(hipMemsetAsync((char*)B.out + k * vb, 0, vb, S()), "zero x_k")) return INVERTER_FAILURE;
         if (!hip_ok(hipMemcpyAsync((char*)B.shiftferm + k * vb, B.b, vb, hipMemcpyDeviceToDevice, S()), "p_k = b"))
             return INVERTER_FAILURE;
@@ -1126,7 +1164,6 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
 
     // residual window (falls back to per-iteration shift updates when fewer
     // than 8 residuals fit)
-    const int W = msw_window(vb);
     char* hist = nullptr;
     if (W >= 2) {
         hist = (char*)g_msw_hist;
@@ -1139,11 +1176,12 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
         }
         hist = (char*)g_msw_hist;
         if (!g_msw && !hip_ok(hipMalloc(&g_msw, sizeof(MsWin)), "multishift window")) return INVERTER_FAILURE;
-        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kAlways), 0);
+        msw_reset(g_msw, ctl_of(kAlways), 0, true);
     }
     auto slot = [&](int j) { return (C*)(hist + (size_t)((j - 1) % W) * vb); };  // residual of iteration j (1-based)
     if constexpr (sizeof(R) == 8) {
         KrSys sys{};
+        sys.b = B.b;
         sys.r = B.r;
         sys.h = B.h;
         sys.s = B.s;
@@ -1176,9 +1214,8 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
                                ctl_of(kIfIter, j), (C*)nullptr);
             if (j % W == 0) {
                 // only when iteration j ran: a window cut short is flushed once, at the end
-                hipLaunchKernelGGL((k_msw_flush<C, C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.out, (C*)B.shiftferm,
-                                   (const C*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kIfIter, j), 0);
-                hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kIfIter, j), 0);
+                msw_flush<C, C>(B.out, B.shiftferm, hist, B.b, n3, order, g_msw, ctl_of(kIfIter, j));
+                msw_reset(g_msw, ctl_of(kIfIter, j), 0, false);
             }
             return check_launch("multishift iteration");
         };
@@ -1188,8 +1225,7 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
     if (hist) {
         // the partial last window, and the final residual where the per-iteration
         // version leaves it
-        hipLaunchKernelGGL((k_msw_flush<C, C>), dim3(nb3), dim3(kBlock), 0, S(), (C*)B.out, (C*)B.shiftferm,
-                           (const C*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kAlways), 0);
+        msw_flush<C, C>(B.out, B.shiftferm, hist, B.b, n3, order, g_msw, ctl_of(kAlways));
         if (cg > 0 && !hip_ok(hipMemcpyAsync(B.r, slot(cg), vb, hipMemcpyDeviceToDevice, S()), "final residual"))
             return INVERTER_FAILURE;
         if (!check_launch("multishift window flush")) return INVERTER_FAILURE;
@@ -1477,16 +1513,10 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
     auto hist = [&](int k) { return (char*)g_mm_hist + (size_t)k * hb; };
     auto slot = [&](int k, int j) { return (double2*)(hist(k) + (size_t)((j - 1) % W) * vb); };
 
-    // x_k = 0 ; r = p = b ; p_k = b ; states as multishift_solve sets them
+    // r = p = b (x_k = 0 and p_k = b: see k_msw_flush); states as multishift_solve sets them
     double sn[kMsMulti];
     for (int k = 0; k < n; k++) {
         const MsSys& d = sy[k];
-        for (int i = 0; i < d.order; i++) {
-            if (!hip_ok(hipMemsetAsync((char*)d.out + i * vb, 0, vb, S()), "zero x_k") ||
-                !hip_ok(hipMemcpyAsync((char*)d.shiftferm + i * vb, d.b, vb, hipMemcpyDeviceToDevice, S()),
-                        "p_k = b"))
-                return false;
-        }
         if (!hip_ok(hipMemcpyAsync(d.r, d.b, vb, hipMemcpyDeviceToDevice, S()), "r = b") ||
             !hip_ok(hipMemcpyAsync(d.p, d.b, vb, hipMemcpyDeviceToDevice, S()), "p = b") ||
             !reduce_to_host(0, d.b, nullptr, 0, &sn[k], nullptr))
@@ -1518,11 +1548,12 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
                 "multi states"))
         return false;
     for (int k = 0; k < n; k++)
-        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_mm_win + k, ctl_of(kAlways), 0);
+        msw_reset(g_mm_win + k, ctl_of(kAlways), 0, true);
 
     KrSys ks[kMsMulti];
     for (int k = 0; k < n; k++) {
         ks[k] = KrSys{};
+        ks[k].b = sy[k].b;
         ks[k].r = sy[k].r;
         ks[k].h = sy[k].h;
         ks[k].s = sy[k].s;
@@ -1540,9 +1571,7 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
         MsSys& d = sy[k];
         const int cg = g_mm_st_host[2 * k].cg;
         d.cg = cg;
-        hipLaunchKernelGGL((k_msw_flush<double2, double2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)d.out,
-                           (double2*)d.shiftferm, (const double2*)hist(k), n3, d.order,
-                           (const MsWin*)(g_mm_win + k), ctl_of(kAlways), 0);
+        msw_flush<double2, double2>(d.out, d.shiftferm, hist(k), d.b, n3, d.order, g_mm_win + k, ctl_of(kAlways));
         if (cg > 0 && !hip_ok(hipMemcpyAsync(d.r, slot(k, cg), vb, hipMemcpyDeviceToDevice, S()), "final residual"))
             return false;
         if (!check_launch("multi multishift window flush")) return false;
@@ -2330,7 +2359,7 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
         }
         hist = (float2*)g_msw_hist;
         if (!g_msw && !hip_ok(hipMalloc(&g_msw, sizeof(MsWin)), "multishift window")) return 0;
-        hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kAlways), 0);
+        msw_reset(g_msw, ctl_of(kAlways), 0, false);
     }
     // Reliable updates are taken at every kMsxRuEvery-th iteration (when the
     // FP32 residual has fallen by mixed_delta since the last one): the other
@@ -2361,9 +2390,8 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
                            g_msw, ctl_of(kIfIter, j), hist + (size_t)((j - 1) % W) * n3);
         if (j % W == 0) {
             // only when iteration j ran: a window cut short is flushed once, at the end
-            hipLaunchKernelGGL((k_msw_flush<double2, float2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)dout,
-                               (float2*)pk, (const float2*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kIfIter, j), 0);
-            hipLaunchKernelGGL(k_msw_reset, dim3(1), dim3(kBlock), 0, S(), g_msw, ctl_of(kIfIter, j), 0);
+            msw_flush<double2, float2>(dout, pk, hist, nullptr, n3, order, g_msw, ctl_of(kIfIter, j));
+            msw_reset(g_msw, ctl_of(kIfIter, j), 0, false);
         }
         return check_launch("mixed multishift iteration");
     };
@@ -2371,8 +2399,7 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
     const int cg = H().cg;
     if (cg_multishift) *cg_multishift = cg;
     if (hist)
-        hipLaunchKernelGGL((k_msw_flush<double2, float2>), dim3(nb3), dim3(kBlock), 0, S(), (double2*)dout,
-                           (float2*)pk, (const float2*)hist, n3, order, (const MsWin*)g_msw, ctl_of(kAlways), 0);
+        msw_flush<double2, float2>(dout, pk, hist, nullptr, n3, order, g_msw, ctl_of(kAlways));
     hipLaunchKernelGGL(k_msx_flush, dim3(nb3), dim3(kBlock), 0, S(), fl, n3, ctl_of(kAlways));
     if (!check_launch("flush")) return 0;
     if (verbosity_lv > 1 && !hip_ok(hipStreamSynchronize(S()), "timing")) return 0;

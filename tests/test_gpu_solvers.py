@@ -634,3 +634,36 @@ def test_mixed_iterations_at_block_edges(shape, delta):
     r = s.b - s.o.mdagm(s.u, x.get(s.b), s.ph, mass)
     # the FP64 residual of what the five FP32 steps added
     assert abs(np.linalg.norm(r) / np.linalg.norm(s.b) - tr.value) <= 1e-6 * tr.value
+
+
+# ten and twenty shifts are the most that one pass of a window's update takes
+@pytest.mark.parametrize("order", [1, 10, 11, 20, 21, 24])
+@pytest.mark.parametrize("window", [9, 64])
+def test_multishift_window_orders(order, window):
+    """Solutions and directions from windowed updates against those of the
+    per-iteration updates (the same recurrence, summed in another order)."""
+    s = Sys((4, 6, 4, 6), seed=3, kind="cold", param=0.5, mass=0.1)
+    ra = remez19(s.mass)
+    ra.approx_order = order
+    for k in range(order):
+        ra.RA_b[k] = 0.003 * 1.4 ** k
+    vb = s.b.nbytes
+    got = []
+    for w in (1, window):
+        prev = lib.ostp_set_multishift_window(w)
+        try:
+            # what the outputs held before is not read
+            out, sf = Dev(np.full(order * 3 * s.o.sizeh, np.nan + 0j)), Dev(np.full(order * 3 * s.o.sizeh, np.nan + 0j))
+            cg = C.c_int(0)
+            st = lib.multishift_invert(s.du.p, C.byref(s.fp), C.byref(ra), out.p, s.db.p, 1e-9,
+                                       *(d.p for d in s.scratch), sf.p, 10000, C.byref(cg))
+            ost.check(0, "multishift_invert")
+        finally:
+            lib.ostp_set_multishift_window(prev)
+        shape = np.zeros((order, 3, s.o.sizeh), dtype=np.complex128)
+        got.append((st, cg.value, out.get(shape), sf.get(shape)))
+    assert got[0][0] == got[1][0] == 1 and got[0][1] == got[1][1]
+    for k in range(order):
+        assert rel(got[1][2][k], got[0][2][k]) < 1e-12, k
+        # the directions' terms cancel, by 1e3 to 1e4 at most over these iterations, times 64 roundings
+        assert rel(got[1][3][k], got[0][3][k]) < 1e-10, k
