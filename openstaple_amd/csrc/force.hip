@@ -252,17 +252,21 @@ static Scratch g_hs, g_th, g_ta, g_conf_f, g_xs_all;
 // the rational solves of several sources on one operator, together (solvers.hip)
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
                           const void* const* in, void* const* out, int n, double res, int max_cg,
-                          int convergence_importance);
+                          int convergence_importance, void* const* hs);
 
-// sum over shifts of the outer products for one pseudofermion
-bool compute_fermion_force(const void* u, void* aux, const void* xs, const void* phases, const RationalApprox* ra) {
+// sum over shifts of the outer products for one pseudofermion; hs: D_oe x_k
+// where the solver has left them, null to form them here
+bool compute_fermion_force(const void* u, void* aux, const void* xs, const void* phases, const RationalApprox* ra,
+                           const void* hs = nullptr) {
     const Lattice& L = ctx().lat;
     const int order = ra->approx_order;
     if (order <= 0) return true;
-    void* hs = g_hs.get((size_t)order * L.vec3_bytes());
-    if (!hs) return false;
-    // all D_oe x_k, the shifts' solutions in chunks through shared-link hops
-    if (!launch_doe_multi(u, phases, xs, hs, order)) return false;
+    if (!hs) {
+        void* h = g_hs.get((size_t)order * L.vec3_bytes());
+        // all D_oe x_k, the shifts' solutions in chunks through shared-link hops
+        if (!h || !launch_doe_multi(u, phases, xs, h, order)) return false;
+        hs = h;
+    }
     return launch_direct_product(aux, xs, hs, ra->RA_a, order);
 }
 
@@ -382,7 +386,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         std::vector<ferm_param*> fps;
         std::vector<const RationalApprox*> ras;
         std::vector<const void*> ins;
-        std::vector<void*> outs;
+        std::vector<void*> outs, hs;
         int maxo = 1;
         for (int iflav = 0; iflav < tNDiffFlavs; iflav++) {
             ferm_param* fp = &tfermion_parameters[iflav];
@@ -396,7 +400,18 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
             }
         }
         const int n = (int)fps.size();
-        char* xs_all = n >= 2 ? (char*)g_xs_all.get((size_t)n * maxo * L.vec3_bytes()) : nullptr;
+        // the solutions of all sources, and D_oe of them from the solver's check, which
+        // saves the force its hops (without ample room for those it forms them itself)
+        const size_t all = (size_t)n * maxo * L.vec3_bytes();
+        char* xs_all = n >= 2 ? (char*)g_xs_all.get(all) : nullptr;
+        char* hs_all = nullptr;
+        size_t free_b = 0, total_b = 0;
+        if (xs_all && (all <= g_hs.n || (hipMemGetInfo(&free_b, &total_b) == hipSuccess && all <= free_b / 4)))
+            hs_all = (char*)g_hs.get(all);
+        if (xs_all && !hs_all) {
+            (void)hipGetLastError();
+            forgive_errors(e0);
+        }
         if (n >= 2 && !xs_all) {
             (void)hipGetLastError();
             forgive_errors(e0);
@@ -405,9 +420,10 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
             for (int k = 0; k < n; k++) {
                 if (!ins[k]) return;
                 outs.push_back(xs_all + (size_t)k * maxo * L.vec3_bytes());
+                if (hs_all) hs.push_back(hs_all + (size_t)k * maxo * L.vec3_bytes());
             }
             together = multishift_fp64_many(conf_to_use, fps.data(), ras.data(), ins.data(), outs.data(), n, res,
-                                            max_cg, CONVERGENCE_NONCRITICAL);
+                                            max_cg, CONVERGENCE_NONCRITICAL, hs_all ? hs.data() : nullptr);
             if (!together && error_count() != e0) return;
         }
         if (together) {
@@ -418,7 +434,9 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
                 const void* dph = resolve(fp->phases, 8 * L.dsoa_bytes(), nm);
                 if (!dph) return;
                 for (int ips = 0; ips < fp->number_of_ps; ips++, k++)
-                    if (!compute_fermion_force(conf_to_use, dtaux, outs[k], dph, &fp->approx_md)) return;
+                    if (!compute_fermion_force(conf_to_use, dtaux, outs[k], dph, &fp->approx_md,
+                                               hs_all ? hs[k] : nullptr))
+                        return;
                 if (!launch_backfield_times_force(dtaux, dgl3, dph)) return;
             }
             // the shifted solutions of the last source stay in tferm_shiftmulti_acc, as after the loop below

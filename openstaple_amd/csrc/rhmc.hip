@@ -57,7 +57,7 @@ namespace ostp {
 // and the recombination of a rational function's shifted solutions
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
                           const void* const* in, void* const* out, int n, double res, int max_cg,
-                          int convergence_importance);
+                          int convergence_importance, void* const* hs);
 bool recombine(const void* xs, const void* in, void* out, const RationalApprox* ra);
 bool find_max_eigenvalues_many(const void* u, ferm_param* const* pars, void* const* r, void* const* h,
                                void* const* p, int n, double* maxv);
@@ -334,7 +334,7 @@ int UPDATE_SOLOACC_UNOSTEP_VERSATILE(su3_soa* tconf_acc, double res_metro, doubl
                     outs.push_back(xs_all + (size_t)k * per);
                 }
                 if (multishift_fp64_many(du_fm, fps.data(), ras.data(), ins.data(), outs.data(), n, res, max_cg,
-                                         CONVERGENCE_CRITICAL)) {
+                                         CONVERGENCE_CRITICAL, nullptr)) {
                     for (int k = 0; k < n; k++) {
                         void* dy = resolve(at(ys, idx[k], vb), vb, nm);
                         if (!dy || !recombine(outs[k], ins[k], dy, ras[k])) return false;

@@ -940,13 +940,18 @@ struct VerArgs {
     const double2* b;
     double* part;      // kVerShifts x gridDim.x block sums of |r_k|^2
     SiteGeom g;
+    int tmajor;
 };
 
 // EO = 1: h_k = D_oe x_k ; EO = 0: r_k = b - (m2_k x_k - D_eo h_k), block sums of |r_k|^2
 template <int EO>
 __global__ __launch_bounds__(kBlock) void k_ms_verify(VerArgs a) {
     const int blk = xcd_block_id();
-    const int idx = blk * kBlock + (int)threadIdx.x;
+    int idx = blk * kBlock + (int)threadIdx.x;
+    if (a.tmajor) {  // as k_dslash: the solutions' +-t re-reads hit the XCD's L2
+        const int tile = blk / a.g.nd3, tt = blk - tile * a.g.nd3;
+        idx = tt * (a.g.sizeh / a.g.nd3) + tile * kBlock + (int)threadIdx.x;
+    }
     const long n3 = 3L * a.g.sizeh;
     bool act[kVerShifts];
 #pragma unroll
@@ -1023,6 +1028,7 @@ static VerArgs ver_args(const void* u, const void* ph) {
     a.g.nd2 = L.nd[2];
     a.g.nd3 = L.nd[3];
     a.g.sizeh = (int)L.sizeh;
+    a.tmajor = (L.sizeh / L.nd[3]) % kBlock == 0;
     a.b = nullptr;
     a.part = nullptr;
     return a;
@@ -1046,14 +1052,15 @@ bool launch_doe_multi(const void* u, const void* ph, const void* xs, void* hs, i
     return check_launch("k_ms_verify<1>");
 }
 
-// |b - (M + shifts_k) x_k|^2 / sn for the FP64 solutions x_k = out + k * vb
+// |b - (M + shifts_k) x_k|^2 / sn for the FP64 solutions x_k = out + k * vb;
+// hs: D_oe x_k is left in hs + k * vb (null: not kept)
 static bool verify_shifts_f64(const void* u, const void* ph, const void* b, const void* out, int order, double m2,
-                              const double* shifts, double sn, double* g) {
+                              const double* shifts, double sn, double* g, void* hs) {
     const Lattice& L = ctx().lat;
     const long sizeh = L.sizeh;
     const size_t vb = L.vec3_bytes();
     const int nb = blocks_for(sizeh);
-    const size_t need = kVerShifts * vb + ((size_t)kVerShifts * nb + kVerShifts) * sizeof(double) + 256;
+    const size_t need = kVerShifts * vb + ((size_t)kVerShifts * nb + kMaxShifts) * sizeof(double) + 256;
     if (g_ver_bytes < need) {
         if (g_ver_buf) (void)hipFree(g_ver_buf);
         g_ver_buf = nullptr;
@@ -1073,16 +1080,16 @@ static bool verify_shifts_f64(const void* u, const void* ph, const void* b, cons
             a.x[r] = (const double2*)((const char*)out + k * vb);
             a.m2[r] = m2 + shifts[k];
         }
+        if (hs) a.h = (double2*)((char*)hs + k0 * vb);
         hipLaunchKernelGGL(k_ms_verify<1>, dim3(nb), dim3(kBlock), 0, S(), a);
         hipLaunchKernelGGL(k_ms_verify<0>, dim3(nb), dim3(kBlock), 0, S(), a);
-        hipLaunchKernelGGL(k_ms_verify_sum, dim3(a.n), dim3(kBlock), 0, S(), (const double*)a.part, nb, sums);
-        double h_sums[kVerShifts];
-        if (!check_launch("multishift verification") ||
-            !hip_ok(hipMemcpyAsync(h_sums, sums, sizeof(double) * a.n, hipMemcpyDeviceToHost, S()), "verification") ||
-            !hip_ok(hipStreamSynchronize(S()), "verification"))
-            return false;
-        for (int r = 0; r < a.n; r++) g[k0 + r] = h_sums[r] / sn;
+        hipLaunchKernelGGL(k_ms_verify_sum, dim3(a.n), dim3(kBlock), 0, S(), (const double*)a.part, nb, sums + k0);
     }
+    if (!check_launch("multishift verification") ||
+        !hip_ok(hipMemcpyAsync(g, sums, sizeof(double) * order, hipMemcpyDeviceToHost, S()), "verification") ||
+        !hip_ok(hipStreamSynchronize(S()), "verification"))
+        return false;
+    for (int k = 0; k < order; k++) g[k] /= sn;
     return true;
 }
 
@@ -1091,6 +1098,7 @@ static bool verify_shifts_f64(const void* u, const void* ph, const void* b, cons
 struct MsBufs {
     const void *u, *ph, *b;
     void *out, *r, *h, *s, *p, *shiftferm;
+    void* hs = nullptr;          // where D_oe x_k is left (FP64; null: nowhere)
 };
 
 static void* g_msw_hist = nullptr;
@@ -1237,7 +1245,8 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
     int check = 1;
     if constexpr (sizeof(R) == 8) {
         double g[kMaxShifts];
-        if (order > 0 && !verify_shifts_f64(B.u, B.ph, B.b, B.out, order, m2, shifts, sn, g)) return INVERTER_FAILURE;
+        if (order > 0 && !verify_shifts_f64(B.u, B.ph, B.b, B.out, order, m2, shifts, sn, g, B.hs))
+            return INVERTER_FAILURE;
         for (int k = 0; k < order; k++) {
             if (shift_res) shift_res[k] = std::sqrt(g[k]);
             check *= (g[k] <= 1) ? 1 : 0;
@@ -1457,6 +1466,7 @@ struct MsSys {
     int max_cg;
     int cg = 0;          // out: CG-M iterations
     int status = INVERTER_FAILURE;
+    void* hs = nullptr;  // as MsBufs
 };
 
 static SolverState* g_mm_st = nullptr;       // device states of the systems
@@ -1580,7 +1590,7 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
         int check = 1;
         if (d.order > 0) {
             double g[kMaxShifts];
-            if (!verify_shifts_f64(u, ph, d.b, d.out, d.order, d.mass * d.mass, d.shifts, sn[k], g)) return false;
+            if (!verify_shifts_f64(u, ph, d.b, d.out, d.order, d.mass * d.mass, d.shifts, sn[k], g, d.hs)) return false;
             for (int i = 0; i < d.order; i++) check *= (g[i] <= 1) ? 1 : 0;
         }
         if (!hip_ok(hipMemcpyAsync(d.p, (const char*)d.out + (d.order > 0 ? (d.order - 1) : 0) * vb, vb,
@@ -1815,10 +1825,12 @@ static int g_ms_many = 1;  // rational solves of several sources together where 
 // together (multishift_solve_multi, in groups of kMsMulti) when every source
 // has the same U(1) phases.  false, with nothing solved, when that does not
 // apply (another precision mode, the single-precision accelerated path,
-// fewer than two sources, different phases, or no memory for it).
+// fewer than two sources, different phases, or no memory for it).  hs (or
+// null): D_oe of the solutions, as the per-shift check forms it, is left there
+// in the solutions' layout.
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
                           const void* const* in, void* const* out, int n, double res, int max_cg,
-                          int convergence_importance) {
+                          int convergence_importance, void* const* hs) {
     if (!g_ms_many || n < 2 || g_ms_precision != 0 || inverter_tricks.singlePInvAccelMultiInv) return false;
     const unsigned long e0 = error_count();
     const Lattice& L = ctx().lat;
@@ -1850,6 +1862,7 @@ bool multishift_fp64_many(const void* u, ferm_param* const* pars, const Rational
             MsSys& d = sy[r];
             d.b = in[k0 + r];
             d.out = out[k0 + r];
+            d.hs = hs ? hs[k0 + r] : nullptr;
             d.r = base;
             d.h = base + vb;
             d.s = base + 2 * vb;
@@ -1870,6 +1883,7 @@ bool multishift_fp64_many(const void* u, ferm_param* const* pars, const Rational
                 B.ph = ph0;
                 B.b = sy[r].b;
                 B.out = sy[r].out;
+                B.hs = sy[r].hs;
                 B.shiftferm = sy[r].shiftferm;
                 B.r = sy[r].r;
                 B.h = sy[r].h;
