@@ -40,12 +40,14 @@ constexpr int kKrSys = 4;
 // Window of CG-M iterations whose shift updates are applied at once (see
 // k_msw_flush)
 constexpr int kMsWinMax = 64;
+constexpr int kMsWinRows = 40;  // whole passes of k_msw_flush: two of 20 shifts
+static_assert(kMaxShifts <= kMsWinRows, "rows of the window coefficients");
 struct MsWin {
     int t;                                  // iterations in the current window
     int first;                              // a solve's first: x_k and p_k not stored yet
     int active[kMaxShifts];                 // shift moved in this window
     double a[kMaxShifts], B[kMaxShifts];
-    double c[kMaxShifts][kMsWinMax], D[kMaxShifts][kMsWinMax];
+    double c[kMsWinRows][kMsWinMax], D[kMsWinRows][kMsWinMax];
 };
 
 struct KrArgs {

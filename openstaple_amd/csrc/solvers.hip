@@ -216,9 +216,10 @@ __global__ __launch_bounds__(kBlock) void k_msw_p(C* __restrict__ p, const C* __
 // registers, two waves a SIMD, the next four residuals in flight).  With the
 // copies into x_k and p_k gone: 204 iterations with 19 shifts on 32^4 43.75 ->
 // 42.47 ms, a force of two systems on 32^3 x 8 8.04 -> 7.65, order 9 on
-// 12x14x10x6 1.196 -> 1.135.  The barrier keeps a shift's coefficients in scalar
-// registers just before their use (left to itself the compiler moves them all
-// ahead, into 450 bytes of scratch a lane).
+// 12x14x10x6 1.196 -> 1.135.  The barrier keeps four shifts' coefficients in
+// scalar registers just before their use (left to itself the compiler moves all
+// ahead, into 450 bytes of scratch a lane; one shift at a time waits for each: a
+// window of 49 and 19 shifts on 32^3 x 8 201 -> 170 us).
 template <typename CX, typename C, int G>
 __global__ __launch_bounds__(kBlock, 2) void k_msw_flush(CX* __restrict__ xs, C* __restrict__ ps,
                                                          const C* __restrict__ hist, const C* __restrict__ b,
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_msw_flush(CX* __restrict__ xs, C*
             ap[q] = make_double2(wb * (double)pv.x, wb * (double)pv.y);
         }
         if (!on) continue;
-        constexpr int U = 4;
+        constexpr int U = 4, Q = 4;
         C nx[U];
 #pragma unroll
         for (int e = 0; e < U; e++) nx[e] = hist[(long)(e < t ? e : 0) * n3 + i];
@@ -259,18 +260,22 @@ __global__ __launch_bounds__(kBlock, 2) void k_msw_flush(CX* __restrict__ xs, C*
                 const int jn = j + U + e;
                 nx[e] = hist[(long)(jn < t ? jn : 0) * n3 + i];
             }
-            // the last group's coefficients beyond t are zero
+            // the last group's coefficients beyond t are zero, as all of a shift that did
+            // not move (its sums are not stored); four shifts at a time, so that their
+            // coefficients are asked for together
 #pragma unroll
-            for (int q = 0; q < G; q++) {
-                if (!(on >> q & 1)) continue;
+            for (int q0 = 0; q0 < G; q0 += Q) {
+                if (!(on >> q0 & ((1u << Q) - 1))) continue;
 #pragma unroll
-                for (int e = 0; e < U; e++) {
-                    const double c = w->c[k0 + q][j + e], d = w->D[k0 + q][j + e];
-                    ax[q].x += c * r[e].x;
-                    ax[q].y += c * r[e].y;
-                    ap[q].x += d * r[e].x;
-                    ap[q].y += d * r[e].y;
-                }
+                for (int q = q0; q < q0 + Q && q < G; q++)
+#pragma unroll
+                    for (int e = 0; e < U; e++) {
+                        const double c = w->c[k0 + q][j + e], d = w->D[k0 + q][j + e];
+                        ax[q].x += c * r[e].x;
+                        ax[q].y += c * r[e].y;
+                        ap[q].x += d * r[e].x;
+                        ap[q].y += d * r[e].y;
+                    }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
