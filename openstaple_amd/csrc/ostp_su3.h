@@ -206,6 +206,24 @@ __device__ __forceinline__ void su3_scale_add(double s, const Su3& m, Su3& acc) 
         for (int c = 0; c < 3; c++)
             acc.c[r][c] = make_double2(fma(s, m.c[r][c].x, acc.c[r][c].x), fma(s, m.c[r][c].y, acc.c[r][c].y));
 }
+// acc += a * b
+__device__ __forceinline__ void su3_mul_acc(const Su3& a, const Su3& b, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) acc.c[r][c] = cfma(a.c[r][k], b.c[k][c], acc.c[r][c]);
+}
+// acc += a^+ * b
+__device__ __forceinline__ void su3_dag_mul_acc(const Su3& a, const Su3& b, Su3& acc) {
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int c = 0; c < 3; c++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) acc.c[r][c] = cfmac(a.c[k][r], b.c[k][c], acc.c[r][c]);
+}
 // full Hermitian matrix of a thmat
 __device__ __forceinline__ void th_full(const Thmat& l, Su3& o) {
     o.c[0][0] = creal2(l.rc00);
@@ -217,6 +235,43 @@ __device__ __forceinline__ void th_full(const Thmat& l, Su3& o) {
     o.c[2][0] = cconj(l.c02);
     o.c[2][1] = cconj(l.c12);
     o.c[2][2] = creal2(-l.rc00 - l.rc11);
+}
+// Products with a thmat: its diagonal is real, so nine of the 27 complex
+// products take two multiply-adds instead of four.
+__device__ __forceinline__ double2 crfma(double r, double2 v, double2 acc) {
+    return make_double2(fma(r, v.x, acc.x), fma(r, v.y, acc.y));
+}
+// element (r, c), c = 0..2 of m * l for the row (m0, m1, m2), added to o
+__device__ __forceinline__ void th_row(double2 m0, double2 m1, double2 m2, const Thmat& l, double2 (&o)[3]) {
+    o[0] = crfma(l.rc00, m0, cfmac(l.c01, m1, cfmac(l.c02, m2, o[0])));
+    o[1] = crfma(l.rc11, m1, cfma(l.c01, m0, cfmac(l.c12, m2, o[1])));
+    o[2] = crfma(-l.rc00 - l.rc11, m2, cfma(l.c02, m0, cfma(l.c12, m1, o[2])));
+}
+// acc += l * m
+__device__ __forceinline__ void th_mul_acc(const Thmat& l, const Su3& m, Su3& acc) {
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const double2 m0 = m.c[0][c], m1 = m.c[1][c], m2 = m.c[2][c];
+        acc.c[0][c] = crfma(l.rc00, m0, cfma(l.c01, m1, cfma(l.c02, m2, acc.c[0][c])));
+        acc.c[1][c] = crfma(l.rc11, m1, cfmac(l.c01, m0, cfma(l.c12, m2, acc.c[1][c])));
+        acc.c[2][c] = crfma(-l.rc00 - l.rc11, m2, cfmac(l.c02, m0, cfmac(l.c12, m1, acc.c[2][c])));
+    }
+}
+__device__ __forceinline__ void th_sub(const Thmat& a, const Thmat& b, Thmat& o) {
+    o.c01 = csub(a.c01, b.c01);
+    o.c02 = csub(a.c02, b.c02);
+    o.c12 = csub(a.c12, b.c12);
+    o.rc00 = a.rc00 - b.rc00;
+    o.rc11 = a.rc11 - b.rc11;
+}
+__device__ __forceinline__ Thmat th_neg(const Thmat& a) {
+    Thmat o;
+    o.c01 = make_double2(-a.c01.x, -a.c01.y);
+    o.c02 = make_double2(-a.c02.x, -a.c02.y);
+    o.c12 = make_double2(-a.c12.x, -a.c12.y);
+    o.rc00 = -a.rc00;
+    o.rc11 = -a.rc11;
+    return o;
 }
 // scaled traceless anti-Hermitian part (RHO_times_mat1_times_mat2_into_tamat3)
 __device__ __forceinline__ void ta_part(const Su3& X, double s, Tamat& q) {
