@@ -228,8 +228,8 @@ bool launch_conf_times_force_ta(const void* u, const void* aux, void* ipdot) {
     return hip_ok(hipGetLastError(), "k_conf_times_force_ta");
 }
 
-bool launch_stout(const void* u, void* uout, double rho, double c0, void* stap, void* qa, void* expo);
-bool launch_sigma_chain(void* sigma, void* lam, void* qa, const void* u, double rho, double c0);
+bool launch_stout_levels(const void* u, char* arr, int steps, double rho, char* qa);
+bool launch_sigma_chain(void* sigma, void* lam, void* qa, const void* u, double rho, double c0, bool qa_given);
 double stout_c_zero();
 
 // library-owned scratch (the reference's globals aux_th, aux_ta, conf_acc_f and
@@ -248,6 +248,12 @@ struct Scratch {
     }
 };
 static Scratch g_hs, g_th, g_ta, g_conf_f, g_xs_all;
+
+// s has room for `need` bytes or a quarter of the free memory holds them
+static bool ample(const Scratch& s, size_t need) {
+    size_t free_b = 0, total_b = 0;
+    return need <= s.n || (hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= free_b / 4);
+}
 
 // the rational solves of several sources on one operator, together (solvers.hip)
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
@@ -366,8 +372,17 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
     void* dtaux = resolve(taux_conf_acc, gb, nm);
     if (!dconf || (steps > 0 && !darr) || !dgl3 || !dip || !dtaux || !tfermion_parameters) return;
     hipStream_t s = ctx().stream;
+    // each level's QA is kept for the chain back through the levels (without ample
+    // room for all of them the chain forms them again)
+    char* qa_all = nullptr;
     if (steps > 0) {
-        stout_wrapper(tconf_acc, tstout_conf_acc_arr, 0);
+        const unsigned long e0 = error_count();
+        if (ample(g_ta, steps * tb)) qa_all = (char*)g_ta.get(steps * tb);
+        if (!qa_all) {
+            (void)hipGetLastError();
+            forgive_errors(e0);
+        }
+        if (!launch_stout_levels(dconf, darr, steps, gl_stout_rho, qa_all)) return;
     }
     const void* conf_to_use = steps > 0 ? (const void*)(darr + (steps - 1) * gb) : dconf;
     if (!hip_ok(hipMemsetAsync(dgl3, 0, gb, s), nm) || !hip_ok(hipMemsetAsync(dip, 0, tb, s), nm)) return;
@@ -405,9 +420,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         const size_t all = (size_t)n * maxo * L.vec3_bytes();
         char* xs_all = n >= 2 ? (char*)g_xs_all.get(all) : nullptr;
         char* hs_all = nullptr;
-        size_t free_b = 0, total_b = 0;
-        if (xs_all && (all <= g_hs.n || (hipMemGetInfo(&free_b, &total_b) == hipSuccess && all <= free_b / 4)))
-            hs_all = (char*)g_hs.get(all);
+        if (xs_all && ample(g_hs, all)) hs_all = (char*)g_hs.get(all);
         if (xs_all && !hs_all) {
             (void)hipGetLastError();
             forgive_errors(e0);
@@ -466,11 +479,12 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
     }
     if (steps > 0) {
         void* th = g_th.get(tb);
-        void* ta = g_ta.get(tb);
+        char* ta = qa_all ? qa_all : (char*)g_ta.get(tb);
         if (!th || !ta) return;
-        for (int level = steps; level > 1; level--)
-            if (!launch_sigma_chain(dgl3, th, ta, darr + (level - 2) * gb, gl_stout_rho, stout_c_zero())) return;
-        if (!launch_sigma_chain(dgl3, th, ta, dconf, gl_stout_rho, stout_c_zero())) return;
+        for (int level = steps - 1; level >= 0; level--)
+            if (!launch_sigma_chain(dgl3, th, qa_all ? ta + level * tb : ta, level ? darr + (level - 1) * gb : dconf,
+                                    gl_stout_rho, stout_c_zero(), qa_all != nullptr))
+                return;
     }
     if (launch_conf_times_force_ta(dconf, dgl3, dip)) hip_ok(hipStreamSynchronize(s), nm);
 }

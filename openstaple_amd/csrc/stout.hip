@@ -1459,16 +1459,20 @@ __device__ void lambda_local(const Tamat& q, const Su3& SP, const Su3& U, Thmat&
     L.c12 = cscale(cadd(G.c[1][2], cconj(G.c[2][1])), 0.5);
 }
 
-// staples -> QA -> Lambda for every link (compute_sigma_from_sigma_prime ... first half)
+// staples -> QA -> Lambda for every link (compute_sigma_from_sigma_prime ... first half);
+// GIVEN: QA is there already, which leaves 368 bytes and the Cayley-Hamilton
+// coefficients per link instead of 18 neighbour links (225 -> 100 us on 32^3 x 8
+// for 6 us more in k_stout, which stores it)
+template <bool GIVEN>
 __global__ __launch_bounds__(kBlock) void k_qa_lambda(GaugePtrs G, const double2* __restrict__ SP, size_t su3_stride,
                                                      void* __restrict__ qa, void* __restrict__ lam, LinkGeom g,
-                                                     double rho, double c0, int qa_given) {
+                                                     double rho, double c0) {
     int dir, idxh;
     if (!link_of_tile(g.sizeh, dir, idxh)) return;
     Su3 U, S;
     load_link(G.at(dir), g.sizeh, idxh, U);
     Tamat q;
-    if (qa_given) {
+    if (GIVEN) {
         ta_load(qa, dir, g.sizeh, idxh, q);
     } else {
         int d[4];
@@ -1622,11 +1626,30 @@ bool launch_stout(const void* u, void* uout, double rho, double c0, void* stap, 
     return hip_ok(hipGetLastError(), "k_stout");
 }
 
-bool launch_sigma_chain(void* sigma, void* lam, void* qa, const void* u, double rho, double c0) {
+// the stout levels arr_1 .. arr_steps of u; qa (or null) receives each level's QA
+bool launch_stout_levels(const void* u, char* arr, int steps, double rho, char* qa) {
+    const size_t gb = 8 * ctx().lat.su3_bytes(), tb = (size_t)8 * 64 * ctx().lat.sizeh;
+    for (int level = 0; level < steps; level++)
+        if (!launch_stout(level ? arr + (level - 1) * gb : u, arr + level * gb, rho, g_c_zero, nullptr,
+                          qa ? qa + level * tb : nullptr, nullptr))
+            return false;
+    return true;
+}
+
+static bool launch_qa_lambda(bool given, const void* u, const void* sp, void* qa, void* lam, double rho, double c0) {
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(nblk_tiles()), dim3(kBlock), 0, ctx().stream, gauge_ptrs(u), (const double2*)sp,
+                           ctx().lat.su3_bytes(), qa, lam, link_geom(), rho, c0);
+    };
+    if (given) go(k_qa_lambda<true>);
+    else go(k_qa_lambda<false>);
+    return hip_ok(hipGetLastError(), "k_qa_lambda");
+}
+
+// qa_given: qa holds u's QA, else it is formed from the staples and left there
+bool launch_sigma_chain(void* sigma, void* lam, void* qa, const void* u, double rho, double c0, bool qa_given) {
     const size_t st = ctx().lat.su3_bytes();
-    hipLaunchKernelGGL(k_qa_lambda, dim3(nblk_tiles()), dim3(kBlock), 0, ctx().stream, gauge_ptrs(u),
-                       (const double2*)sigma, st, qa, lam, link_geom(), rho, c0, 0);
-    if (!hip_ok(hipGetLastError(), "k_qa_lambda")) return false;
+    if (!launch_qa_lambda(qa_given, u, sigma, qa, lam, rho, c0)) return false;
     hipLaunchKernelGGL(k_sigma, dim3(nblk_tiles()), dim3(kBlock), 0, ctx().stream, gauge_ptrs(u), (const void*)lam,
                        (const void*)qa, (double2*)sigma, st, link_geom(), rho);
     return hip_ok(hipGetLastError(), "k_sigma");
@@ -1854,11 +1877,7 @@ void stout_wrapper(const su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr, const
     const void* du = resolve(tconf_acc, gb, nm);
     char* arr = (char*)resolve(tstout_conf_acc_arr, steps * gb, nm);
     if (!du || !arr) return;
-    const double rho = rho_of(istopo);
-    if (!launch_stout(du, arr, rho, g_c_zero, nullptr, nullptr, nullptr)) return;
-    for (int level = 1; level < steps; level++)
-        if (!launch_stout(arr + (level - 1) * gb, arr + level * gb, rho, g_c_zero, nullptr, nullptr, nullptr)) return;
-    sync(nm);
+    if (launch_stout_levels(du, arr, steps, rho_of(istopo), nullptr)) sync(nm);
 }
 
 void exp_minus_QA_times_conf(const su3_soa* tu, const tamat_soa* QA, su3_soa* tu_out, su3_soa* exp_aux) {
@@ -1912,9 +1931,7 @@ void compute_lambda(thmat_soa* Lm, const su3_soa* SP, const su3_soa* U, const ta
     const void* du = resolve(U, gb, nm);
     const void* dq = resolve(QA, tb, nm);
     if (!dl || !ds || !du || !dq) return;
-    hipLaunchKernelGGL(k_qa_lambda, dim3(nblk_tiles()), dim3(kBlock), 0, ctx().stream, gauge_ptrs(du), (const double2*)ds,
-                       L.su3_bytes(), const_cast<void*>(dq), dl, link_geom(), 0.0, g_c_zero, 1);
-    if (hip_ok(hipGetLastError(), nm)) sync(nm);
+    if (launch_qa_lambda(true, du, ds, const_cast<void*>(dq), dl, 0.0, g_c_zero)) sync(nm);
 }
 
 void compute_sigma(const thmat_soa* Lm, const su3_soa* U, su3_soa* S, const tamat_soa* QA, su3_soa* TMP,
@@ -1946,7 +1963,7 @@ void compute_sigma_from_sigma_prime_backinto_sigma_prime(su3_soa* Sigma, thmat_s
     void* dq = resolve(QA, tb, nm);
     const void* du = resolve(U, gb, nm);
     if (!ds || !dl || !dq || !du) return;
-    if (launch_sigma_chain(ds, dl, dq, du, rho_of(istopo), g_c_zero)) sync(nm);
+    if (launch_sigma_chain(ds, dl, dq, du, rho_of(istopo), g_c_zero, false)) sync(nm);
 }
 
 void unitarize_conf(su3_soa* u) {
