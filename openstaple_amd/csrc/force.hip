@@ -51,7 +51,7 @@ struct ShiftCoeffs {
 //   p = 1 (odd x) : l = x_k (even field),          r = h_k (odd),  c_k = -a_k
 __global__ __launch_bounds__(kBlock) void k_direct_product(double2* __restrict__ aux, size_t su3_stride,
                                                           const double2* __restrict__ xs, const double2* __restrict__ hs,
-                                                          long vstride, ShiftCoeffs co, FGeom g) {
+                                                          long vstride, ShiftCoeffs co, FGeom g, int fresh) {
     const int gid = xcd_block_id() * kBlock + (int)threadIdx.x;
     const int sh = g.sizeh;
     if (gid >= 8 * sh) return;
@@ -81,7 +81,10 @@ __global__ __launch_bounds__(kBlock) void k_direct_product(double2* __restrict__
 #pragma unroll
     for (int a = 0; a < 3; a++)
 #pragma unroll
-        for (int b = 0; b < 3; b++) A[(3 * a + b) * sh + idxh] = cadd(A[(3 * a + b) * sh + idxh], acc.c[a][b]);
+        for (int b = 0; b < 3; b++) {
+            const long e = (3 * a + b) * sh + idxh;
+            A[e] = fresh ? acc.c[a][b] : cadd(A[e], acc.c[a][b]);
+        }
 }
 
 // The same sums with one thread per half-site and NMU directions: the
@@ -95,7 +98,7 @@ template <int NMU>
 __global__ __launch_bounds__(kBlock) void k_direct_product_sites(double2* __restrict__ aux, size_t su3_stride,
                                                                 const double2* __restrict__ xs,
                                                                 const double2* __restrict__ hs, long vstride,
-                                                                ShiftCoeffs co, FGeom g) {
+                                                                ShiftCoeffs co, FGeom g, int fresh) {
     const int gid = xcd_block_id() * kBlock + (int)threadIdx.x;
     const int sh = g.sizeh;
     constexpr int NG = 4 / NMU;
@@ -134,15 +137,18 @@ __global__ __launch_bounds__(kBlock) void k_direct_product_sites(double2* __rest
 #pragma unroll
         for (int a = 0; a < 3; a++)
 #pragma unroll
-            for (int b = 0; b < 3; b++)
-                A[(3 * a + b) * sh + idxh] = cadd(A[(3 * a + b) * sh + idxh], acc[m].c[a][b]);
+            for (int b = 0; b < 3; b++) {
+                const long e = (3 * a + b) * sh + idxh;
+                A[e] = fresh ? acc[m].c[a][b] : cadd(A[e], acc[m].c[a][b]);
+            }
     }
 }
 
 // out[dir] += aux[dir] * e^{i phase[dir]}
 __global__ __launch_bounds__(kBlock) void k_backfield_times_force(const double2* __restrict__ aux,
                                                                  double2* __restrict__ out, size_t su3_stride,
-                                                                 const double* __restrict__ phases, int sizeh) {
+                                                                 const double* __restrict__ phases, int sizeh,
+                                                                 int fresh) {
     const int gid = blockIdx.x * kBlock + (int)threadIdx.x;
     if (gid >= 8 * sizeh) return;
     const int dir = gid / sizeh, i = gid - dir * sizeh;
@@ -152,13 +158,14 @@ __global__ __launch_bounds__(kBlock) void k_backfield_times_force(const double2*
     const double2* A = (const double2*)((const char*)aux + dir * su3_stride);
     double2* O = (double2*)((char*)out + dir * su3_stride);
 #pragma unroll
-    for (int k = 0; k < 9; k++) O[k * sizeh + i] = cfma(A[k * sizeh + i], ph, O[k * sizeh + i]);
+    for (int k = 0; k < 9; k++)
+        O[k * sizeh + i] = cfma(A[k * sizeh + i], ph, fresh ? make_double2(0.0, 0.0) : O[k * sizeh + i]);
 }
 
 // ipdot[dir] -= TA(U[dir] * aux[dir])
 __global__ __launch_bounds__(kBlock) void k_conf_times_force_ta(const double2* __restrict__ u,
                                                                const double2* __restrict__ aux, size_t su3_stride,
-                                                               void* __restrict__ ipdot, int sizeh) {
+                                                               void* __restrict__ ipdot, int sizeh, int fresh) {
     const int gid = blockIdx.x * kBlock + (int)threadIdx.x;
     if (gid >= 8 * sizeh) return;
     const int dir = gid / sizeh, i = gid - dir * sizeh;
@@ -180,11 +187,12 @@ __global__ __launch_bounds__(kBlock) void k_conf_times_force_ta(const double2* _
     char* b = (char*)ipdot + (size_t)dir * 64 * sizeh;
     double2* pc = (double2*)b;
     double* pd = (double*)(b + (size_t)48 * sizeh);
-    pc[i] = csub(pc[i], t.c01);
-    pc[sizeh + i] = csub(pc[sizeh + i], t.c02);
-    pc[2 * sizeh + i] = csub(pc[2 * sizeh + i], t.c12);
-    pd[i] -= t.ic00;
-    pd[sizeh + i] -= t.ic11;
+    const double2 zero = make_double2(0.0, 0.0);
+    pc[i] = csub(fresh ? zero : pc[i], t.c01);
+    pc[sizeh + i] = csub(fresh ? zero : pc[sizeh + i], t.c02);
+    pc[2 * sizeh + i] = csub(fresh ? zero : pc[2 * sizeh + i], t.c12);
+    pd[i] = (fresh ? 0.0 : pd[i]) - t.ic00;
+    pd[sizeh + i] = (fresh ? 0.0 : pd[sizeh + i]) - t.ic11;
 }
 
 static FGeom fgeom() {
@@ -198,7 +206,9 @@ static int nblk8() { return blocks_for(8 * ctx().lat.sizeh); }
 
 static int g_dp_kernel = 4;  // links of a site per thread in the outer-product kernel (0: one thread per link)
 
-bool launch_direct_product(void* aux, const void* xs, const void* hs, const double* a, int order) {
+// The three steps add to their outputs; fresh: as if those were zero, without
+// reading them (nor need anyone have cleared them).
+bool launch_direct_product(void* aux, const void* xs, const void* hs, const double* a, int order, bool fresh) {
     ShiftCoeffs co;
     co.order = order;
     for (int k = 0; k < kMaxShifts; k++) co.a[k] = k < order ? a[k] : 0.0;
@@ -206,25 +216,25 @@ bool launch_direct_product(void* aux, const void* xs, const void* hs, const doub
     const size_t st = ctx().lat.su3_bytes();
     if (g_dp_kernel == 4)
         hipLaunchKernelGGL((k_direct_product_sites<4>), dim3(blocks_for(2 * sh)), dim3(kBlock), 0, ctx().stream,
-                           (double2*)aux, st, (const double2*)xs, (const double2*)hs, 3 * sh, co, fgeom());
+                           (double2*)aux, st, (const double2*)xs, (const double2*)hs, 3 * sh, co, fgeom(), (int)fresh);
     else if (g_dp_kernel == 2)
         hipLaunchKernelGGL((k_direct_product_sites<2>), dim3(blocks_for(4 * sh)), dim3(kBlock), 0, ctx().stream,
-                           (double2*)aux, st, (const double2*)xs, (const double2*)hs, 3 * sh, co, fgeom());
+                           (double2*)aux, st, (const double2*)xs, (const double2*)hs, 3 * sh, co, fgeom(), (int)fresh);
     else
         hipLaunchKernelGGL(k_direct_product, dim3(nblk8()), dim3(kBlock), 0, ctx().stream, (double2*)aux, st,
-                           (const double2*)xs, (const double2*)hs, 3 * sh, co, fgeom());
+                           (const double2*)xs, (const double2*)hs, 3 * sh, co, fgeom(), (int)fresh);
     return hip_ok(hipGetLastError(), "k_direct_product");
 }
 
-bool launch_backfield_times_force(const void* aux, void* out, const void* phases) {
+bool launch_backfield_times_force(const void* aux, void* out, const void* phases, bool fresh) {
     hipLaunchKernelGGL(k_backfield_times_force, dim3(nblk8()), dim3(kBlock), 0, ctx().stream, (const double2*)aux,
-                       (double2*)out, ctx().lat.su3_bytes(), (const double*)phases, (int)ctx().lat.sizeh);
+                       (double2*)out, ctx().lat.su3_bytes(), (const double*)phases, (int)ctx().lat.sizeh, (int)fresh);
     return hip_ok(hipGetLastError(), "k_backfield_times_force");
 }
 
-bool launch_conf_times_force_ta(const void* u, const void* aux, void* ipdot) {
+bool launch_conf_times_force_ta(const void* u, const void* aux, void* ipdot, bool fresh) {
     hipLaunchKernelGGL(k_conf_times_force_ta, dim3(nblk8()), dim3(kBlock), 0, ctx().stream, (const double2*)u,
-                       (const double2*)aux, ctx().lat.su3_bytes(), ipdot, (int)ctx().lat.sizeh);
+                       (const double2*)aux, ctx().lat.su3_bytes(), ipdot, (int)ctx().lat.sizeh, (int)fresh);
     return hip_ok(hipGetLastError(), "k_conf_times_force_ta");
 }
 
@@ -260,20 +270,21 @@ bool multishift_fp64_many(const void* u, ferm_param* const* pars, const Rational
                           const void* const* in, void* const* out, int n, double res, int max_cg,
                           int convergence_importance, void* const* hs);
 
-// sum over shifts of the outer products for one pseudofermion; hs: D_oe x_k
+// sum over shifts of the outer products for one pseudofermion, to aux (fresh: of
+// any content) or added to it; hs: D_oe x_k
 // where the solver has left them, null to form them here
 bool compute_fermion_force(const void* u, void* aux, const void* xs, const void* phases, const RationalApprox* ra,
-                           const void* hs = nullptr) {
+                           const void* hs, bool fresh) {
     const Lattice& L = ctx().lat;
     const int order = ra->approx_order;
-    if (order <= 0) return true;
+    if (order <= 0) return !fresh || hip_ok(hipMemsetAsync(aux, 0, 8 * L.su3_bytes(), ctx().stream), "no shifts");
     if (!hs) {
         void* h = g_hs.get((size_t)order * L.vec3_bytes());
         // all D_oe x_k, the shifts' solutions in chunks through shared-link hops
         if (!h || !launch_doe_multi(u, phases, xs, h, order)) return false;
         hs = h;
     }
-    return launch_direct_product(aux, xs, hs, ra->RA_a, order);
+    return launch_direct_product(aux, xs, hs, ra->RA_a, order, fresh);
 }
 
 }  // namespace ostp
@@ -306,7 +317,7 @@ void direct_product_of_fermions_into_auxmat(const vec3_soa* loc_s, const vec3_so
     if (!ds || !dh || !da || !approx) return;
     if (iter < 0 || iter >= approx->approx_order) { fail("%s: shift %d out of range", nm, iter); return; }
     double a = approx->RA_a[iter];
-    if (launch_direct_product(da, ds, dh, &a, 1)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
+    if (launch_direct_product(da, ds, dh, &a, 1, false)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
 }
 
 void multiply_backfield_times_force(ferm_param* tpars, const su3_soa* auxmat, su3_soa* pseudo_ipdot) {
@@ -317,7 +328,7 @@ void multiply_backfield_times_force(ferm_param* tpars, const su3_soa* auxmat, su
     const void* da = resolve(auxmat, 8 * L.su3_bytes(), nm);
     void* dout = resolve(pseudo_ipdot, 8 * L.su3_bytes(), nm);
     if (!dph || !da || !dout) return;
-    if (launch_backfield_times_force(da, dout, dph)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
+    if (launch_backfield_times_force(da, dout, dph, false)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
 }
 
 void multiply_conf_times_force_and_take_ta_nophase(const su3_soa* u, const su3_soa* auxmat, tamat_soa* ipdot) {
@@ -328,7 +339,7 @@ void multiply_conf_times_force_and_take_ta_nophase(const su3_soa* u, const su3_s
     const void* da = resolve(auxmat, 8 * L.su3_bytes(), nm);
     void* dp = resolve(ipdot, (size_t)8 * 64 * L.sizeh, nm);
     if (!du || !da || !dp) return;
-    if (launch_conf_times_force_ta(du, da, dp)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
+    if (launch_conf_times_force_ta(du, da, dp, false)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
 }
 
 void ker_openacc_compute_fermion_force(const su3_soa* u, su3_soa* aux_u, const vec3_soa* in_shiftmulti,
@@ -345,7 +356,7 @@ void ker_openacc_compute_fermion_force(const su3_soa* u, su3_soa* aux_u, const v
     const void* dx = resolve(in_shiftmulti, (size_t)(order > 0 ? order : 1) * L.vec3_bytes(), nm);
     const void* dph = resolve(tpars->phases, 8 * L.dsoa_bytes(), nm);
     if (!du || !da || !dx || !dph) return;
-    if (compute_fermion_force(du, da, dx, dph, &tpars->approx_md)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
+    if (compute_fermion_force(du, da, dx, dph, &tpars->approx_md, nullptr, false)) hip_ok(hipStreamSynchronize(ctx().stream), nm);
 }
 
 int inverter_multishift_wrapper(inverter_package ip, ferm_param* pars, RationalApprox* approx, vec3_soa* out,
@@ -385,7 +396,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         if (!launch_stout_levels(dconf, darr, steps, gl_stout_rho, qa_all)) return;
     }
     const void* conf_to_use = steps > 0 ? (const void*)(darr + (steps - 1) * gb) : dconf;
-    if (!hip_ok(hipMemsetAsync(dgl3, 0, gb, s), nm) || !hip_ok(hipMemsetAsync(dip, 0, tb, s), nm)) return;
+    if (tNDiffFlavs <= 0 && !hip_ok(hipMemsetAsync(dgl3, 0, gb, s), nm)) return;
     ipt.u = (const su3_soa*)conf_to_use;
     if (inverter_tricks.singlePInvAccelMultiInv) {
         void* cf = g_conf_f.get(8 * L.su3f_bytes());
@@ -443,14 +454,14 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
             int k = 0;
             for (int iflav = 0; iflav < tNDiffFlavs; iflav++) {
                 ferm_param* fp = &tfermion_parameters[iflav];
-                if (!hip_ok(hipMemsetAsync(dtaux, 0, gb, s), nm)) return;
+                if (fp->number_of_ps <= 0 && !hip_ok(hipMemsetAsync(dtaux, 0, gb, s), nm)) return;
                 const void* dph = resolve(fp->phases, 8 * L.dsoa_bytes(), nm);
                 if (!dph) return;
                 for (int ips = 0; ips < fp->number_of_ps; ips++, k++)
                     if (!compute_fermion_force(conf_to_use, dtaux, outs[k], dph, &fp->approx_md,
-                                               hs_all ? hs[k] : nullptr))
+                                               hs_all ? hs[k] : nullptr, ips == 0))
                         return;
-                if (!launch_backfield_times_force(dtaux, dgl3, dph)) return;
+                if (!launch_backfield_times_force(dtaux, dgl3, dph, iflav == 0)) return;
             }
             // the shifted solutions of the last source stay in tferm_shiftmulti_acc, as after the loop below
             const int order = fps[n - 1]->approx_md.approx_order;
@@ -463,7 +474,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
     }
     for (int iflav = 0; !together && iflav < tNDiffFlavs; iflav++) {
         ferm_param* fp = &tfermion_parameters[iflav];
-        if (!hip_ok(hipMemsetAsync(dtaux, 0, gb, s), nm)) return;
+        if (fp->number_of_ps <= 0 && !hip_ok(hipMemsetAsync(dtaux, 0, gb, s), nm)) return;
         const int ifps = fp->index_of_the_first_ps;
         const void* dph = resolve(fp->phases, 8 * L.dsoa_bytes(), nm);
         const int order = fp->approx_md.approx_order;
@@ -473,9 +484,9 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
             const vec3_soa* in = (const vec3_soa*)((const char*)ferm_in_acc + (size_t)(ifps + ips) * L.vec3_bytes());
             inverter_multishift_wrapper(ipt, fp, &fp->approx_md, tferm_shiftmulti_acc, in, res, max_cg,
                                         CONVERGENCE_NONCRITICAL);
-            if (!compute_fermion_force(conf_to_use, dtaux, dxs, dph, &fp->approx_md)) return;
+            if (!compute_fermion_force(conf_to_use, dtaux, dxs, dph, &fp->approx_md, nullptr, ips == 0)) return;
         }
-        if (!launch_backfield_times_force(dtaux, dgl3, dph)) return;
+        if (!launch_backfield_times_force(dtaux, dgl3, dph, iflav == 0)) return;
     }
     if (steps > 0) {
         void* th = g_th.get(tb);
@@ -486,7 +497,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
                                     gl_stout_rho, stout_c_zero(), qa_all != nullptr))
                 return;
     }
-    if (launch_conf_times_force_ta(dconf, dgl3, dip)) hip_ok(hipStreamSynchronize(s), nm);
+    if (launch_conf_times_force_ta(dconf, dgl3, dip, true)) hip_ok(hipStreamSynchronize(s), nm);
 }
 
 }  // extern "C"
