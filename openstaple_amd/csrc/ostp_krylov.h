@@ -74,21 +74,23 @@ struct KrArgs {
     int n, tmajor, rev;
 };
 
-// sum of n partials by one wave, in the same order wherever it runs
-// (kr_part a lane's share, kr_wave the wave's total)
-__device__ __forceinline__ double kr_part(const double* __restrict__ part, int n, int stride, int lane) {
+// sum of n partials by T threads (a wave; a block, for whom the thousands of a
+// large lattice are one round of loads), in the same order wherever it runs:
+// kr_part a thread's share, kr_wave the wave's total, kr_block the block's
+template <int T = 64>
+__device__ __forceinline__ double kr_part(const double* __restrict__ part, int n, int stride, int thread) {
     double v = 0.0;
-    int i = lane;
-    for (; i + 448 < n; i += 512) {
+    int i = thread;
+    for (; i + 7 * T < n; i += 8 * T) {
         double t[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) t[q] = part[(long)(i + 64 * q) * stride];
+        for (int q = 0; q < 8; q++) t[q] = part[(long)(i + T * q) * stride];
 #pragma unroll
         for (int q = 0; q < 8; q++) v += t[q];
     }
     double t[8];
 #pragma unroll
-    for (int q = 0; q < 8; q++) t[q] = i + 64 * q < n ? part[(long)(i + 64 * q) * stride] : 0.0;
+    for (int q = 0; q < 8; q++) t[q] = i + T * q < n ? part[(long)(i + T * q) * stride] : 0.0;
 #pragma unroll
     for (int q = 0; q < 8; q++) v += t[q];
     return v;
@@ -98,17 +100,27 @@ __device__ __forceinline__ double kr_wave(double v) {
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
+__device__ __forceinline__ double kr_block(double v, double (&lds)[kBlock / 64]) {
+    v = kr_wave(v);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = v;
+    __syncthreads();
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; w++) t += lds[w];
+    return t;
+}
 
 // End of iteration j - 1 of system k by one wave: the new state (stored when
 // `store`), *gamma and whether iteration j runs.  The window's coefficients
-// are advanced by the storing block (per-shift values through sh).
+// are advanced by the storing block (per-shift values through sh).  total: |r|^2
+// where the block has summed it already.
 __device__ __forceinline__ void kr_end(const KrArgs& a, int k, int lane, bool store, double* gamma, int* running,
-                                       double (*sh)[kMaxShifts], int* on) {
+                                       double (*sh)[kMaxShifts], int* on, const double* total = nullptr) {
     const SolverState* prev = a.st[k] + ((a.j - 1) & 1);
     SolverState* next = a.st[k] + (a.j & 1);
     // every load is issued before the first wait
     double sum = 0.0;
-    if (a.j > 1) sum = kr_part(a.partB[k], a.nB, 1, lane);
+    if (a.j > 1 && !total) sum = kr_part(a.partB[k], a.nB, 1, lane);
     const int status0 = prev->status;
     int status = status0, cg = prev->cg, restarted = prev->cg_restarted, maxiter = prev->maxiter;
     double g = 0.0, delta = prev->delta, lambda = prev->lambda;
@@ -124,7 +136,7 @@ __device__ __forceinline__ void kr_end(const KrArgs& a, int k, int lane, bool st
         f = prev->flags[0][lane];
     }
     if (a.j > 1 && status0 == kRunning) {
-        lambda = kr_wave(sum);
+        lambda = total ? *total : kr_wave(sum);
         g = lambda / delta;
         cg += 1;
         if (a.ms) {
@@ -465,13 +477,13 @@ __global__ __launch_bounds__(kKrThreads) void k_kr_deo(KrArgs a) {
 }
 
 // The streaming kernels: blockIdx.y = system, blocks over the half-sites in
-// strides; the first two sites' operands are loaded before the block waits
-// for its scalars.
+// strides; the operands of a thread's first two sites (of its one site, where
+// the grid covers the lattice) are loaded before the block waits for its scalars.
 constexpr int kKrAhead = 2;
 
 // End of iteration j - 1 and p = r + gamma p
 __global__ __launch_bounds__(kBlock) void k_kr_p(KrArgs a) {
-    __shared__ double sh_gamma, sh_k[3][kMaxShifts];
+    __shared__ double sh_gamma, sh_k[3][kMaxShifts], lds[kBlock / 64];
     __shared__ int sh_run, sh_on[kMaxShifts + 1];
     const int k = (int)blockIdx.y, tid = (int)threadIdx.x, sh = a.g.sizeh;
     const bool store = blockIdx.x == 0;
@@ -480,14 +492,17 @@ __global__ __launch_bounds__(kBlock) void k_kr_p(KrArgs a) {
     double2* p = a.p[k];
     double2 rr[kKrAhead][3], pp[kKrAhead][3];
 #pragma unroll
-    for (int q = 0; q < kKrAhead; q++)
+    for (int q = 0; q < kKrAhead; q++) {
+        if (q * step >= sh) break;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const long e = (long)c * sh + (i0 + q * step < sh ? i0 + q * step : 0);
             rr[q][c] = r[e];
             pp[q][c] = p[e];
         }
-    if (tid < 64) kr_end(a, k, tid, store, &sh_gamma, &sh_run, sh_k, sh_on);
+    }
+    const double total = kr_block(a.j > 1 ? kr_part<kBlock>(a.partB[k], a.nB, 1, tid) : 0.0, lds);
+    if (tid < 64) kr_end(a, k, tid, store, &sh_gamma, &sh_run, sh_k, sh_on, &total);
     __syncthreads();
     if (store && a.ms && sh_on[kMaxShifts] && a.win[k]) kr_window(a.win[k], a.st[k][a.j & 1].order, sh_k, sh_on, tid, kBlock);
     if (!sh_run || a.close) return;
@@ -537,7 +552,8 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
     double2 *rn = a.rn[k], *x = a.x[k];
     double2 ra[kKrAhead][3], sa[kKrAhead][3], pa[kKrAhead][3], xa[kKrAhead][3];
 #pragma unroll
-    for (int q = 0; q < kKrAhead; q++)
+    for (int q = 0; q < kKrAhead; q++) {
+        if (q * step >= sh) break;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const long e = (long)c * sh + (i0 + q * step < sh ? i0 + q * step : 0);
@@ -548,11 +564,11 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
                 xa[q][c] = x[e];
             }
         }
+    }
+    const double tot = kr_block(kr_part<kBlock>(a.partA[k], a.nA, a.sA, tid), lds);
     if (tid < 64) {
-        const double part = kr_part(a.partA[k], a.nA, a.sA, lane);
         const double delta = st->delta;
         const int running = st->status == kRunning;
-        const double tot = kr_wave(part);
         const double om = MS ? -delta / tot : delta / tot;
         if (lane == 0) {
             sh_om = om;
@@ -601,7 +617,7 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
             const long e = (long)c * sh + i;
             one(e, r[e], s[e], MS ? r[e] : p[e], MS ? r[e] : x[e]);
         }
-    const double t = block_sum<kBlock>(v, lds);
+    const double t = block_sum<kBlock>(v, lds);  // (the barrier above lies after every read of lds)
     if (tid == 0) a.partB[k][blockIdx.x] = t;
 }
 
@@ -635,30 +651,31 @@ __device__ __forceinline__ float2 mx_p(float2 r, float2 p, double g) {
 }
 
 __global__ __launch_bounds__(kBlock) void k_mx_p(MxArgs a) {
-    __shared__ double sh_gamma;
+    __shared__ double sh_gamma, lds[kBlock / 64], ldst[kBlock / 64];
     __shared__ int sh_run;
     const int tid = (int)threadIdx.x, sh = a.sizeh;
     const int i0 = (int)blockIdx.x * kBlock + tid, step = (int)gridDim.x * kBlock;
     float2 rr[kKrAhead][3], pp[kKrAhead][3];
 #pragma unroll
-    for (int q = 0; q < kKrAhead; q++)
+    for (int q = 0; q < kKrAhead; q++) {
+        if (q * step >= sh) break;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const long e = (long)c * sh + (i0 + q * step < sh ? i0 + q * step : 0);
             rr[q][c] = a.rf[e];
             pp[q][c] = a.pf[e];
         }
+    }
+    const double sumt = a.tail ? kr_block(kr_part<kBlock>(a.partT, a.nT, 2, tid), ldst) : 0.0;
+    const double sum = kr_block(a.j > 1 ? kr_part<kBlock>(a.partB, a.nB, 1, tid) : 0.0, lds);
     if (tid < 64) {
         const SolverState* prev = a.st + ((a.j - 1) & 1);
         SolverState* next = a.st + (a.j & 1);
-        double sum = 0.0, sumt = 0.0;
-        if (a.j > 1) sum = kr_part(a.partB, a.nB, 1, tid);
-        if (a.tail) sumt = kr_part(a.partT, a.nT, 2, tid);
         double delta = prev->delta, lambda = prev->lambda, g = 0.0, last = prev->last_max_res;
         int status = prev->status, cg = prev->cg, rus = prev->ru_count, ru = prev->ru;
         const bool hold = a.j > 1 && status == kRunning && ru && !a.tail;
         if (a.j > 1 && status == kRunning && !hold) {
-            lambda = kr_wave(ru ? sumt : sum);
+            lambda = ru ? sumt : sum;
             g = lambda / delta;
             delta = lambda;
             cg += 1;
@@ -723,7 +740,8 @@ __global__ __launch_bounds__(kBlock) void k_mx_xr(MxArgs a) {
     const int i0 = (int)blockIdx.x * kBlock + tid, step = (int)gridDim.x * kBlock;
     float2 pa[kKrAhead][3], oa[kKrAhead][3], ra[kKrAhead][3], sa[kKrAhead][3];
 #pragma unroll
-    for (int q = 0; q < kKrAhead; q++)
+    for (int q = 0; q < kKrAhead; q++) {
+        if (q * step >= sh) break;
 #pragma unroll
         for (int c = 0; c < 3; c++) {
             const long e = (long)c * sh + (i0 + q * step < sh ? i0 + q * step : 0);
@@ -732,10 +750,11 @@ __global__ __launch_bounds__(kBlock) void k_mx_xr(MxArgs a) {
             ra[q][c] = a.rf[e];
             sa[q][c] = a.sf[e];
         }
+    }
+    const double tot = kr_block(kr_part<kBlock>(a.partA, a.nA, 2, tid), lds);
     if (tid < 64) {
-        const double part = kr_part(a.partA, a.nA, 2, tid);
         const int go = st->status == kRunning && !st->hold, ru = st->ru;
-        const double tot = kr_wave(part), om = st->delta / tot;
+        const double om = st->delta / tot;
         if (tid == 0) {
             sh_om = om;
             sh_go = go;
