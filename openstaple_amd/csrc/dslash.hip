@@ -32,6 +32,7 @@ struct DslashArgs {
     double m2;
     const double2* b;   // kMdagMResid
     float2* rf;
+    const unsigned char* sg;  // signs of the hops (SGN), of this output parity
     SiteGeom g;
     int tmajor;         // workgroup order: t-slices fastest (see k_dslash)
     int rev;            // each XCD walks its slab backwards
@@ -84,7 +85,7 @@ __device__ __forceinline__ int dslash_idx(const DslashArgs<R>& a, int blk, int s
 }
 
 // EO = 0: Deo (even output, odd input); EO = 1: Doe.
-template <typename R, int EO, int MODE>
+template <typename R, int EO, int MODE, bool SGN = false>
 __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<R> a) {
     using C = typename Cplx<R>::T;
     if (!pred_pass(a.ctl)) return;
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(kBlock) void k_dslash(DslashArgs<R> a) {
     double dot = 0.0;
     if (idx < a.g.sizeh) {
         C o[3];
-        dslash_site<R, EO>(a.u, a.ph, a.in, a.g, idx, o[0], o[1], o[2]);
+        dslash_site<R, EO, SGN>(a.u, a.ph, a.in, a.g, idx, o[0], o[1], o[2], SGN ? a.sg[idx] : 0u);
         C x[3];
 #pragma unroll
         for (int c = 0; c < 3; c++) x[c] = MODE == kPlain ? o[c] : a.x[(long)c * a.g.sizeh + idx];
@@ -177,6 +178,11 @@ static void go(const DslashArgs<R>& a) {
     const dim3 blocks(dslash_blocks<R>());
     if constexpr (sizeof(R) == 8)
         if (!dslash_split<R>()) {
+            if constexpr (MODE == kPlain || MODE == kMdagMDot)
+                if (a.sg) {
+                    hipLaunchKernelGGL((k_dslash<R, EO, MODE, true>), blocks, dim3(kBlock), 0, ctx().stream, a);
+                    return;
+                }
             hipLaunchKernelGGL((k_dslash<R, EO, MODE>), blocks, dim3(kBlock), 0, ctx().stream, a);
             return;
         }
@@ -199,6 +205,7 @@ static bool fill_args(DslashArgs<R>& a, const void* u_dev, const void* ph_dev, c
     a.m2 = 0.0;
     a.b = nullptr;
     a.rf = nullptr;
+    a.sg = nullptr;
     a.g.nd0 = L.nd[0];
     a.g.nd0h = L.nd[0] / 2;
     a.g.nd1 = L.nd[1];
@@ -215,9 +222,10 @@ static bool fill_args(DslashArgs<R>& a, const void* u_dev, const void* ph_dev, c
 // Launch one Dslash on device pointers.  mode/fin select the fused epilogue.
 template <typename R>
 bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, const void* in, void* out,
-                   const void* x, double m2, const SolverCtl& ctl) {
+                   const void* x, double m2, const SolverCtl& ctl, const unsigned char* sg) {
     DslashArgs<R> a;
     fill_args<R>(a, u, ph, in, out);
+    if (sg) a.sg = sg + eo * ctx().lat.sizeh;
     a.x = (const typename Cplx<R>::T*)x;
     a.m2 = m2;
     a.ctl = ctl;
@@ -237,9 +245,71 @@ bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, con
 }
 
 template bool launch_dslash<double>(int, int, int, const void*, const void*, const void*, void*, const void*,
-                                    double, const SolverCtl&);
+                                    double, const SolverCtl&, const unsigned char*);
 template bool launch_dslash<float>(int, int, int, const void*, const void*, const void*, void*, const void*,
-                                   double, const SolverCtl&);
+                                   double, const SolverCtl&, const unsigned char*);
+
+// Signs of the hops.  A phase that is +-1 to rounding (its sine within two
+// roundings of pi) is taken as its sign: 1 byte a half-site instead of 64 of
+// the 928 a hop reads, and a hop without its rotation.  The solvers scan the
+// phases once per solve where their hops are the ordinary ones (above
+// kHopSplitSizeh, where a solve takes milliseconds against the scan's 30 us; the
+// small lattices' iterations are not bound by bytes): 204 iterations with 19
+// shifts on 32^4 42.28 -> 41.49 ms, a force of two systems on 32^3 x 8 6.50 -> 6.39.
+struct SignArgs {
+    const double* ph[8];
+    SiteGeom g;
+    unsigned char* sg;
+    int* bad;
+};
+template <int EO>
+__device__ __forceinline__ unsigned sign_bits(const SignArgs& a, int idx, bool& bad) {
+    constexpr int F = EO == 0 ? 0 : 1, B = 1 - F;
+    const Nbrs nb = site_neighbours<EO>(a.g, idx);
+    unsigned bits = 0;
+#pragma unroll
+    for (int h = 0; h < 8; h++) {
+        const int mu = h & 3;
+        double s, c;
+        phase_sincos(a.ph[2 * mu + (h < 4 ? B : F)][h < 4 ? nb.im[mu] : idx], &s, &c);
+        if (!(fabs(s) <= 2.5e-16) || fabs(c) != 1.0) bad = true;
+        bits |= c < 0.0 ? 1u << h : 0u;
+    }
+    return bits;
+}
+__global__ __launch_bounds__(kBlock) void k_phase_signs(SignArgs a) {
+    const int idx = (int)blockIdx.x * kBlock + (int)threadIdx.x, sh = a.g.sizeh;
+    if (idx >= sh) return;
+    bool bad = false;
+    a.sg[idx] = (unsigned char)sign_bits<0>(a, idx, bad);
+    a.sg[sh + idx] = (unsigned char)sign_bits<1>(a, idx, bad);
+    if (bad) *a.bad = 1;
+}
+static Workspace g_signs;
+const unsigned char* phase_signs(const void* ph) {
+    const Lattice& L = ctx().lat;
+    const size_t n = (2 * (size_t)L.sizeh + 255) / 256 * 256;
+    char* w = (char*)g_signs.try_get(n + 256);
+    if (!w) return nullptr;
+    SignArgs a;
+    for (int l = 0; l < 8; l++) a.ph[l] = (const double*)((const char*)ph + l * L.dsoa_bytes());
+    a.g.nd0 = L.nd[0];
+    a.g.nd0h = L.nd[0] / 2;
+    a.g.nd1 = L.nd[1];
+    a.g.nd2 = L.nd[2];
+    a.g.nd3 = L.nd[3];
+    a.g.sizeh = (int)L.sizeh;
+    a.sg = (unsigned char*)w;
+    a.bad = (int*)(w + n);
+    int bad = 1;
+    if (!hip_ok(hipMemsetAsync(a.bad, 0, sizeof(int), ctx().stream), "phase signs")) return nullptr;
+    hipLaunchKernelGGL(k_phase_signs, dim3(blocks_for(L.sizeh)), dim3(kBlock), 0, ctx().stream, a);
+    if (!hip_ok(hipGetLastError(), "k_phase_signs") ||
+        !hip_ok(hipMemcpyAsync(&bad, a.bad, sizeof(int), hipMemcpyDeviceToHost, ctx().stream), "phase signs") ||
+        !hip_ok(hipStreamSynchronize(ctx().stream), "phase signs"))
+        return nullptr;
+    return bad ? nullptr : a.sg;
+}
 
 // The two hops of a reliable update: temp = Doe x, then r_f = (float)(b - M x)
 // with the block partials of |r_f|^2.

@@ -15,7 +15,12 @@ template <> __host__ __device__ __forceinline__ float2 mkc<float2>(double a, dou
 // Re<x,out> reduction handed to finalizer `fin`.
 template <typename R>
 bool launch_dslash(int eo, int mode, int fin, const void* u, const void* ph, const void* in, void* out,
-                   const void* x, double m2, const SolverCtl& ctl);
+                   const void* x, double m2, const SolverCtl& ctl, const unsigned char* sg = nullptr);
+// The signs of the eight hops into each half-site where every phase is +-1:
+// sg[EO sizeh + i], for launch_dslash<double> in kPlain and kMdagMDot and the
+// hops of several systems; null where some phase is not, or without memory.
+// Valid until the next call.
+const unsigned char* phase_signs(const void* ph);
 // blocks of a launch_dslash launch (block b's partial at partials[2 b])
 template <typename R>
 int dslash_blocks();

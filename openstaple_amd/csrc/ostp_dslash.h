@@ -44,22 +44,33 @@ template <> __device__ __forceinline__ float2 mk<float2>(double a, double b) { r
 
 // One hop: o += U(iu) e^{+i th} in(iv)  (DAG=false, mat_vec_mul_arg)
 //          o -= U(iu)^dag e^{-i th} in(iv)  (DAG=true, conjmat_vec_mul_arg)
-template <typename R, bool DAG>
+// SGN: the phase is +-1 and given by neg instead of P (see phase_signs).
+template <typename C> __device__ __forceinline__ C sgn_if(C v, bool neg) {
+    return mk<C>(neg ? -v.x : v.x, neg ? -v.y : v.y);
+}
+template <typename R, bool DAG, bool SGN = false>
 __device__ __forceinline__ void hop(const typename Cplx<R>::T* __restrict__ U, const R* __restrict__ P,
                                     const typename Cplx<R>::T* __restrict__ in, int sizeh, int iu, int iv,
                                     typename Cplx<R>::T& o0, typename Cplx<R>::T& o1,
-                                    typename Cplx<R>::T& o2) {
+                                    typename Cplx<R>::T& o2, bool neg = false) {
     using C = typename Cplx<R>::T;
     const C a0 = ld_link(U + iu), a1 = ld_link(U + sizeh + iu), a2 = ld_link(U + 2 * sizeh + iu);
     const C b0 = ld_link(U + 3 * sizeh + iu), b1 = ld_link(U + 4 * sizeh + iu), b2 = ld_link(U + 5 * sizeh + iu);
-    const R arg = ld_link(P + iu);
+    R arg = 0;
+    if constexpr (!SGN) arg = ld_link(P + iu);
     C v0 = in[iv], v1 = in[sizeh + iv], v2 = in[2 * sizeh + iv];
-    R s, c;
-    sincos_t(arg, &s, &c);
-    const C phase = DAG ? mk<C>(c, -s) : mk<C>(c, s);
-    v0 = cmul(v0, phase);
-    v1 = cmul(v1, phase);
-    v2 = cmul(v2, phase);
+    if constexpr (SGN) {
+        v0 = sgn_if(v0, neg);
+        v1 = sgn_if(v1, neg);
+        v2 = sgn_if(v2, neg);
+    } else {
+        R s, c;
+        sincos_t(arg, &s, &c);
+        const C phase = DAG ? mk<C>(c, -s) : mk<C>(c, s);
+        v0 = cmul(v0, phase);
+        v1 = cmul(v1, phase);
+        v2 = cmul(v2, phase);
+    }
     // x = row0 x row1 ; row2 = conj(x)
     const C x0 = csub(cmul(a1, b2), cmul(a2, b1));
     const C x1 = csub(cmul(a2, b0), cmul(a0, b2));
@@ -90,11 +101,12 @@ struct SiteGeom {
 // out(idx) = 1/2 [ sum_mu U_mu(x) e^{i th} in(x+mu) - sum_mu U_mu(x-mu)^dag e^{-i th} in(x-mu) ]
 // for the output half-site idx of parity EO (0: Deo, even output; 1: Doe).
 // u[2*mu+parity], ph[2*mu+parity]: link planes and phases of the 8 arrays.
-template <typename R, int EO>
+// SGN: bits, the signs of the eight hops in the order of the code (phase_signs).
+template <typename R, int EO, bool SGN = false>
 __device__ __forceinline__ void dslash_site(const typename Cplx<R>::T* const* u, const R* const* ph,
                                             const typename Cplx<R>::T* __restrict__ in, const SiteGeom& a,
                                             int idx, typename Cplx<R>::T& o0, typename Cplx<R>::T& o1,
-                                            typename Cplx<R>::T& o2) {
+                                            typename Cplx<R>::T& o2, unsigned bits = 0) {
     using C = typename Cplx<R>::T;
     const int nd0h = a.nd0h, nd1 = a.nd1, nd2 = a.nd2, nd3 = a.nd3;
     int t = idx / nd0h;
@@ -119,14 +131,14 @@ __device__ __forceinline__ void dslash_site(const typename Cplx<R>::T* const* u,
     o0 = mk<C>(0, 0);
     o1 = mk<C>(0, 0);
     o2 = mk<C>(0, 0);
-    hop<R, true>(u[0 + B], ph[0 + B], in, a.sizeh, im0, im0, o0, o1, o2);
-    hop<R, true>(u[2 + B], ph[2 + B], in, a.sizeh, im1, im1, o0, o1, o2);
-    hop<R, true>(u[4 + B], ph[4 + B], in, a.sizeh, im2, im2, o0, o1, o2);
-    hop<R, true>(u[6 + B], ph[6 + B], in, a.sizeh, im3, im3, o0, o1, o2);
-    hop<R, false>(u[0 + F], ph[0 + F], in, a.sizeh, idx, ip0, o0, o1, o2);
-    hop<R, false>(u[2 + F], ph[2 + F], in, a.sizeh, idx, ip1, o0, o1, o2);
-    hop<R, false>(u[4 + F], ph[4 + F], in, a.sizeh, idx, ip2, o0, o1, o2);
-    hop<R, false>(u[6 + F], ph[6 + F], in, a.sizeh, idx, ip3, o0, o1, o2);
+    hop<R, true, SGN>(u[0 + B], ph[0 + B], in, a.sizeh, im0, im0, o0, o1, o2, bits & 1u);
+    hop<R, true, SGN>(u[2 + B], ph[2 + B], in, a.sizeh, im1, im1, o0, o1, o2, bits & 2u);
+    hop<R, true, SGN>(u[4 + B], ph[4 + B], in, a.sizeh, im2, im2, o0, o1, o2, bits & 4u);
+    hop<R, true, SGN>(u[6 + B], ph[6 + B], in, a.sizeh, im3, im3, o0, o1, o2, bits & 8u);
+    hop<R, false, SGN>(u[0 + F], ph[0 + F], in, a.sizeh, idx, ip0, o0, o1, o2, bits & 16u);
+    hop<R, false, SGN>(u[2 + F], ph[2 + F], in, a.sizeh, idx, ip1, o0, o1, o2, bits & 32u);
+    hop<R, false, SGN>(u[4 + F], ph[4 + F], in, a.sizeh, idx, ip2, o0, o1, o2, bits & 64u);
+    hop<R, false, SGN>(u[6 + F], ph[6 + F], in, a.sizeh, idx, ip3, o0, o1, o2, bits & 128u);
     const R half = (R)0.5;
     o0.x *= half; o0.y *= half; o1.x *= half; o1.y *= half; o2.x *= half; o2.y *= half;
 }
@@ -134,17 +146,19 @@ __device__ __forceinline__ void dslash_site(const typename Cplx<R>::T* const* u,
 // Hop of several right-hand sides on one gauge field: the link (two rows,
 // the rebuilt third, its phase) is loaded and prepared once and applied to
 // each active system's spinor with the arithmetic of hop<R, DAG>.
-template <typename R, bool DAG, int NR>
+template <typename R, bool DAG, int NR, bool SGN = false>
 __device__ __forceinline__ void hop_mr(const typename Cplx<R>::T* __restrict__ U, const R* __restrict__ P,
                                        const typename Cplx<R>::T* const (&in)[NR], const bool (&act)[NR], int sizeh,
-                                       int iu, int iv, typename Cplx<R>::T (&o)[NR][3]) {
+                                       int iu, int iv, typename Cplx<R>::T (&o)[NR][3], bool neg = false) {
     using C = typename Cplx<R>::T;
     const C a0 = ld_link(U + iu), a1 = ld_link(U + sizeh + iu), a2 = ld_link(U + 2 * sizeh + iu);
     const C b0 = ld_link(U + 3 * sizeh + iu), b1 = ld_link(U + 4 * sizeh + iu), b2 = ld_link(U + 5 * sizeh + iu);
-    const R arg = ld_link(P + iu);
-    R s, c;
-    sincos_t(arg, &s, &c);
-    const C phase = DAG ? mk<C>(c, -s) : mk<C>(c, s);
+    C phase;
+    if constexpr (!SGN) {
+        R s, c;
+        sincos_t(ld_link(P + iu), &s, &c);
+        phase = DAG ? mk<C>(c, -s) : mk<C>(c, s);
+    }
     const C x0 = csub(cmul(a1, b2), cmul(a2, b1));
     const C x1 = csub(cmul(a2, b0), cmul(a0, b2));
     const C x2 = csub(cmul(a0, b1), cmul(a1, b0));
@@ -152,7 +166,16 @@ __device__ __forceinline__ void hop_mr(const typename Cplx<R>::T* __restrict__ U
     for (int r = 0; r < NR; r++) {
         if (!act[r]) continue;
         const C* v = in[r];
-        const C v0 = cmul(v[iv], phase), v1 = cmul(v[sizeh + iv], phase), v2 = cmul(v[2 * sizeh + iv], phase);
+        C v0 = v[iv], v1 = v[sizeh + iv], v2 = v[2 * sizeh + iv];
+        if constexpr (SGN) {
+            v0 = sgn_if(v0, neg);
+            v1 = sgn_if(v1, neg);
+            v2 = sgn_if(v2, neg);
+        } else {
+            v0 = cmul(v0, phase);
+            v1 = cmul(v1, phase);
+            v2 = cmul(v2, phase);
+        }
         if (!DAG) {
             C r0 = cmul(a0, v0); r0 = cfma(a1, v1, r0); r0 = cfma(a2, v2, r0);
             C r1 = cmul(b0, v0); r1 = cfma(b1, v1, r1); r1 = cfma(b2, v2, r1);

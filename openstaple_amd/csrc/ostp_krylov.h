@@ -53,6 +53,7 @@ struct MsWin {
 struct KrArgs {
     const double2* u[8];
     const double* ph[8];
+    const unsigned char* sg;     // ordinary hops: signs of the hops, or null (phase_signs)
     SiteGeom g;
     const double2* r[kKrSys];    // residual after iteration j - 1
     double2* rn[kKrSys];         // k_kr_r: after iteration j (CG: the same array)

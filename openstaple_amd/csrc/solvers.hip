@@ -553,6 +553,9 @@ struct KrSys {
 // 24^3 x 6 (41472), even at 24^3 x 8 (55296), behind from 32^3 x 4 (65536) on.
 constexpr long kKrSplitSizeh = kHopSplitSizeh;
 
+// inside ker_invert_openacc_noalloc, which may not allocate (the signs of the hops)
+static bool g_no_alloc = false;
+
 static bool kr_split() { return ctx().lat.sizeh <= kKrSplitSizeh; }
 static int kr_blocks_hop() { return blocks_for(ctx().lat.sizeh, kr_split() ? kKrSites : kBlock); }
 static int kr_blocks_r() { return std::min(blocks_for(ctx().lat.sizeh), 1024); }
@@ -624,6 +627,7 @@ static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bo
     a.g.nd3 = L.nd[3];
     a.g.sizeh = (int)sizeh;
     a.tmajor = (sizeh / L.nd[3]) % (split ? kKrSites : kBlock) == 0;  // whole tiles per t-slice, as k_dslash
+    a.sg = split || g_no_alloc ? nullptr : phase_signs(ph);
     a.n = n;
     a.ms = ms ? 1 : 0;
     a.nA = nb;
@@ -1312,10 +1316,11 @@ struct MsMultiHop {
     SolverState* st[kMsMulti];
     double* part[kMsMulti];
     int n, pred, tmajor, rev;
+    const unsigned char* sg = nullptr;  // signs of the hops (SGN), both output parities
     SiteGeom g;
 };
 
-template <int EO, int NR>
+template <int EO, int NR, bool SGN>
 __global__ __launch_bounds__(kBlock) void k_ms_multi_hop(MsMultiHop a) {
     static_assert(NR <= kMsMulti, "systems per launch");
     bool act[NR];
@@ -1352,14 +1357,15 @@ __global__ __launch_bounds__(kBlock) void k_ms_multi_hop(MsMultiHop a) {
         for (int r = 0; r < NR; r++) o[r][0] = o[r][1] = o[r][2] = make_double2(0.0, 0.0);
         const Nbrs nb = site_neighbours<EO>(a.g, idx);
         constexpr int F = EO == 0 ? 0 : 1, B = 1 - F;
+        const unsigned bits = SGN ? a.sg[(long)EO * a.g.sizeh + idx] : 0u;
 #pragma unroll
         for (int mu = 0; mu < 4; mu++)
-            hop_mr<double, true, NR>(a.u[2 * mu + B], a.ph[2 * mu + B], in, act, a.g.sizeh, nb.im[mu],
-                                           nb.im[mu], o);
+            hop_mr<double, true, NR, SGN>(a.u[2 * mu + B], a.ph[2 * mu + B], in, act, a.g.sizeh, nb.im[mu],
+                                          nb.im[mu], o, bits >> mu & 1u);
 #pragma unroll
         for (int mu = 0; mu < 4; mu++)
-            hop_mr<double, false, NR>(a.u[2 * mu + F], a.ph[2 * mu + F], in, act, a.g.sizeh, idx, nb.ip[mu],
-                                            o);
+            hop_mr<double, false, NR, SGN>(a.u[2 * mu + F], a.ph[2 * mu + F], in, act, a.g.sizeh, idx, nb.ip[mu], o,
+                                           bits >> (4 + mu) & 1u);
         const long sh = a.g.sizeh;
 #pragma unroll
         for (int r = 0; r < NR; r++) {
@@ -1414,10 +1420,14 @@ __global__ __launch_bounds__(kBlock) void k_ms_multi_hop(MsMultiHop a) {
 // two systems (the common case: two flavours) with the two-system form
 template <int EO>
 static void launch_multi_hop(const MsMultiHop& a, int nbh) {
-    if (a.n <= 2)
-        hipLaunchKernelGGL((k_ms_multi_hop<EO, 2>), dim3(nbh), dim3(kBlock), 0, S(), a);
-    else
-        hipLaunchKernelGGL((k_ms_multi_hop<EO, kMsMulti>), dim3(nbh), dim3(kBlock), 0, S(), a);
+    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(nbh), dim3(kBlock), 0, S(), a); };
+    if (a.sg) {
+        if (a.n <= 2) go(k_ms_multi_hop<EO, 2, true>);
+        else go(k_ms_multi_hop<EO, kMsMulti, true>);
+    } else {
+        if (a.n <= 2) go(k_ms_multi_hop<EO, 2, false>);
+        else go(k_ms_multi_hop<EO, kMsMulti, false>);
+    }
 }
 
 static bool kr_plain_hops(const void* u, const void* ph, const KrArgs& a) {
@@ -1427,8 +1437,9 @@ static bool kr_plain_hops(const void* u, const void* ph, const KrArgs& a) {
         c.st = a.st[0] + (a.j & 1);
         c.partials = a.partA[0];
         c.pred = kIfRunning;
-        return launch_dslash<double>(1, kPlain, kFinStore, u, ph, a.p[0], a.h[0], nullptr, 0.0, c) &&
-               launch_dslash<double>(0, kMdagMDot, kFinNone, u, ph, a.h[0], a.s[0], a.p[0], a.m2[0], c);
+        return launch_dslash<double>(1, kPlain, kFinStore, u, ph, a.p[0], a.h[0], nullptr, 0.0, c, a.sg) &&
+               launch_dslash<double>(0, kMdagMDot, kFinNone, u, ph, a.h[0], a.s[0], a.p[0], a.m2[0], c,
+                                     a.sg);
     }
     MsMultiHop m;
     for (int l = 0; l < 8; l++) {
@@ -1436,6 +1447,7 @@ static bool kr_plain_hops(const void* u, const void* ph, const KrArgs& a) {
         m.ph[l] = a.ph[l];
     }
     m.g = a.g;
+    m.sg = a.sg;
     m.tmajor = a.tmajor;
     m.n = a.n;
     m.pred = kIfRunning;
@@ -1679,11 +1691,13 @@ struct ScratchSwap {
         ctx().partials = (double*)base;
         ctx().state = (SolverState*)((char*)base + kNoAllocPartialBytes);
         ctx().max_blocks = (int)((kNoAllocMaxSizeh + 63) / 64 + 64);
+        g_no_alloc = true;
     }
     ~ScratchSwap() {
         ctx().partials = partials;
         ctx().state = state;
         ctx().max_blocks = max_blocks;
+        g_no_alloc = false;
     }
 };
 

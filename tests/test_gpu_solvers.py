@@ -667,3 +667,27 @@ def test_multishift_window_orders(order, window):
         assert rel(got[1][2][k], got[0][2][k]) < 1e-12, k
         # the directions' terms cancel, by 1e3 to 1e4 at most over these iterations, times 64 roundings
         assert rel(got[1][3][k], got[0][3][k]) < 1e-10, k
+
+
+# above 49152 half-sites the solver's hops take phases that are +-1 as signs;
+# 1e-5 off is not +-1
+@pytest.mark.parametrize("phases", [dict(), dict(mu=1e-5), dict(bf=(0, 0, 1, 0, 0, 0), charge=1.0)])
+def test_solver_phases_of_large_lattices(phases):
+    """CG-M with one shift against the oracle: both residuals times the
+    condition number, far below what phases off by 1e-5 change."""
+    mass = 0.4
+    s = Sys((16, 16, 16, 26), seed=9, kind="cold", param=0.4, mass=mass)
+    ph = s.o.phases(**phases)
+    dph = Dev(ph)
+    fp = ost.ferm_param(mass, dph.p)
+    ra = remez19(mass)
+    ra.approx_order = 1
+    vb = s.b.nbytes
+    out, sf = Dev(nbytes=vb), Dev(nbytes=vb)
+    cg = C.c_int(0)
+    st = lib.multishift_invert(s.du.p, C.byref(fp), C.byref(ra), out.p, s.db.p, 1e-10, *(d.p for d in s.scratch),
+                               sf.p, 10000, C.byref(cg))
+    ost.check(0, "multishift_invert")
+    _, ocg, ox = s.o.multishift(s.u, ph, mass, [ra.RA_b[0]], s.b, 1e-10)
+    assert st == 1 and iters_close(cg.value, ocg), (cg.value, ocg)
+    assert rel(out.get(s.b), ox[0]) < 2e-10 * (1 + 64 / mass ** 2)
