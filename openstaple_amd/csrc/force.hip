@@ -258,12 +258,9 @@ struct Scratch {
     }
 };
 static Scratch g_hs, g_th, g_ta, g_conf_f, g_xs_all;
-
-// s has room for `need` bytes or a quarter of the free memory holds them
-static bool ample(const Scratch& s, size_t need) {
-    size_t free_b = 0, total_b = 0;
-    return need <= s.n || (hipMemGetInfo(&free_b, &total_b) == hipSuccess && need <= free_b / 4);
-}
+// D_oe of all sources' solutions and the stout levels' QA, kept through a force
+// where there is ample memory for them
+static Workspace g_hs_all, g_qa_all;
 
 // the rational solves of several sources on one operator, together (solvers.hip)
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
@@ -387,12 +384,8 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
     // room for all of them the chain forms them again)
     char* qa_all = nullptr;
     if (steps > 0) {
-        const unsigned long e0 = error_count();
-        if (ample(g_ta, steps * tb)) qa_all = (char*)g_ta.get(steps * tb);
-        if (!qa_all) {
-            (void)hipGetLastError();
-            forgive_errors(e0);
-        }
+        if (!g_th.get(tb)) return;  // the chain's own needs first
+        qa_all = (char*)g_qa_all.try_get(steps * tb);
         if (!launch_stout_levels(dconf, darr, steps, gl_stout_rho, qa_all)) return;
     }
     const void* conf_to_use = steps > 0 ? (const void*)(darr + (steps - 1) * gb) : dconf;
@@ -430,12 +423,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         // saves the force its hops (without ample room for those it forms them itself)
         const size_t all = (size_t)n * maxo * L.vec3_bytes();
         char* xs_all = n >= 2 ? (char*)g_xs_all.get(all) : nullptr;
-        char* hs_all = nullptr;
-        if (xs_all && ample(g_hs, all)) hs_all = (char*)g_hs.get(all);
-        if (xs_all && !hs_all) {
-            (void)hipGetLastError();
-            forgive_errors(e0);
-        }
+        char* hs_all = xs_all ? (char*)g_hs_all.try_get(all) : nullptr;
         if (n >= 2 && !xs_all) {
             (void)hipGetLastError();
             forgive_errors(e0);

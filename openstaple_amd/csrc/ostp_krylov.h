@@ -13,7 +13,7 @@
 //   k_kr_deo  stores p = r + gamma p at its own sites, s = m2 p - D_eo h, <p, s>
 //   k_kr_r    omega from <p, s>; r and (CG) x, |r|^2; the shifts' omegas, zetas
 // (the reference: OpenAcc/inverter_full.c:71-105, inverter_multishift_full.c:
-// 100-190; the expressions are those of finalize and finalize_ms_lanes).
+// 100-190; the per-shift expressions are those of finalize_ms_lanes).
 //
 // The hops of these kernels are split: a block takes 64 sites, one hop per
 // wave, so that a small lattice fills the compute units and a site does not
@@ -26,9 +26,10 @@
 // (state, partials, links, LDS: 3 to 5 us each), not by bytes, hence few
 // launches with every load issued before the first wait.  41 CG iterations on
 // 16^3 x 4: 1107 us with two hop kernels, two vector kernels and two one-block
-// finalizers an iteration, 804 us so; 19 shifts on 12x14x10x6, 52 iterations:
-// 1855 -> 1196 us; a force of two systems on 32^3 x 8: 8.87 -> 8.04 ms; 204
-// iterations on 32^4, bound by the links' bytes: 44.6 -> 43.7 ms.
+// finalizers an iteration, 804 us so and 740 to 780 with the streaming kernels'
+// sums over whole blocks; 52 CG-M iterations of order 9 on 12x14x10x6: 1855 ->
+// 1196 us; a force of two systems on 32^3 x 8: 8.87 -> 8.04 ms; 204 iterations
+// on 32^4, bound by the links' bytes: 44.6 -> 43.7 ms.
 #pragma once
 
 #include "ostp_dslash.h"
@@ -631,7 +632,8 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
 // kMxTailEvery-th iteration only: an update that falls between two of them
 // pauses the solver (hold) until the next.  79 iterations on 32^3 x 8: 4370
 // us with nine launches each, four of them for an update that seldom came, 3747
-// so (21 us an iteration in the FP32 hops, 10 in these two kernels).
+// so, 3630 to 3650 with sums over whole blocks (21 us an iteration in the FP32
+// hops, 10 in these two kernels).
 constexpr int kMxTailEvery = 2;
 struct MxArgs {
     float2 *pf, *rf, *outf;
