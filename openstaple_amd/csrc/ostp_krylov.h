@@ -634,6 +634,9 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
 // us with nine launches each, four of them for an update that seldom came, 3747
 // so, 3630 to 3650 with sums over whole blocks (21 us an iteration in the FP32
 // hops, 10 in these two kernels).
+// Every iteration, second, third, fourth: 3.72, 3.66, 3.62, 3.88 ms on 32^3 x 8,
+// 2.12, 1.68 to 1.98, 1.90, 2.06 on 16^3 x 8 (predicated launches that do nothing
+// against iterations that wait).
 constexpr int kMxTailEvery = 2;
 struct MxArgs {
     float2 *pf, *rf, *outf;
