@@ -116,10 +116,14 @@ __device__ __forceinline__ double kr_block(double v, double (&lds)[kBlock / 64])
 // `store`), *gamma and whether iteration j runs.  The window's coefficients
 // are advanced by the storing block (per-shift values through sh).  total: |r|^2
 // where the block has summed it already.
+//
+// The first launch of the next batch ends the iteration that a close has ended
+// once more, from the copy that the close read: a running system's step is left
+// to it.  A system that has finished takes its step in the close, which stores
+// the final state in both copies, so that the launch finds it finished.
 __device__ __forceinline__ void kr_end(const KrArgs& a, int k, int lane, bool store, double* gamma, int* running,
                                        double (*sh)[kMaxShifts], int* on, const double* total = nullptr) {
-    const SolverState* prev = a.st[k] + ((a.j - 1) & 1);
-    SolverState* next = a.st[k] + (a.j & 1);
+    SolverState* prev = a.st[k] + ((a.j - 1) & 1);
     // every load is issued before the first wait
     double sum = 0.0;
     if (a.j > 1 && !total) sum = kr_part(a.partB[k], a.nB, 1, lane);
@@ -166,49 +170,56 @@ __device__ __forceinline__ void kr_end(const KrArgs& a, int k, int lane, bool st
         *running = status == kRunning;
     }
     if (!store) return;
+    // the iteration that ended, its window step still to be taken by this block (or by the next launch,
+    // when this one only closes a batch of a solver that goes on)
+    const int ended = a.j > 1 && status0 == kRunning && !(a.close && status == kRunning);
     if (a.ms && lane < order) {
-        next->zeta_i[lane] = zi;
-        next->zeta_ii[lane] = zii;
-        next->zeta_iii[lane] = ziii;
-        next->gammas[lane] = gk;
-        next->omegas[lane] = om_k;
-        next->flags[0][lane] = f;
-        next->flags[1][lane] = moved;  // in the iteration that ended
-        next->shifts[lane] = prev->shifts[lane];
         sh[0][lane] = om_k;
         sh[1][lane] = gk;
         sh[2][lane] = ziii;
         on[lane] = moved;
     }
-    if (lane == 0) {
-        next->delta = delta;
-        next->lambda = lambda;
-        next->gammag = g;
-        next->alpha = prev->alpha;
-        next->omega = prev->omega;
-        next->omega_save = prev->omega_save;
-        next->source_norm = prev->source_norm;
-        next->res = prev->res;
-        next->safety = prev->safety;
-        next->cg = cg;
-        next->cg_restarted = restarted;
-        next->restart_every = prev->restart_every;
-        next->max_cg = prev->max_cg;
-        next->status = status;
-        next->order = order;
-        next->maxiter = maxiter;
-        // the iteration that ended, its window step still to be taken by this block (or by the next launch,
-        // when this one only closes a batch of a solver that goes on)
-        const int ended = a.j > 1 && status0 == kRunning && !(a.close && status == kRunning);
-        on[kMaxShifts] = ended;
-        next->hold = ended;
-    }
+    if (lane == 0) on[kMaxShifts] = ended;
+    auto put = [&](SolverState* next) {
+        if (a.ms && lane < order) {
+            next->zeta_i[lane] = zi;
+            next->zeta_ii[lane] = zii;
+            next->zeta_iii[lane] = ziii;
+            next->gammas[lane] = gk;
+            next->omegas[lane] = om_k;
+            next->flags[0][lane] = f;
+            next->flags[1][lane] = moved;  // in the iteration that ended
+            next->shifts[lane] = prev->shifts[lane];
+        }
+        if (lane == 0) {
+            next->delta = delta;
+            next->lambda = lambda;
+            next->gammag = g;
+            next->alpha = prev->alpha;
+            next->omega = prev->omega;
+            next->omega_save = prev->omega_save;
+            next->source_norm = prev->source_norm;
+            next->res = prev->res;
+            next->safety = prev->safety;
+            next->cg = cg;
+            next->cg_restarted = restarted;
+            next->restart_every = prev->restart_every;
+            next->max_cg = prev->max_cg;
+            next->status = status;
+            next->order = order;
+            next->maxiter = maxiter;
+            next->hold = ended;
+        }
+    };
+    put(a.st[k] + (a.j & 1));
+    if (a.close && status != kRunning) put(prev);
 }
 
 // window coefficients of the shifts that moved in iteration j - 1 (as k_msw_p)
 __device__ __forceinline__ void kr_window(MsWin* w, int order, const double (*sh)[kMaxShifts], const int* on, int tid,
                                           int nt) {
     const int t = w->t;
+    if (t >= kMsWinMax) return;  // the flushes come at W <= kMsWinMax: a row is never left
     const int per = t + 2;  // j < t, the new column t, and the scalar pair
     for (int e = tid; e < order * per; e += nt) {
         const int k = e / per, j = e - k * per;

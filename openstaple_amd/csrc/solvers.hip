@@ -224,9 +224,9 @@ template <typename CX, typename C, int G>
 __global__ __launch_bounds__(kBlock, 2) void k_msw_flush(CX* __restrict__ xs, C* __restrict__ ps,
                                                          const C* __restrict__ hist, const C* __restrict__ b,
                                                          long n3, int order, const MsWin* __restrict__ w,
-                                                         SolverCtl ctl, int full) {
+                                                         SolverCtl ctl, int W, int full) {
     if (!pred_pass(ctl)) return;
-    const int t = w->t;
+    const int t = min(w->t, W);  // hist holds W residuals
     if (t == 0 || t < full) return;  // full: only a window of that many iterations
     const bool first = w->first;
     const long i = (long)blockIdx.x * kBlock + threadIdx.x;
@@ -455,13 +455,13 @@ static SolverCtl ctl_of(int pred, int iter = 0) {
 
 static bool check_launch(const char* what) { return hip_ok(hipGetLastError(), what); }
 
-// apply a window (see k_msw_flush); b: the source, for a solve's first window
+// apply a window of at most W iterations (see k_msw_flush); b: the source, for a solve's first window
 template <typename CX, typename C>
 static void msw_flush(void* xs, void* ps, const void* hist, const void* b, long n3, int order, const MsWin* w,
-                      const SolverCtl& ctl, int full = 0) {
+                      const SolverCtl& ctl, int W, int full = 0) {
     auto go = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3(blocks_for(n3)), dim3(kBlock), 0, S(), (CX*)xs, (C*)ps, (const C*)hist,
-                           (const C*)b, n3, order, w, ctl, full);
+                           (const C*)b, n3, order, w, ctl, W, full);
     };
     if (order <= 10) go(k_msw_flush<CX, C, 10>);
     else go(k_msw_flush<CX, C, 20>);
@@ -610,6 +610,7 @@ static int kr_batch(int batch, double d, double* prev_d, int j, int* prev_j) {
 // return st_host[2 k] holds system k's last state.
 static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bool ms, int W, SolverState* st,
                        SolverState* st_host, double* part, size_t part_stride) {
+    if (W > kMsWinMax) return fail("solver window: %d iterations, at most %d", W, kMsWinMax);
     const Lattice& L = ctx().lat;
     const long sizeh = L.sizeh, n3 = 3 * sizeh;
     const size_t vb = L.vec3_bytes();
@@ -680,7 +681,7 @@ static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bo
                 for (int k = 0; k < n; k++) {
                     // the windows that iteration j - 1 filled
                     msw_flush<double2, double2>(sy[k].out, sy[k].shiftferm, sy[k].hist, sy[k].b, n3, sy[k].order,
-                                                sy[k].win, ctl_of(kAlways), W);
+                                                sy[k].win, ctl_of(kAlways), W, W);
                     msw_reset(sy[k].win, ctl_of(kAlways), W, false);
                 }
             if (split) {
@@ -1231,7 +1232,7 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
                                ctl_of(kIfIter, j), (C*)nullptr);
             if (j % W == 0) {
                 // only when iteration j ran: a window cut short is flushed once, at the end
-                msw_flush<C, C>(B.out, B.shiftferm, hist, B.b, n3, order, g_msw, ctl_of(kIfIter, j));
+                msw_flush<C, C>(B.out, B.shiftferm, hist, B.b, n3, order, g_msw, ctl_of(kIfIter, j), W);
                 msw_reset(g_msw, ctl_of(kIfIter, j), 0, false);
             }
             return check_launch("multishift iteration");
@@ -1242,7 +1243,7 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
     if (hist) {
         // the partial last window, and the final residual where the per-iteration
         // version leaves it
-        msw_flush<C, C>(B.out, B.shiftferm, hist, B.b, n3, order, g_msw, ctl_of(kAlways));
+        msw_flush<C, C>(B.out, B.shiftferm, hist, B.b, n3, order, g_msw, ctl_of(kAlways), W);
         if (cg > 0 && !hip_ok(hipMemcpyAsync(B.r, slot(cg), vb, hipMemcpyDeviceToDevice, S()), "final residual"))
             return INVERTER_FAILURE;
         if (!check_launch("multishift window flush")) return INVERTER_FAILURE;
@@ -1598,7 +1599,7 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
         MsSys& d = sy[k];
         const int cg = g_mm_st_host[2 * k].cg;
         d.cg = cg;
-        msw_flush<double2, double2>(d.out, d.shiftferm, hist(k), d.b, n3, d.order, g_mm_win + k, ctl_of(kAlways));
+        msw_flush<double2, double2>(d.out, d.shiftferm, hist(k), d.b, n3, d.order, g_mm_win + k, ctl_of(kAlways), W);
         if (cg > 0 && !hip_ok(hipMemcpyAsync(d.r, slot(k, cg), vb, hipMemcpyDeviceToDevice, S()), "final residual"))
             return false;
         if (!check_launch("multi multishift window flush")) return false;
@@ -2423,7 +2424,7 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
                            g_msw, ctl_of(kIfIter, j), hist + (size_t)((j - 1) % W) * n3);
         if (j % W == 0) {
             // only when iteration j ran: a window cut short is flushed once, at the end
-            msw_flush<double2, float2>(dout, pk, hist, nullptr, n3, order, g_msw, ctl_of(kIfIter, j));
+            msw_flush<double2, float2>(dout, pk, hist, nullptr, n3, order, g_msw, ctl_of(kIfIter, j), W);
             msw_reset(g_msw, ctl_of(kIfIter, j), 0, false);
         }
         return check_launch("mixed multishift iteration");
@@ -2432,7 +2433,7 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
     const int cg = H().cg;
     if (cg_multishift) *cg_multishift = cg;
     if (hist)
-        msw_flush<double2, float2>(dout, pk, hist, nullptr, n3, order, g_msw, ctl_of(kAlways));
+        msw_flush<double2, float2>(dout, pk, hist, nullptr, n3, order, g_msw, ctl_of(kAlways), W);
     hipLaunchKernelGGL(k_msx_flush, dim3(nb3), dim3(kBlock), 0, S(), fl, n3, ctl_of(kAlways));
     if (!check_launch("flush")) return 0;
     if (verbosity_lv > 1 && !hip_ok(hipStreamSynchronize(S()), "timing")) return 0;

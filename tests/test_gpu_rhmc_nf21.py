@@ -359,6 +359,51 @@ def test_systems_iterated_together_match_one_by_one(shape, ps):
     assert np.abs(forces[0]).max() > 1e-3 and np.array_equal(forces[0], forces[1]), rel(forces[0], forces[1])
 
 
+@pytest.mark.parametrize("shape, ps", [((4, 4, 4, 8), (1, 1)), ((16, 16, 16, 26), (1, 2))])
+@pytest.mark.parametrize("window", [0, 8, 16])
+def test_system_that_stops_where_a_batch_ends(shape, ps, window):
+    """The second flavour's mass is chosen so that it stops at every iteration
+    from 14 to 49 while the first goes on: before, at and after the end of the
+    first batch (16), of the one that follows (at most 48) and of windows of 8,
+    16 and 64 residuals.  The force is that of the one-by-one solves bit for
+    bit, in the iterations of those."""
+    F = Nf21(shape)
+    lat, vb = F.lat, F.lat.vec3_bytes
+    F.chi = Dev(nbytes=sum(ps) * vb)
+    for k in range(sum(ps)):
+        lib.ostp_generate_vec3_soa_gauss(F.chi.p + k * vb, 77, 10 + k)
+    for f in range(2):
+        F.fps[f].number_of_ps, F.fps[f].index_of_the_first_ps = ps[f], f * ps[0]
+    F.fps[0].ferm_mass = 0.02
+    du, ipd = Dev(F.u0), Dev(nbytes=F.tb)
+    count = C.c_int.in_dll(lib, "multishift_invert_iterations")
+
+    def force(batch, nflav=2):
+        old = lib.ostp_set_multishift_batching(batch), lib.ostp_set_multishift_window(window)
+        try:
+            before = count.value
+            lib.fermion_force_soloopenacc(du.p, F.arr.p, F.gl3.p, ipd.p, F.fps, nflav, F.chi.p, F.res, F.taux.p, F.xs.p,
+                                          F.ip(du.p), 50000)
+            ost.check(0, "fermion_force_soloopenacc")
+            return ipd.get(np.zeros(F.tb // 8)), count.value - before
+        finally:
+            lib.ostp_set_multishift_batching(old[0])
+            lib.ostp_set_multishift_window(old[1])
+
+    slow = force(0, 1)[1] // ps[0]
+    stops = {}
+    for mass in np.geomspace(4.5, 0.05, 800 if shape[0] == 4 else 100):
+        F.fps[1].ferm_mass = mass
+        f0, its0 = force(0)
+        stop = (its0 - slow * ps[0]) / ps[1]
+        if stop in stops or not 14 <= stop <= 49:
+            continue
+        f1, its1 = force(1)
+        stops[stop] = np.abs(f0).max() > 1e-3 and np.array_equal(f1, f0) and its1 == its0
+    assert slow > 60 and {16} | set(range(14, 50) if shape[0] == 4 else []) <= set(stops), (slow, sorted(stops))
+    assert all(stops.values()), [k for k, ok in stops.items() if not ok]
+
+
 def test_config5_trajectory_reversible_48x48x48x12():
     F = Nf21((48, 48, 48, 12), eps=0.5, seed=7, res=1e-10)
     moved, back_u, back_m = forward_back(F, 10, 5, 1.0, 2026)
