@@ -380,6 +380,16 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
     void* dtaux = resolve(taux_conf_acc, gb, nm);
     if (!dconf || (steps > 0 && !darr) || !dgl3 || !dip || !dtaux || !tfermion_parameters) return;
     hipStream_t s = ctx().stream;
+    // The kernels store the force and the flavours' sum without clearing them first; a call that fails on the
+    // way leaves no force of an earlier call behind: zero, and the sum of the flavours there are.
+    struct Unfinished {
+        void *ip, *gl3;  // still to be stored, or null
+        size_t ip_bytes, gl3_bytes;
+        ~Unfinished() {
+            if (ip) (void)hipMemsetAsync(ip, 0, ip_bytes, ctx().stream);
+            if (ip && gl3) (void)hipMemsetAsync(gl3, 0, gl3_bytes, ctx().stream);
+        }
+    } unfinished{dip, dgl3, tb, gb};
     // each level's QA is kept for the chain back through the levels (without ample
     // room for all of them the chain forms them again)
     char* qa_all = nullptr;
@@ -450,6 +460,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
                                                hs_all ? hs[k] : nullptr, ips == 0))
                         return;
                 if (!launch_backfield_times_force(dtaux, dgl3, dph, iflav == 0)) return;
+                unfinished.gl3 = nullptr;
             }
             // the shifted solutions of the last source stay in tferm_shiftmulti_acc, as after the loop below
             const int order = fps[n - 1]->approx_md.approx_order;
@@ -475,6 +486,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
             if (!compute_fermion_force(conf_to_use, dtaux, dxs, dph, &fp->approx_md, nullptr, ips == 0)) return;
         }
         if (!launch_backfield_times_force(dtaux, dgl3, dph, iflav == 0)) return;
+        unfinished.gl3 = nullptr;
     }
     if (steps > 0) {
         void* th = g_th.get(tb);
@@ -485,7 +497,9 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
                                     gl_stout_rho, stout_c_zero(), qa_all != nullptr))
                 return;
     }
-    if (launch_conf_times_force_ta(dconf, dgl3, dip, true)) hip_ok(hipStreamSynchronize(s), nm);
+    if (!launch_conf_times_force_ta(dconf, dgl3, dip, true)) return;
+    unfinished.ip = nullptr;
+    hip_ok(hipStreamSynchronize(s), nm);
 }
 
 }  // extern "C"

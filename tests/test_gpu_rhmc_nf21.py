@@ -359,6 +359,31 @@ def test_systems_iterated_together_match_one_by_one(shape, ps):
     assert np.abs(forces[0]).max() > 1e-3 and np.array_equal(forces[0], forces[1]), rel(forces[0], forces[1])
 
 
+@pytest.mark.parametrize("batch", [1, 0])
+@pytest.mark.parametrize("bad", [0, 1])
+def test_failed_force_leaves_no_old_force(batch, bad):
+    """A force that fails on the way (a flavour without phases, recorded as an
+    error) leaves a zero force, and the flavours' sum as far as it came."""
+    F = Nf21((4, 4, 4, 4))
+    du = Dev(F.u0)
+    F.ipd.put(np.ones(F.tb // 8))
+    F.gl3.put(np.ones(F.gb // 8))
+    F.fps[bad].phases = None
+    prev = lib.ostp_set_multishift_batching(batch)
+    lib.fermion_force_soloopenacc(du.p, F.arr.p, F.gl3.p, F.ipd.p, F.fps, 2, F.chi.p, F.res, F.taux.p, F.xs.p,
+                                  F.ip(du.p), 50000)
+    lib.ostp_set_multishift_batching(prev)
+    msg = lib.ostp_last_error()
+    lib.ostp_clear_error()
+    assert b"null pointer" in msg
+    assert not F.ipd.get(np.zeros(F.tb // 8)).any()
+    gl3 = F.gl3.get(np.zeros(F.gb // 8))
+    if batch or bad == 0:
+        assert not gl3.any()
+    else:
+        assert not (gl3 == 1.0).any() and np.abs(gl3).max() > 1e-3
+
+
 @pytest.mark.parametrize("shape, ps", [((4, 4, 4, 8), (1, 1)), ((16, 16, 16, 26), (1, 2))])
 @pytest.mark.parametrize("window", [0, 8, 16])
 def test_system_that_stops_where_a_batch_ends(shape, ps, window):
