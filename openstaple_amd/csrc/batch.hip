@@ -1222,7 +1222,7 @@ static int batched_solve(int nsys, const ostp_batch_system* sys, double res, int
         if (B.arena) (void)hipFree(B.arena);
         B.arena = nullptr;
         B.arena_bytes = 0;
-        if (!hip_ok(hipMalloc(&B.arena, arena), "batch arena")) return 0;
+        if (!hip_ok(device_malloc(&B.arena, arena), "batch arena")) return 0;
         B.arena_bytes = arena;
     }
     if ((size_t)nsys > B.st_cap) {
@@ -1236,11 +1236,11 @@ static int batched_solve(int nsys, const ostp_batch_system* sys, double res, int
         B.st_snap[0] = B.st_snap[1] = nullptr;
         B.dsys = nullptr;
         B.st_cap = 0;
-        if (!hip_ok(hipMalloc(&B.st, sizeof(SolverState) * nsys), "batch states") ||
+        if (!hip_ok(device_malloc(&B.st, sizeof(SolverState) * nsys), "batch states") ||
             !hip_ok(hipHostMalloc(&B.st_host, sizeof(SolverState) * nsys, hipHostMallocDefault), "batch states") ||
             !hip_ok(hipHostMalloc(&B.st_snap[0], sizeof(SolverState) * nsys, hipHostMallocDefault), "batch states") ||
             !hip_ok(hipHostMalloc(&B.st_snap[1], sizeof(SolverState) * nsys, hipHostMallocDefault), "batch states") ||
-            !hip_ok(hipMalloc(&B.dsys, sizeof(BSys) * nsys), "batch descriptors"))
+            !hip_ok(device_malloc(&B.dsys, sizeof(BSys) * nsys), "batch descriptors"))
             return 0;
         B.st_cap = nsys;
     }

@@ -327,7 +327,7 @@ int ostp_compute_nnp_and_nnm(int* nnp, int* nnm) {
     const Lattice& L = ctx().lat;
     const size_t bytes = (size_t)L.sizeh * 8 * sizeof(int);
     int *dp = nullptr, *dm = nullptr;
-    if (!hip_ok(hipMalloc(&dp, bytes), "nn alloc") || !hip_ok(hipMalloc(&dm, bytes), "nn alloc")) return 1;
+    if (!hip_ok(device_malloc(&dp, bytes), "nn alloc") || !hip_ok(device_malloc(&dm, bytes), "nn alloc")) return 1;
     const long vol = 2 * L.sizeh;
     hipLaunchKernelGGL(k_nn_tables, dim3(blocks_for(vol)), dim3(kBlock), 0, ctx().stream, dp, dm, geom_args());
     bool ok = hip_ok(hipGetLastError(), "k_nn_tables") && hip_ok(hipStreamSynchronize(ctx().stream), "sync") &&

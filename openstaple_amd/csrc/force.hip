@@ -252,7 +252,7 @@ struct Scratch {
         if (p) (void)hipFree(p);
         p = nullptr;
         n = 0;
-        if (!hip_ok(hipMalloc(&p, need), "force scratch")) return nullptr;
+        if (!hip_ok(device_malloc(&p, need), "force scratch")) return nullptr;
         n = need;
         return p;
     }
@@ -265,7 +265,7 @@ static Workspace g_hs_all, g_qa_all;
 // the rational solves of several sources on one operator, together (solvers.hip)
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
                           const void* const* in, void* const* out, int n, double res, int max_cg,
-                          int convergence_importance, void* const* hs);
+                          int convergence_importance, const WorkspacePart* hs);
 
 // sum over shifts of the outer products for one pseudofermion, to aux (fresh: of
 // any content) or added to it; hs: D_oe x_k
@@ -391,7 +391,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         }
     } unfinished{dip, dgl3, tb, gb};
     // each level's QA is kept for the chain back through the levels (without ample
-    // room for all of them the chain forms them again)
+    // room for all of them, or when the solves need it, the chain forms them again)
     char* qa_all = nullptr;
     if (steps > 0) {
         if (!g_th.get(tb)) return;  // the chain's own needs first
@@ -415,7 +415,8 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         std::vector<ferm_param*> fps;
         std::vector<const RationalApprox*> ras;
         std::vector<const void*> ins;
-        std::vector<void*> outs, hs;
+        std::vector<void*> outs;
+        std::vector<WorkspacePart> hs;
         int maxo = 1;
         for (int iflav = 0; iflav < tNDiffFlavs; iflav++) {
             ferm_param* fp = &tfermion_parameters[iflav];
@@ -430,10 +431,11 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
         }
         const int n = (int)fps.size();
         // the solutions of all sources, and D_oe of them from the solver's check, which
-        // saves the force its hops (without ample room for those it forms them itself)
+        // saves the force its hops (without ample room for those, or when the solves need
+        // it, the force forms them itself)
         const size_t all = (size_t)n * maxo * L.vec3_bytes();
         char* xs_all = n >= 2 ? (char*)g_xs_all.get(all) : nullptr;
-        char* hs_all = xs_all ? (char*)g_hs_all.try_get(all) : nullptr;
+        const bool keep_hs = xs_all && g_hs_all.try_get(all);
         if (n >= 2 && !xs_all) {
             (void)hipGetLastError();
             forgive_errors(e0);
@@ -442,10 +444,10 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
             for (int k = 0; k < n; k++) {
                 if (!ins[k]) return;
                 outs.push_back(xs_all + (size_t)k * maxo * L.vec3_bytes());
-                if (hs_all) hs.push_back(hs_all + (size_t)k * maxo * L.vec3_bytes());
+                if (keep_hs) hs.push_back(WorkspacePart{&g_hs_all, (size_t)k * maxo * L.vec3_bytes()});
             }
             together = multishift_fp64_many(conf_to_use, fps.data(), ras.data(), ins.data(), outs.data(), n, res,
-                                            max_cg, CONVERGENCE_NONCRITICAL, hs_all ? hs.data() : nullptr);
+                                            max_cg, CONVERGENCE_NONCRITICAL, keep_hs ? hs.data() : nullptr);
             if (!together && error_count() != e0) return;
         }
         if (together) {
@@ -457,7 +459,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
                 if (!dph) return;
                 for (int ips = 0; ips < fp->number_of_ps; ips++, k++)
                     if (!compute_fermion_force(conf_to_use, dtaux, outs[k], dph, &fp->approx_md,
-                                               hs_all ? hs[k] : nullptr, ips == 0))
+                                               keep_hs ? hs[k].p() : nullptr, ips == 0))
                         return;
                 if (!launch_backfield_times_force(dtaux, dgl3, dph, iflav == 0)) return;
                 unfinished.gl3 = nullptr;
@@ -490,6 +492,7 @@ void fermion_force_soloopenacc(su3_soa* tconf_acc, su3_soa* tstout_conf_acc_arr,
     }
     if (steps > 0) {
         void* th = g_th.get(tb);
+        if (qa_all) qa_all = (char*)g_qa_all.p;
         char* ta = qa_all ? qa_all : (char*)g_ta.get(tb);
         if (!th || !ta) return;
         for (int level = steps - 1; level >= 0; level--)

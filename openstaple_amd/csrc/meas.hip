@@ -213,7 +213,7 @@ int ostp_fermion_measures(const su3_soa* u, const su3_soa_f* u_f, ferm_param* pa
     const bool mag = pars->mag_re && pars->mag_im;
     enum { kRe, kRo, kXe, kXo, kPhi, kBe, kBo, kYe, kYo, kNv };
     char* buf = nullptr;
-    if (!hip_ok(hipMalloc(&buf, (size_t)kNv * vb * nvec), "measure vectors")) return 0;
+    if (!hip_ok(device_malloc(&buf, (size_t)kNv * vb * nvec), "measure vectors")) return 0;
     auto V = [&](int k, int j) { return (vec3_soa*)(buf + ((size_t)k * kNv + j) * vb); };
     int cg_total = 0, unconverged = 0;
     // (y_e, y_o) = M^-1 (x_e, x_o) for the vectors in ks (ferm_meas.c:50-71)

@@ -86,10 +86,11 @@ inline T* resolve_as(const void* p, size_t bytes, const char* what) {
 }
 
 // Device buffer of the library that lives from call to call and is given back
-// by ostp_finalize (release_workspaces) or when another allocation of the
-// library runs out of memory.  try_get grows it, and returns null without
-// recording an error where that would take more than a quarter of the free
-// memory: the caller then takes a path without it.
+// by ostp_finalize (release_workspaces) or when device_malloc runs out of
+// memory.  try_get grows it, and returns null without recording an error where
+// that would take more than a quarter of the free memory: the caller then takes
+// a path without it.  Whoever allocates between try_get and the workspace's use
+// reads p again (null: given back).
 struct Workspace {
     void* p = nullptr;
     size_t n = 0;
@@ -98,6 +99,21 @@ struct Workspace {
     void release();
 };
 void release_workspaces();
+size_t workspace_bytes();  // of all workspaces: what device_malloc can still take
+// a place in a workspace
+struct WorkspacePart {
+    Workspace* w = nullptr;
+    size_t at = 0;
+    void* p() const { return w && w->p ? (char*)w->p + at : nullptr; }
+};
+
+// hipMalloc for every other buffer, the library's and its callers': out of
+// memory, it takes back the workspaces and tries again.
+hipError_t device_malloc_bytes(void** p, size_t bytes);
+template <typename T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return device_malloc_bytes((void**)p, bytes);
+}
 
 // Launch geometry over sizeh half-sites.
 inline int blocks_for(long n, int nt = kBlock) { return (int)((n + nt - 1) / nt); }

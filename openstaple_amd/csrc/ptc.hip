@@ -439,7 +439,7 @@ static bool ptc_scratch() {
     if (g_ps.bytes < need) {
         if (g_ps.p) (void)hipFree(g_ps.p);
         g_ps = PtcScratch{};
-        if (!hip_ok(hipMalloc(&g_ps.p, need), "ptc scratch")) return false;
+        if (!hip_ok(device_malloc(&g_ps.p, need), "ptc scratch")) return false;
         g_ps.bytes = need;
     }
     char* c = (char*)g_ps.p;
@@ -668,7 +668,7 @@ int ostp_fcg_solve(const su3_soa* u, ferm_param* pars, const su3_soa_f* u_f, con
         if (work) (void)hipFree(work);
         work = nullptr;
         work_bytes = 0;
-        if (!hip_ok(hipMalloc(&work, 5 * vb), "fcg work")) return INVERTER_FAILURE;
+        if (!hip_ok(device_malloc(&work, 5 * vb), "fcg work")) return INVERTER_FAILURE;
         work_bytes = 5 * vb;
     }
     char* wv = (char*)work;
@@ -776,7 +776,7 @@ int ostp_fcg_mixed_solve(const su3_soa* u, ferm_param* pars, const su3_soa_f* u_
         if (work) (void)hipFree(work);
         work = nullptr;
         work_bytes = 0;
-        if (!hip_ok(hipMalloc(&work, need), "fcg work")) return INVERTER_FAILURE;
+        if (!hip_ok(device_malloc(&work, need), "fcg work")) return INVERTER_FAILURE;
         work_bytes = need;
     }
     char* wv = (char*)work;

@@ -57,7 +57,7 @@ namespace ostp {
 // and the recombination of a rational function's shifted solutions
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
                           const void* const* in, void* const* out, int n, double res, int max_cg,
-                          int convergence_importance, void* const* hs);
+                          int convergence_importance, const WorkspacePart* hs);
 bool recombine(const void* xs, const void* in, void* out, const RationalApprox* ra);
 bool find_max_eigenvalues_many(const void* u, ferm_param* const* pars, void* const* r, void* const* h,
                                void* const* p, int n, double* maxv);
@@ -94,7 +94,7 @@ struct DevScratch {
         if (p) (void)hipFree(p);
         p = nullptr;
         bytes = 0;
-        if (!hip_ok(hipMalloc(&p, need), "rhmc scratch")) return nullptr;
+        if (!hip_ok(device_malloc(&p, need), "rhmc scratch")) return nullptr;
         bytes = need;
         return p;
     }

@@ -165,8 +165,13 @@ void release_workspaces() {
     for (Workspace* w : workspaces()) w->release();
 }
 
-// hipMalloc for the callers' memory; the library's workspaces make room for it
-static hipError_t malloc_for_caller(void** p, size_t bytes) {
+size_t workspace_bytes() {
+    size_t n = 0;
+    for (const Workspace* w : workspaces()) n += w->n;
+    return n;
+}
+
+hipError_t device_malloc_bytes(void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipErrorOutOfMemory) {
         (void)hipGetLastError();
@@ -220,8 +225,8 @@ int ostp_init(int nd0, int nd1, int nd2, int nd3, int par_temp) {
     int blocks = blocks_for(L.sizeh, 64) + 64;
     if (!c.partials || blocks > c.max_blocks) {
         release_scratch();
-        if (!hip_ok(hipMalloc(&c.partials, sizeof(double) * 4 * (size_t)blocks), "hipMalloc partials")) return 1;
-        if (!hip_ok(hipMalloc(&c.state, 2 * sizeof(SolverState)), "hipMalloc state")) return 1;
+        if (!hip_ok(device_malloc(&c.partials, sizeof(double) * 4 * (size_t)blocks), "hipMalloc partials")) return 1;
+        if (!hip_ok(device_malloc(&c.state, 2 * sizeof(SolverState)), "hipMalloc state")) return 1;
         if (!hip_ok(hipHostMalloc(&c.state_host, 2 * sizeof(SolverState), hipHostMallocDefault), "hipHostMalloc"))
             return 1;
         c.max_blocks = blocks;
@@ -290,7 +295,7 @@ int ostp_acc_create(void* host, size_t bytes) {
     if (it != g_map.end() && it->first < a + bytes)
         return fail("ostp_acc_create: range overlaps a present region") ? 0 : 1;
     void* dev = nullptr;
-    hipError_t e = malloc_for_caller(&dev, bytes);
+    hipError_t e = device_malloc(&dev, bytes);
     if (e != hipSuccess) return hip_ok(e, "ostp_acc_create hipMalloc") ? 0 : 1;
     g_map[a] = Mapping{bytes, dev, 1};
     return 0;
@@ -356,7 +361,7 @@ int ostp_acc_is_present(const void* host, size_t bytes) {
 
 void* ostp_malloc(size_t bytes) {
     void* p = nullptr;
-    if (!hip_ok(malloc_for_caller(&p, bytes), "ostp_malloc")) return nullptr;
+    if (!hip_ok(device_malloc(&p, bytes), "ostp_malloc")) return nullptr;
     return p;
 }
 

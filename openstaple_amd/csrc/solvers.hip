@@ -1063,9 +1063,9 @@ bool launch_doe_multi(const void* u, const void* ph, const void* xs, void* hs, i
 }
 
 // |b - (M + shifts_k) x_k|^2 / sn for the FP64 solutions x_k = out + k * vb;
-// hs: D_oe x_k is left in hs + k * vb (null: not kept)
+// hs: D_oe x_k is left in hs + k * vb (where that has not been given back)
 static bool verify_shifts_f64(const void* u, const void* ph, const void* b, const void* out, int order, double m2,
-                              const double* shifts, double sn, double* g, void* hs) {
+                              const double* shifts, double sn, double* g, const WorkspacePart& hs) {
     const Lattice& L = ctx().lat;
     const long sizeh = L.sizeh;
     const size_t vb = L.vec3_bytes();
@@ -1075,7 +1075,7 @@ static bool verify_shifts_f64(const void* u, const void* ph, const void* b, cons
         if (g_ver_buf) (void)hipFree(g_ver_buf);
         g_ver_buf = nullptr;
         g_ver_bytes = 0;
-        if (!hip_ok(hipMalloc(&g_ver_buf, need), "multishift verification scratch")) return false;
+        if (!hip_ok(device_malloc(&g_ver_buf, need), "multishift verification scratch")) return false;
         g_ver_bytes = need;
     }
     VerArgs a = ver_args(u, ph);
@@ -1090,7 +1090,7 @@ static bool verify_shifts_f64(const void* u, const void* ph, const void* b, cons
             a.x[r] = (const double2*)((const char*)out + k * vb);
             a.m2[r] = m2 + shifts[k];
         }
-        if (hs) a.h = (double2*)((char*)hs + k0 * vb);
+        if (void* h = hs.p()) a.h = (double2*)((char*)h + k0 * vb);
         hipLaunchKernelGGL(k_ms_verify<1>, dim3(nb), dim3(kBlock), 0, S(), a);
         hipLaunchKernelGGL(k_ms_verify<0>, dim3(nb), dim3(kBlock), 0, S(), a);
         hipLaunchKernelGGL(k_ms_verify_sum, dim3(a.n), dim3(kBlock), 0, S(), (const double*)a.part, nb, sums + k0);
@@ -1108,7 +1108,7 @@ static bool verify_shifts_f64(const void* u, const void* ph, const void* b, cons
 struct MsBufs {
     const void *u, *ph, *b;
     void *out, *r, *h, *s, *p, *shiftferm;
-    void* hs = nullptr;          // where D_oe x_k is left (FP64; null: nowhere)
+    WorkspacePart hs;            // where D_oe x_k is left (FP64; null: nowhere)
 };
 
 static void* g_msw_hist = nullptr;
@@ -1116,8 +1116,9 @@ static size_t g_msw_hist_bytes = 0;
 static MsWin* g_msw = nullptr;
 static int g_msw_forced = 0;  // 0 automatic, 1 per-iteration updates, 2..64 fixed
 
-// window length: as many residuals as fit in a quarter of the free memory,
-// at most 64 (fewer than 8: per-iteration updates)
+// window length: as many residuals as fit in a quarter of the free memory (the
+// workspaces counted as free, device_malloc takes them back), at most 64 (fewer
+// than 8: per-iteration updates)
 static int msw_window(size_t vb) {
     if (g_msw_forced == 1) return 0;
     if (g_msw_forced >= 2) return g_msw_forced;
@@ -1126,7 +1127,7 @@ static int msw_window(size_t vb) {
         (void)hipGetLastError();
         free_b = 0;
     }
-    const size_t have = g_msw_hist_bytes + free_b / 4;
+    const size_t have = g_msw_hist_bytes + (free_b + workspace_bytes()) / 4;
     size_t w = vb ? have / vb : 0;
     if (w > (size_t)kMsWinMax) w = kMsWinMax;
     return w >= 8 ? (int)w : 0;
@@ -1189,11 +1190,11 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
             if (g_msw_hist) (void)hipFree(g_msw_hist);
             g_msw_hist = nullptr;
             g_msw_hist_bytes = 0;
-            if (!hip_ok(hipMalloc(&g_msw_hist, (size_t)W * vb), "multishift residual window")) return INVERTER_FAILURE;
+            if (!hip_ok(device_malloc(&g_msw_hist, (size_t)W * vb), "multishift residual window")) return INVERTER_FAILURE;
             g_msw_hist_bytes = (size_t)W * vb;
         }
         hist = (char*)g_msw_hist;
-        if (!g_msw && !hip_ok(hipMalloc(&g_msw, sizeof(MsWin)), "multishift window")) return INVERTER_FAILURE;
+        if (!g_msw && !hip_ok(device_malloc(&g_msw, sizeof(MsWin)), "multishift window")) return INVERTER_FAILURE;
         msw_reset(g_msw, ctl_of(kAlways), 0, true);
     }
     auto slot = [&](int j) { return (C*)(hist + (size_t)((j - 1) % W) * vb); };  // residual of iteration j (1-based)
@@ -1484,7 +1485,7 @@ struct MsSys {
     int max_cg;
     int cg = 0;          // out: CG-M iterations
     int status = INVERTER_FAILURE;
-    void* hs = nullptr;  // as MsBufs
+    WorkspacePart hs;    // as MsBufs
 };
 
 static SolverState* g_mm_st = nullptr;       // device states of the systems
@@ -1497,7 +1498,7 @@ static bool mm_partials() {
     if (g_mm_part) (void)hipFree(g_mm_part);
     g_mm_part = nullptr;
     g_mm_part_n = 0;
-    if (!hip_ok(hipMalloc(&g_mm_part, sizeof(double) * need * kMsMulti), "multi partials")) return false;
+    if (!hip_ok(device_malloc(&g_mm_part, sizeof(double) * need * kMsMulti), "multi partials")) return false;
     g_mm_part_n = need;
     return true;
 }
@@ -1520,10 +1521,10 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
     if (W < 2) return false;
     // device resources
     if (!g_mm_st) {
-        if (!hip_ok(hipMalloc(&g_mm_st, 2 * kMsMulti * sizeof(SolverState)), "multi states") ||
+        if (!hip_ok(device_malloc(&g_mm_st, 2 * kMsMulti * sizeof(SolverState)), "multi states") ||
             !hip_ok(hipHostMalloc(&g_mm_st_host, 2 * kMsMulti * sizeof(SolverState), hipHostMallocDefault),
                     "multi states") ||
-            !hip_ok(hipMalloc(&g_mm_win, kMsMulti * sizeof(MsWin)), "multi windows"))
+            !hip_ok(device_malloc(&g_mm_win, kMsMulti * sizeof(MsWin)), "multi windows"))
             return false;
     }
     if (!mm_partials()) return false;
@@ -1532,7 +1533,7 @@ static bool multishift_solve_multi(const void* u, const void* ph, MsSys* sy, int
         if (g_mm_hist) (void)hipFree(g_mm_hist);
         g_mm_hist = nullptr;
         g_mm_hist_bytes = 0;
-        if (hipMalloc(&g_mm_hist, (size_t)n * hb) != hipSuccess) {
+        if (device_malloc(&g_mm_hist, (size_t)n * hb) != hipSuccess) {
             (void)hipGetLastError();
             return false;
         }
@@ -1653,7 +1654,7 @@ static void* grow_buffer(void*& p, size_t& have, size_t need) {
     if (p) (void)hipFree(p);
     p = nullptr;
     have = 0;
-    if (!hip_ok(hipMalloc(&p, need), "scratch allocation")) return nullptr;
+    if (!hip_ok(device_malloc(&p, need), "scratch allocation")) return nullptr;
     have = need;
     return p;
 }
@@ -1714,10 +1715,10 @@ static bool power_method_multi(const void* u, const void* ph, const double* coef
     const int nbh = blocks_for(sizeh);
     if (n < 1 || n > kMsMulti) return false;
     if (!g_mm_st) {
-        if (!hip_ok(hipMalloc(&g_mm_st, 2 * kMsMulti * sizeof(SolverState)), "multi states") ||
+        if (!hip_ok(device_malloc(&g_mm_st, 2 * kMsMulti * sizeof(SolverState)), "multi states") ||
             !hip_ok(hipHostMalloc(&g_mm_st_host, 2 * kMsMulti * sizeof(SolverState), hipHostMallocDefault),
                     "multi states") ||
-            !hip_ok(hipMalloc(&g_mm_win, kMsMulti * sizeof(MsWin)), "multi windows"))
+            !hip_ok(device_malloc(&g_mm_win, kMsMulti * sizeof(MsWin)), "multi windows"))
             return false;
     }
     if (!mm_partials()) return false;
@@ -1823,7 +1824,7 @@ static int* g_differ_flag = nullptr;
 static bool same_phases(const void* a, const void* b) {
     if (a == b) return true;
     const long n = 8 * ctx().lat.sizeh;
-    if (!g_differ_flag && !hip_ok(hipMalloc(&g_differ_flag, sizeof(int)), "phase comparison")) return false;
+    if (!g_differ_flag && !hip_ok(device_malloc(&g_differ_flag, sizeof(int)), "phase comparison")) return false;
     int h = 0;
     if (!hip_ok(hipMemsetAsync(g_differ_flag, 0, sizeof(int), S()), "phase comparison")) return false;
     hipLaunchKernelGGL(k_differ, dim3(blocks_for(n)), dim3(kBlock), 0, S(), (const unsigned long long*)a,
@@ -1847,10 +1848,10 @@ static int g_ms_many = 1;  // rational solves of several sources together where 
 // apply (another precision mode, the single-precision accelerated path,
 // fewer than two sources, different phases, or no memory for it).  hs (or
 // null): D_oe of the solutions, as the per-shift check forms it, is left there
-// in the solutions' layout.
+// in the solutions' layout (unless the memory has been needed for the solves).
 bool multishift_fp64_many(const void* u, ferm_param* const* pars, const RationalApprox* const* ras,
                           const void* const* in, void* const* out, int n, double res, int max_cg,
-                          int convergence_importance, void* const* hs) {
+                          int convergence_importance, const WorkspacePart* hs) {
     if (!g_ms_many || n < 2 || g_ms_precision != 0 || inverter_tricks.singlePInvAccelMultiInv) return false;
     const unsigned long e0 = error_count();
     const Lattice& L = ctx().lat;
@@ -1882,7 +1883,7 @@ bool multishift_fp64_many(const void* u, ferm_param* const* pars, const Rational
             MsSys& d = sy[r];
             d.b = in[k0 + r];
             d.out = out[k0 + r];
-            d.hs = hs ? hs[k0 + r] : nullptr;
+            if (hs) d.hs = hs[k0 + r];
             d.r = base;
             d.h = base + vb;
             d.s = base + 2 * vb;
@@ -2120,7 +2121,7 @@ int ostp_chiral_condensate(const su3_soa* u, const su3_soa_f* u_f, ferm_param* p
     const size_t vb = L.vec3_bytes();
     // per vector: eta_e, eta_o, phi (source, then temporary), x_e, x_o
     char* buf = nullptr;
-    if (!hip_ok(hipMalloc(&buf, 5 * vb * (size_t)nvec), "chiral condensate vectors")) return 0;
+    if (!hip_ok(device_malloc(&buf, 5 * vb * (size_t)nvec), "chiral condensate vectors")) return 0;
     auto vec = [&](int k, int j) { return (vec3_soa*)(buf + ((size_t)k * 5 + j) * vb); };
     const double m = pars->ferm_mass;
     std::vector<ostp_batch_system> sys(nvec);
@@ -2388,11 +2389,11 @@ int ostp_multishift_mixed_solve(inverter_package ip, ferm_param* pars, RationalA
             if (g_msw_hist) (void)hipFree(g_msw_hist);
             g_msw_hist = nullptr;
             g_msw_hist_bytes = 0;
-            if (!hip_ok(hipMalloc(&g_msw_hist, (size_t)W * vbf), "multishift residual window")) return 0;
+            if (!hip_ok(device_malloc(&g_msw_hist, (size_t)W * vbf), "multishift residual window")) return 0;
             g_msw_hist_bytes = (size_t)W * vbf;
         }
         hist = (float2*)g_msw_hist;
-        if (!g_msw && !hip_ok(hipMalloc(&g_msw, sizeof(MsWin)), "multishift window")) return 0;
+        if (!g_msw && !hip_ok(device_malloc(&g_msw, sizeof(MsWin)), "multishift window")) return 0;
         msw_reset(g_msw, ctl_of(kAlways), 0, false);
     }
     // Reliable updates are taken at every kMsxRuEvery-th iteration (when the

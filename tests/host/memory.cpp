@@ -1,0 +1,164 @@
+// Calls of the library on the fake device of fake_device.cpp: what they do
+// when memory runs out.  Prints one line
+// per check, "name : ok" or what went wrong.
+#include "ostp_krylov.h"
+
+#include <string>
+
+using namespace ostp;
+
+extern "C" {
+extern size_t fake_capacity, fake_used;
+int fake_is_live(const void* p);
+void on_launch(const char* kernel, void** args);
+}
+
+namespace {
+std::string gone;            // kernels that were given memory that is no longer there
+int with_qa, with_hops;      // launches that took a kept QA; that formed D_oe of solutions
+
+void* arg(void** args, int i) {
+    void* p;
+    memcpy(&p, args[i], sizeof p);
+    return p;
+}
+void used(const char* kernel, const void* p) {
+    if (!fake_is_live(p)) gone += std::string(" ") + kernel;
+}
+}  // namespace
+
+extern "C" void on_launch(const char* kernel, void** args) {
+    const std::string k = kernel;
+    auto is = [&](const char* s) { return k.find(s) != std::string::npos; };
+    if (is("k_kr_doe") || is("k_kr_p")) {
+        const KrArgs& a = *(const KrArgs*)args[0];
+        for (int q = 0; q < a.n; q++) {
+            used("k_kr", a.p[q]);
+            if (a.win[q]) used("k_kr_win", a.rn[q] ? a.rn[q] : a.r[q]);
+            if (!a.close) continue;
+            for (int c = 0; c < 2; c++) {
+                a.st[q][c].status = kDone;
+                a.st[q][c].cg = 1;
+            }
+        }
+    } else if (is("k_finalize")) {
+        ((const SolverCtl*)args[0])->st->sum = 1.0;
+    } else if (is("k_direct_product_sites")) {  // aux, stride, xs, hs
+        used("k_direct_product", arg(args, 0));
+        used("k_direct_product", arg(args, 2));
+        used("k_direct_product", arg(args, 3));
+    } else if (is("k_qa_lambda")) {  // links, S', stride, QA, Lambda
+        used("k_qa_lambda", arg(args, 3));
+        used("k_qa_lambda", arg(args, 4));
+        with_qa += is("ILb1E") ? 1 : 0;
+    } else if (is("k_sigma")) {
+        used("k_sigma", arg(args, 1));
+        used("k_sigma", arg(args, 2));
+    } else if (is("k_gf_tile")) {
+        used("k_gf_tile", arg(args, 0));
+        used("k_gf_tile", arg(args, 4));
+    } else if (is("k_ms_verifyILi1E")) {
+        // u[8], ph[8], x[8], m2[8], n, h
+        const char* v = (const char*)args[0];
+        void* h;
+        memcpy(&h, v + 32 * 8 + 8, sizeof h);
+        used("k_ms_verify", h);
+        with_hops++;
+    }
+}
+
+namespace {
+
+constexpr int kShape[4] = {8, 8, 8, 8};
+constexpr size_t kSh = 2048, kGauge = 8 * 144 * kSh, kVec = 48 * kSh, kIp = 8 * 64 * kSh;
+constexpr int kOrder = 4;
+
+struct Fields {
+    char *u, *arr, *gl3, *ip, *taux, *mom, *chi, *xs, *sf, *ph;
+    vec3_soa* w[4];
+    ferm_param fp[2] = {};
+    Fields() {
+        ostp_set_abort_on_error(0);
+        ostp_init(kShape[0], kShape[1], kShape[2], kShape[3], 0);
+        ostp_set_stout(0.15, 2, 0.0, 0, 0, 1);
+        auto get = [](size_t n) { return (char*)ostp_malloc(n); };
+        u = get(kGauge), arr = get(2 * kGauge), gl3 = get(kGauge), taux = get(kGauge);
+        ip = get(kIp), mom = get(kIp), chi = get(2 * kVec), xs = get(kOrder * kVec), sf = get(kOrder * kVec);
+        ph = get(64 * kSh);
+        for (auto& p : w) p = (vec3_soa*)get(kVec);
+        for (int f = 0; f < 2; f++) {
+            fp[f].ferm_mass = 0.1 + f;
+            fp[f].number_of_ps = 1;
+            fp[f].index_of_the_first_ps = f;
+            fp[f].phases = (double_soa*)ph;
+            fp[f].approx_md.approx_order = kOrder;
+            for (int k = 0; k < kOrder; k++) fp[f].approx_md.RA_b[k] = 0.1 * (k + 1);
+        }
+    }
+    void gauge_force() {
+        ostp_time_gauge_force((su3_soa*)u, nullptr, (tamat_soa*)ip, (thmat_soa*)mom, 0.1, 1);
+    }
+    void force() {
+        inverter_package p = {};
+        p.u = (su3_soa*)u;
+        p.ferm_shift_temp = (vec3_soa*)sf;
+        p.nshifts = kOrder;
+        p.loc_r = w[0], p.loc_h = w[1], p.loc_s = w[2], p.loc_p = w[3];
+        fermion_force_soloopenacc((su3_soa*)u, (su3_soa*)arr, (su3_soa*)gl3, (tamat_soa*)ip, fp, 2, (vec3_soa*)chi, 1e-9,
+                                  (su3_soa*)taux, (vec3_soa*)xs, p, 100);
+    }
+    int multishift() {
+        int cg = 0;
+        return multishift_invert((su3_soa*)u, &fp[0], &fp[0].approx_md, (vec3_soa*)xs, (vec3_soa*)chi, 1e-9, w[0], w[1],
+                                 w[2], w[3], (vec3_soa*)sf, 100, &cg);
+    }
+};
+
+// what went wrong since the last call, or "ok"
+const char* verdict() {
+    static std::string s;
+    s = ostp_last_error();
+    if (s.empty()) s = gone.empty() ? "ok" : "gone:" + gone;
+    ostp_clear_error();
+    gone.clear();
+    return s.c_str();
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::string what = argv[1];
+    Fields f;
+    const size_t base = fake_used;
+    if (what == "given_back") {
+        // The gauge force's work space first; the memory that is left beside it is too little for the call.
+        f.gauge_force();
+        const size_t held = fake_used - base;
+        printf("work space : %s\n", held == 288 * 8 * kSh ? "ok" : "none");
+        auto tight = [&](const char* name, auto call) {
+            f.gauge_force();  // holds its work space again
+            fake_capacity = fake_used + 64;
+            call();
+            fake_capacity = (size_t)1 << 40;
+            printf("%s : %s\n", name, verdict());
+        };
+        tight("caller", [&] { ostp_free(ostp_malloc(held / 2)); });
+        tight("tables", [&] {
+            std::vector<int> a(8 * kSh), b(8 * kSh);
+            ostp_compute_nnp_and_nnm(a.data(), b.data());
+        });
+        ostp_set_multishift_window(16);
+        tight("window", [&] { f.multishift(); });
+        ostp_set_multishift_window(0);
+        tight("again", [&] { f.gauge_force(); });
+    } else if (what == "force") {
+        // A gauge force, then a fermion force, in the memory given: the bytes it took, whether the levels' QA and
+        // the solutions' D_oe were kept to the end, and whether all went well.
+        fake_capacity = base + strtoull(argv[2], nullptr, 0);
+        ostp_set_multishift_window(8);
+        if (argc > 3) f.gauge_force();
+        f.force();
+        printf("force %zu %d %d : %s\n", fake_used - base, with_qa == 2, with_hops == 2, verdict());
+    }
+    return 0;
+}
