@@ -1153,6 +1153,14 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
         if (!hip_ok(hipMemcpyAsync((char*)B.shiftferm + k * vb, B.b, vb, hipMemcpyDeviceToDevice, S()), "p_k = b"))
             return INVERTER_FAILURE;
     }
+    // a solve that fails before its windows are applied leaves no solutions of an earlier one: zero
+    struct Unfinished {
+        void* x;
+        size_t bytes;
+        ~Unfinished() {
+            if (x && bytes) (void)hipMemsetAsync(x, 0, bytes, S());
+        }
+    } unfinished{W < 2 ? nullptr : B.out, order * vb};
     if (!hip_ok(hipMemcpyAsync(B.r, B.b, vb, hipMemcpyDeviceToDevice, S()), "r = b") ||
         !hip_ok(hipMemcpyAsync(B.p, B.b, vb, hipMemcpyDeviceToDevice, S()), "p = b"))
         return INVERTER_FAILURE;
@@ -1249,6 +1257,7 @@ int multishift_solve(const MsBufs& B, double mass, int order, const double* shif
             return INVERTER_FAILURE;
         if (!check_launch("multishift window flush")) return INVERTER_FAILURE;
     }
+    unfinished.x = nullptr;
     multishift_invert_iterations += cg;
     if (cg == max_cg) printf("WARNING: maximum number of iterations reached in invert\n");
 

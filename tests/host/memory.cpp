@@ -1,5 +1,5 @@
 // Calls of the library on the fake device of fake_device.cpp: what they do
-// when memory runs out.  Prints one line
+// when memory runs out, and what a solve that fails leaves.  Prints one line
 // per check, "name : ok" or what went wrong.
 #include "ostp_krylov.h"
 
@@ -14,6 +14,7 @@ void on_launch(const char* kernel, void** args);
 }
 
 namespace {
+bool solves_end = true;
 std::string gone;            // kernels that were given memory that is no longer there
 int with_qa, with_hops;      // launches that took a kept QA; that formed D_oe of solutions
 
@@ -35,8 +36,8 @@ extern "C" void on_launch(const char* kernel, void** args) {
         for (int q = 0; q < a.n; q++) {
             used("k_kr", a.p[q]);
             if (a.win[q]) used("k_kr_win", a.rn[q] ? a.rn[q] : a.r[q]);
-            if (!a.close) continue;
-            for (int c = 0; c < 2; c++) {
+            if (!solves_end) a.st[q][a.j & 1] = a.st[q][(a.j - 1) & 1];
+            for (int c = 0; c < 2 && a.close && solves_end; c++) {
                 a.st[q][c].status = kDone;
                 a.st[q][c].cg = 1;
             }
@@ -159,6 +160,17 @@ int main(int argc, char** argv) {
         if (argc > 3) f.gauge_force();
         f.force();
         printf("force %zu %d %d : %s\n", fake_used - base, with_qa == 2, with_hops == 2, verdict());
+    } else if (what == "failed_solve") {
+        solves_end = false;  // the state does not advance: an error
+        for (int w : {0, 1}) {
+            ostp_set_multishift_window(w);
+            ostp_memset(f.xs, 1, kOrder * kVec);
+            const int st = f.multishift();
+            bool zero = st == 0 && *ostp_last_error();
+            ostp_clear_error();
+            for (size_t i = 0; i < kOrder * kVec; i++) zero = zero && !f.xs[i];
+            printf("window %d : %s\n", w, zero ? "ok" : "old solutions");
+        }
     }
     return 0;
 }

@@ -1,6 +1,6 @@
-"""What the library does when device memory runs out, on the CPU: its entry
-points with a stand-in for the device of a set capacity, on which kernels do
-not run (tests/host/fake_device.cpp)."""
+"""What the library does when device memory runs out, and what a failed solve
+leaves, on the CPU: its entry points with a stand-in for the device of a set
+capacity, on which kernels do not run (tests/host/fake_device.cpp)."""
 import os
 import subprocess
 
@@ -56,3 +56,9 @@ def test_force_in_little_memory(run, after_gauge_force):
         assert v == "ok", (room - least, k, v)
         kept.add(tuple(k.split()[2:]))
     assert ("0", "0") in kept and ("1", "1") in kept, kept
+
+
+def test_failed_multishift_leaves_no_old_solutions(run):
+    """A solve that fails (its state does not advance) leaves zero solutions,
+    with windows of residuals and with per-iteration updates."""
+    assert run("failed_solve") == {"window 0": "ok", "window 1": "ok"}
