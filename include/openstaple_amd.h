@@ -591,8 +591,9 @@ double ostp_time_gauge_force(const su3_soa *u, su3_soa *stap, tamat_soa *ipdot, 
                              int reps);
 /* No reference counterpart: which kernels form the gauge force: 1 (default)
  * tiles of the lattice's planes with their links in LDS, where every extent
- * is even and the work space (288 B per link) takes no more than a quarter of
- * the free memory; 0 the per-link kernel.  Returns the previous setting. */
+ * is even and the work space's two buffers (96 B per link for the links, 192 B
+ * for the force's parts) each take no more than a quarter of the memory that is
+ * then free; 0 the per-link kernel.  Returns the previous setting. */
 int ostp_set_gauge_force_kernel(int planes);
 /* No reference counterpart: the kernel that accumulates the fermion force's
  * outer products (ker_openacc_compute_fermion_force,

@@ -1752,7 +1752,9 @@ bool gf_planes_ready() {
     // 24-bit products of a coordinate and its stride
     if ((long)L.nd[0] * L.nd[1] * L.nd[2] >= (1L << 24) || L.nd[3] >= (1 << 24)) return false;
     const size_t links = (size_t)8 * L.sizeh;
-    return g_gf_rec.try_get(96 * links) && g_gf_part.try_get(3 * 64 * links);
+    if (g_gf_rec.try_get(96 * links) && g_gf_part.try_get(3 * 64 * links)) return true;
+    g_gf_rec.release();  // one without the other is of no use
+    return false;
 }
 static dim3 gf_grid8() { return dim3(blocks_for(ctx().lat.sizeh), 8); }
 

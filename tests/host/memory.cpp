@@ -152,6 +152,16 @@ int main(int argc, char** argv) {
         tight("window", [&] { f.multishift(); });
         ostp_set_multishift_window(0);
         tight("again", [&] { f.gauge_force(); });
+    } else if (what == "refused") {
+        // Free memory of four times the links' records and a little less than four times the force's parts on
+        // top: the parts are refused, the per-link kernel takes the call, and nothing stays allocated.
+        const size_t rec = 96 * 8 * kSh, part = 2 * rec;
+        fake_capacity = fake_used + rec + 4 * part - 64;
+        f.gauge_force();
+        printf("refused : %s\n", fake_used == base ? verdict() : "kept");
+        fake_capacity += 64;
+        f.gauge_force();
+        printf("taken : %s\n", fake_used == base + rec + part ? verdict() : "not kept");
     } else if (what == "force") {
         // A gauge force, then a fermion force, in the memory given: the bytes it took, whether the levels' QA and
         // the solutions' D_oe were kept to the end, and whether all went well.

@@ -39,6 +39,12 @@ def test_work_space_is_given_back(run):
     assert not {k: v for k, v in got.items() if v != "ok"}
 
 
+def test_gauge_work_space_is_taken_whole(run):
+    """Where there is room for the first of the gauge force's two buffers only,
+    it is not kept; with room for both, both are."""
+    assert run("refused") == {"refused": "ok", "taken": "ok"}
+
+
 @pytest.mark.parametrize("after_gauge_force", [0, 1])
 def test_force_in_little_memory(run, after_gauge_force):
     """The fermion force keeps the stout levels' QA and D_oe of the solutions
