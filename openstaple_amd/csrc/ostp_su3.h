@@ -23,6 +23,9 @@ struct Thmat {
     double rc00, rc11;
 };
 
+// byte offset of 16-B entry e of link record h (96 B: rows 0,1) in its array; 32 bits do while 96 sizeh < 2^32
+__device__ __forceinline__ unsigned link_record(int h, int e) { return (unsigned)h * 96u + (unsigned)e * 16u; }
+
 __device__ __forceinline__ double2 cmul_nc(double2 a, double2 b) {
 #pragma clang fp contract(off)
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);

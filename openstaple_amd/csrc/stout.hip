@@ -868,9 +868,8 @@ __global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ 
             for (int k = 0; k < kGfFetch; k++) {
                 int arr, h;
                 link_at(t, li[k], arr, h);
-                // 32-bit offset within the link array (96 sizeh < 2^32)
                 const ostp_dvec2* R = (const ostp_dvec2*)((const char*)rec + (size_t)((unsigned)arr) * rec_stride +
-                                                          (unsigned)(h * 96 + lpart * 16));
+                                                          link_record(h, lpart));
                 pre[2 * k] = R[0];
                 pre[2 * k + 1] = R[1];
                 if (PT) prek[k] = ((const double*)(G.at(arr) + (size_t)9 * g.sizeh))[h];

@@ -3,11 +3,13 @@ the Dslash neighbour formula (k_dslash in openstaple_amd/csrc/dslash.hip) must
 reproduce the oracle's neighbour tables and stay in [0, sizeh), and the
 XCD-aware workgroup remap must be a bijection of [0, G)."""
 import itertools
+import subprocess
 
 import numpy as np
 import pytest
 
 from oracle import Oracle
+from test_krylov_host import build_host
 
 
 def kernel_neighbours(nd, eo):
@@ -184,3 +186,21 @@ def test_gauge_force_tile_arrays():
             for i, j, (r, o, p) in itertools.product((0, tm - 1), (0, tn - 1), reads):
                 inside(r, i + (p if d else o), j + (o if d else p))
     assert tiles > 100
+
+
+def test_link_record_offsets(tmp_path):
+    """link_record (ostp_su3.h) over the largest array that the gauge force's
+    tiles take (96 sizeh just below 2^32), with arithmetic overflow trapped."""
+    src = tmp_path / "rec.cpp"
+    src.write_text(r"""
+#include "ostp_su3.h"
+int main() {
+    const int last = (int)(((1LL << 32) - 1) / 96) - 1;
+    for (long long h : {0LL, 1LL, 22369621LL, 22369622LL, (long long)last})
+        for (int e = 0; e < 6; e++)
+            if (ostp::link_record((int)h, e) != h * 96 + e * 16) return 1;
+    return 0;
+}
+""")
+    build_host(src, tmp_path / "rec", "-fsanitize=signed-integer-overflow", "-fno-sanitize-recover=all")
+    subprocess.run([str(tmp_path / "rec")], check=True)
