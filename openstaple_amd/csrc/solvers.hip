@@ -579,6 +579,14 @@ static void kr_split_hop(bool doe, const KrArgs& a, int nb) {
 // both hops of iteration a.j by the ordinary kernels
 static bool kr_plain_hops(const void* u, const void* ph, const KrArgs& a);
 
+// Iterations of the first batch, for which no convergence rate is known.  Those
+// queued past the end still read their vectors before they see that the solver
+// has stopped: 25 us each on 32^4, where a CG of five iterations takes 1.58 ms
+// with 8 and 1.85 with 16 (seven: 1.92, 2.18; with 4 1.53, 1.94), and one of 40
+// 8.67 and 8.59.  A batch's end costs 15 us, which small lattices feel more: 16
+// there (five iterations on 16^3 x 8: 0.29 ms).
+static int kr_first_batch() { return kr_split() ? 16 : 8; }
+
 // ln(residual / target) of a state the loop left (NaN when unknown)
 static double kr_dist(const SolverState& s, bool ms) {
     double m = s.delta;
@@ -660,7 +668,7 @@ static bool kr_iterate(const void* u, const void* ph, const KrSys* sy, int n, bo
             hipLaunchKernelGGL(k_kr_p, dim3(a.close ? 1 : nr, n), dim3(kBlock), 0, S(), a);
         }
     };
-    int j = 0, batch = 16;
+    int j = 0, batch = kr_first_batch();
     double prev_d = NAN;
     for (int k = 0; k < n; k++) {
         const double d = kr_dist(st_host[2 * k], ms);
@@ -881,7 +889,7 @@ int mixed_solve(const MxBufs& B, double mass, double shift, double res, int max_
     a.partA = a.partB + a.nB;
     a.partT = a.partA + 2 * a.nA;
     a.sizeh = (int)sizeh;
-    int j = 0, batch = 16, prev_j = 0, last_cg = -1;
+    int j = 0, batch = kr_first_batch(), prev_j = 0, last_cg = -1;
     double prev_d = kr_dist(H(), false);
     for (;;) {
         for (int i = 0; i < batch; i++) {

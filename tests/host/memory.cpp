@@ -15,6 +15,7 @@ void on_launch(const char* kernel, void** args);
 
 namespace {
 bool solves_end = true;
+int stop, iterations;        // (not 0) a CG converges in that many; launched
 std::string gone;            // kernels that were given memory that is no longer there
 int with_qa, with_hops;      // launches that took a kept QA; that formed D_oe of solutions
 
@@ -36,6 +37,18 @@ extern "C" void on_launch(const char* kernel, void** args) {
         for (int q = 0; q < a.n; q++) {
             used("k_kr", a.p[q]);
             if (a.win[q]) used("k_kr_win", a.rn[q] ? a.rn[q] : a.r[q]);
+            if (stop) {
+                const SolverState& prev = a.st[q][(a.j - 1) & 1];
+                SolverState next = prev;
+                if (prev.status == kRunning && a.j > 1) {
+                    next.cg = a.j - 1;
+                    next.delta = next.lambda = prev.source_norm * pow(prev.res * prev.safety, 2.0 * next.cg / stop);
+                    if (next.cg >= stop) next.status = kInnerExit;
+                }
+                a.st[q][a.j & 1] = next;
+                iterations += !a.close;
+                continue;
+            }
             if (!solves_end) a.st[q][a.j & 1] = a.st[q][(a.j - 1) & 1];
             for (int c = 0; c < 2 && a.close && solves_end; c++) {
                 a.st[q][c].status = kDone;
@@ -180,6 +193,22 @@ int main(int argc, char** argv) {
             ostp_clear_error();
             for (size_t i = 0; i < kOrder * kVec; i++) zero = zero && !f.xs[i];
             printf("window %d : %s\n", w, zero ? "ok" : "old solutions");
+        }
+    } else if (what == "short") {
+        // CG solves that take few iterations: how many were queued
+        ostp_init(16, 16, 16, 2 * strtol(argv[2], nullptr, 0), 0);  // half-sites: 4096 each
+        const size_t sh = ostp_sizeh();
+        char* big[7];
+        for (auto& p : big) p = (char*)ostp_malloc(48 * sh);
+        const su3_soa* u = (su3_soa*)ostp_malloc(8 * 144 * sh);
+        ferm_param fp = f.fp[0];
+        fp.phases = (double_soa*)ostp_malloc(64 * sh);
+        for (stop = 1; stop <= 12; stop++) {
+            int cg = 0;
+            iterations = 0;
+            auto v = [&](int k) { return (vec3_soa*)big[k]; };
+            ker_invert_openacc(u, &fp, v(0), v(1), 1e-9, v(2), v(3), v(4), v(5), 100, 0.0, &cg);
+            printf("%d %d : %d\n", stop, iterations, cg);
         }
     }
     return 0;

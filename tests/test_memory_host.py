@@ -68,3 +68,17 @@ def test_failed_multishift_leaves_no_old_solutions(run):
     """A solve that fails (its state does not advance) leaves zero solutions,
     with windows of residuals and with per-iteration updates."""
     assert run("failed_solve") == {"window 0": "ok", "window 1": "ok"}
+
+
+@pytest.mark.parametrize("tens,first", [(12, 16), (13, 8)])  # 49152 half-sites, 53248
+def test_short_solves_queue_few_iterations(run, tens, first):
+    """A CG that takes 1 to 12 iterations: the first batch is shorter on large
+    lattices, where an iteration queued in vain costs more than a batch's end;
+    those that follow come from the rate of convergence, with a margin of a
+    tenth and one iteration."""
+    got = run("short", tens)
+    assert len(got) == 12
+    for k, v in got.items():
+        stop, queued = map(int, k.split())
+        assert int(v) == stop
+        assert queued <= (first if stop <= first else stop + 4), (stop, queued)
