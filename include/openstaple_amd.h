@@ -589,11 +589,13 @@ double calc_rettangolo_soloopenacc(const su3_soa *tconf_acc, su3_soa *local_plaq
  * mom_sum_mult(mom, ipdot, fact) when mom is not null), averaged over reps */
 double ostp_time_gauge_force(const su3_soa *u, su3_soa *stap, tamat_soa *ipdot, thmat_soa *mom, double fact,
                              int reps);
-/* No reference counterpart: which kernels form the gauge force: 1 (default)
- * tiles of the lattice's planes with their links in LDS, where every extent
- * is even and the work space's two buffers (96 B per link for the links, 192 B
- * for the force's parts) each take no more than a quarter of the memory that is
- * then free; 0 the per-link kernel.  Returns the previous setting. */
+/* No reference counterpart: which kernels form the gauge force where its
+ * staples are not asked for: 0 the per-link kernel; 2 tiles of the lattice's
+ * planes with their links in LDS, for the action with rectangles, where every
+ * extent is even and the work space's two buffers (96 B per link for the links,
+ * 192 B for the force's parts) each take no more than a quarter of the memory
+ * that is then free; 1 (default) those where they are faster.  Returns the
+ * previous setting. */
 int ostp_set_gauge_force_kernel(int planes);
 /* No reference counterpart: the kernel that accumulates the fermion force's
  * outer products (ker_openacc_compute_fermion_force,

@@ -131,10 +131,10 @@ bool launch_invert_momenta(void* mom) {
 }
 
 // the plane kernels of the gauge force (stout.hip)
-bool gf_planes_ready();
+bool gf_planes_ready(bool moves);
 bool gf_pack(const void* u);
 bool gf_unpack(void* u);
-bool gf_parts(const void* u, void* stap);
+bool gf_parts(const void* u);
 bool gf_ipdot(void* ipdot, void* mom, double fact);
 bool gf_move(void* mom, double fact, double delta);
 
@@ -144,10 +144,10 @@ bool gf_move(void* mom, double fact, double delta);
 // and the last force; the momentum step and the link update are one kernel.
 bool md_gauge(void* u, void* stap, void* ipdot, void* mom) {
     const int gs = md_parameters.gauge_scale;
-    const bool planes = gf_planes_ready();
+    const bool planes = gf_planes_ready(true);
     if (planes && !gf_pack(u)) return false;
     auto bloc = [&](int idx) {
-        if (planes) return gf_parts(u, nullptr) && gf_move(mom, deltas_Omelyan[idx], deltas_Omelyan[4]);
+        if (planes) return gf_parts(u) && gf_move(mom, deltas_Omelyan[idx], deltas_Omelyan[4]);
         return launch_gauge_force(u, nullptr, ipdot, mom, deltas_Omelyan[idx]) &&
                launch_mom_exp(u, mom, deltas_Omelyan[4]);
     };
@@ -155,8 +155,9 @@ bool md_gauge(void* u, void* stap, void* ipdot, void* mom) {
     for (int md = 1; md < gs; md++)
         if (!bloc(5) || !bloc(6)) return false;
     if (!bloc(5)) return false;
-    // the last force also leaves its staples, as calc_ipdot_gauge_soloopenacc does
-    if (planes) return gf_unpack(u) && gf_parts(u, stap) && gf_ipdot(ipdot, mom, deltas_Omelyan[3]);
+    // the last force also leaves its staples, as calc_ipdot_gauge_soloopenacc does (the per-link kernel)
+    if (planes && !gf_unpack(u)) return false;
+    if (planes && !stap) return gf_parts(u) && gf_ipdot(ipdot, mom, deltas_Omelyan[3]);
     return launch_gauge_force(u, stap, ipdot, mom, deltas_Omelyan[3]);
 }
 

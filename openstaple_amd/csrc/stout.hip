@@ -585,10 +585,11 @@ __global__ __launch_bounds__(3 * kGfLinks, 2) void k_gauge_force(GaugePtrs G, do
     }
 }
 
-// Gauge force by planes.  TA(U S) is linear, so every plane (mu, nu) forms
-// its own part TA(U S_plane) of its two directions' links, in a buffer of
-// its own (three planes per direction), and the kernels that consume the
-// force add the three parts.
+// Gauge force by planes, for the action with rectangles (gf_planes_pay says
+// where).  TA(U S) is linear, so every plane (mu, nu) forms its own part
+// TA(U S_plane) of its two directions' links, in a buffer of its own (three
+// planes per direction), and the kernels that consume the force add the three
+// parts.
 //
 // A block takes tm x tn tiles (at most 64 sites, one lane each) of a plane at
 // fixed coordinates along the other two directions.  Within a tile every
@@ -715,9 +716,7 @@ __device__ __forceinline__ GfArr uni(const GfArr& a) {
 // c02, c12, (ic00, ic11)) at part[((slot 8 + link array) sizeh + site) 4].
 template <bool PT>
 __global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ rec, GaugePtrs G,
-                                                    double2* __restrict__ stap, size_t su3_stride,
-                                                    double2* __restrict__ part, LinkGeom g, GfPlans plans, int p0,
-                                                    int p1, int tlsm, double c0) {
+                                                    double2* __restrict__ part, LinkGeom g, GfPlans plans, double c0) {
     __shared__ double2 pool[6 * kGfPool];
     __shared__ double lk[PT ? kGfPoolLinks : 1];
     const int tid = (int)threadIdx.x, lane = tid & 63;
@@ -732,11 +731,10 @@ __global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ 
     auto share = [](int tiles, int x) { return (tiles >> 3) * x + ((tiles & 7) * x >> 3); };
     int total = 0;
 #pragma unroll
-    for (int p = 0; p < 6; p++)
-        if (p >= p0 && p < p1) total += share(plans.tiles[p], xcd + 1) - share(plans.tiles[p], xcd);
+    for (int p = 0; p < 6; p++) total += share(plans.tiles[p], xcd + 1) - share(plans.tiles[p], xcd);
     const int each = total / nbx, rest = total - each * nbx;
     int q = each * bx + min(bx, rest), left = each + (bx < rest ? 1 : 0);
-    for (int p = p0; p < p1 && left > 0; p++) {
+    for (int p = 0; p < 6 && left > 0; p++) {
         const GfPlan& pl = plans.p[p];
         const int tiles = uni(pl.tiles), base = share(tiles, xcd), count = share(tiles, xcd + 1) - base;
         if (q >= count) {
@@ -902,26 +900,24 @@ __global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ 
                 tn = advance(t);
                 fetch(tn);
             }
-            if (tlsm) {
 #pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    const int s = item(k);
-                    if (s < np) {
-                        Su3 A, C;
-                        gf_load2(pool + sA[k], A);
-                        gf_load(pool + sC[k], C);
-                        mul_dag_r2(A, C, A);
-                        gf_store2(pool + sO[k], A);
-                    } else if (s >= p64 && s < ns) {
-                        Su3 A, C, X;
-                        gf_load(pool + sA[k], A);
-                        gf_load(pool + sC[k], C);
-                        dag_mul_r2(C, A, X);
-                        gf_store2(pool + sO[k], X);
-                    }
+            for (int k = 0; k < 2; k++) {
+                const int s = item(k);
+                if (s < np) {
+                    Su3 A, C;
+                    gf_load2(pool + sA[k], A);
+                    gf_load(pool + sC[k], C);
+                    mul_dag_r2(A, C, A);
+                    gf_store2(pool + sO[k], A);
+                } else if (s >= p64 && s < ns) {
+                    Su3 A, C, X;
+                    gf_load(pool + sA[k], A);
+                    gf_load(pool + sC[k], C);
+                    dag_mul_r2(C, A, X);
+                    gf_store2(pool + sO[k], X);
                 }
-                __syncthreads();
             }
+            __syncthreads();
             // one side of one direction's links per wave
             const bool live = inside && t.om + im < ndm && t.on + jn < ndn;
             auto pick = [&](const GfArr& a, const GfArr& b) {  // dsel ? b : a, in scalar registers
@@ -945,56 +941,44 @@ __global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ 
                 if (side == 0) {
                     const double ka = kP(1, 0), kc = kP(0, 0) * kO(0, 1);
                     ld(aP, 1, 0, A);
-                    if (tlsm) {
-                        Su3 X, W;
-                        ld2(aSO, 0, 1, X);
-                        ld(aP, 0, 0, B);
-                        mul_dag_r2(X, B, X);
-                        rebuild3row(X);
-                        su3_scale(kCOne * ka * kP(1, 1) * kO(0, 2) * kP(0, 1) * kP(0, 0), X, W);
-                        ld(aO, 0, 1, B);
-                        Su3 Y;
-                        ld(aSPm, 0, 0, Y);
-                        dag_mul_r2(B, Y, X);
-                        rebuild3row(X);
-                        axpy3(kCOne * ka * kO(0, 1) * kP(-1, 0) * kO(-1, 1) * kO(-1, 0), X, W);
-                        su3_mul(A, W, T);
-                        su3_scale(c0 * ka * kc, A, A);
-                        ld(aSPp, 1, 0, B);
-                        axpy3_dag(kCOne * kc * kO(1, 1) * kP(2, 0) * kO(1, 0), B, A);
-                        ld(aC, 0, 0, B);
-                        su3_mul_dag_add(A, B, T);
-                    } else {
-                        ld(aC, 0, 0, B);
-                        su3_scale(c0 * ka * kc, A, A);
-                        su3_mul_dag(A, B, T);
-                    }
+                    Su3 X, W;
+                    ld2(aSO, 0, 1, X);
+                    ld(aP, 0, 0, B);
+                    mul_dag_r2(X, B, X);
+                    rebuild3row(X);
+                    su3_scale(kCOne * ka * kP(1, 1) * kO(0, 2) * kP(0, 1) * kP(0, 0), X, W);
+                    ld(aO, 0, 1, B);
+                    Su3 Y;
+                    ld(aSPm, 0, 0, Y);
+                    dag_mul_r2(B, Y, X);
+                    rebuild3row(X);
+                    axpy3(kCOne * ka * kO(0, 1) * kP(-1, 0) * kO(-1, 1) * kO(-1, 0), X, W);
+                    su3_mul(A, W, T);
+                    su3_scale(c0 * ka * kc, A, A);
+                    ld(aSPp, 1, 0, B);
+                    axpy3_dag(kCOne * kc * kO(1, 1) * kP(2, 0) * kO(1, 0), B, A);
+                    ld(aC, 0, 0, B);
+                    su3_mul_dag_add(A, B, T);
                 } else {
                     const double kn = kP(0, -1), kc = kO(0, -1) * kP(1, -1);
                     ld(aP, 0, -1, A);
-                    if (tlsm) {
-                        Su3 X, Y, W;
-                        ld(aP, 1, -1, B);
-                        ld(aSO, 0, -1, Y);
-                        dag_mul_r2(B, Y, X);
-                        rebuild3row(X);
-                        su3_scale(kCOne * kn * kP(1, -1) * kP(1, -2) * kO(0, -2) * kP(0, -2), X, W);
-                        ld2(aSPp, 1, -1, X);
-                        ld(aO, 0, -1, B);
-                        mul_dag_r2(X, B, X);
-                        rebuild3row(X);
-                        axpy3(kCOne * kn * kO(0, -1) * kO(1, 0) * kP(2, -1) * kO(1, -1), X, W);
-                        su3_mul(W, A, T);
-                        su3_scale(c0 * kc * kn, A, A);
-                        ld(aSPm, 0, -1, B);
-                        axpy3_dag(kCOne * kc * kP(-1, -1) * kO(-1, 0) * kO(-1, -1), B, A);
-                        ld(aC, 0, -1, B);
-                        su3_dag_mul_add(B, A, T);
-                    } else {
-                        ld(aC, 0, -1, B);
-                        su3_scale(c0 * kc * kn, A, A);
-                        su3_dag_mul(B, A, T);
-                    }
+                    Su3 X, Y, W;
+                    ld(aP, 1, -1, B);
+                    ld(aSO, 0, -1, Y);
+                    dag_mul_r2(B, Y, X);
+                    rebuild3row(X);
+                    su3_scale(kCOne * kn * kP(1, -1) * kP(1, -2) * kO(0, -2) * kP(0, -2), X, W);
+                    ld2(aSPp, 1, -1, X);
+                    ld(aO, 0, -1, B);
+                    mul_dag_r2(X, B, X);
+                    rebuild3row(X);
+                    axpy3(kCOne * kn * kO(0, -1) * kO(1, 0) * kP(2, -1) * kO(1, -1), X, W);
+                    su3_mul(W, A, T);
+                    su3_scale(c0 * kc * kn, A, A);
+                    ld(aSPm, 0, -1, B);
+                    axpy3_dag(kCOne * kc * kP(-1, -1) * kO(-1, 0) * kO(-1, -1), B, A);
+                    ld(aC, 0, -1, B);
+                    su3_dag_mul_add(B, A, T);
                 }
             }
             // the lower sides' sums go to the upper sides' threads through the pool past the links
@@ -1027,19 +1011,6 @@ __global__ __launch_bounds__(256, 2) void k_gf_tile(const double2* __restrict__ 
                 o[kGfPool] = f.c02;
                 o[2 * kGfPool] = f.c12;
                 o[3 * kGfPool] = make_double2(f.ic00, f.ic11);
-                if (stap) {
-                    // staples times K(x, d), summed over the planes (calc_ipdot_gauge_soloopenacc's output)
-                    int arr, h;
-                    site(im, jn, dsel, arr, h);
-                    const bool first = gf_slot(dsel ? nu : mu, dsel ? mu : nu) == 0;
-                    double2* O = (double2*)((char*)stap + (size_t)arr * su3_stride) + h;
-#pragma unroll
-                    for (int e = 0; e < 9; e++) {
-                        double2 v = make_double2(ku * T.c[e / 3][e % 3].x, ku * T.c[e / 3][e % 3].y);
-                        if (!first) v = cadd(v, O[(size_t)e * g.sizeh]);
-                        O[(size_t)e * g.sizeh] = v;
-                    }
-                }
             }
             __syncthreads();
             // four lanes write one link's 64-B record
@@ -1654,7 +1625,7 @@ bool launch_sigma_chain(void* sigma, void* lam, void* qa, const void* u, double 
     return hip_ok(hipGetLastError(), "k_sigma");
 }
 
-static int g_gf_planes = 1;  // the plane kernel (0: the per-link kernel)
+static int g_gf_planes = 1;  // the plane kernel where it is faster (2: wherever it can; 0: the per-link kernel)
 
 // the LDS arrays of a tm x tn tile; false when they exceed the pool
 static bool gf_plan(int tm, int tn, GfPlan& p) {
@@ -1741,15 +1712,32 @@ static const GfPlans& gf_plans() {
 // lane offsets within a link array are 32-bit in the per-link kernel (up to 6 planes of 16 sizeh bytes)
 static bool gf_size_ok() { return (size_t)96 * ctx().lat.sizeh < ((size_t)1 << 32); }
 
+// Whether the plane kernel is the faster one; moves: for the integrator, whose links stay in records between the
+// forces.  Only for the action with rectangles, whose staples share products (per force on 24^4: tiles 591 us, links
+// 782; Wilson 417, 261), and not where the staples are asked for (their sums over the planes took a launch a plane:
+// 1161 us, 840 by links).  The tiles come 512 at a time, two blocks per CU, the per-link kernel a block per CU for
+// every 2048 half-sites, at 6 to 10 us a round, so few sites a tile (extents of 2) or a last round that is nearly
+// empty decide: steps of the integrator, links against tiles, 16^3 x 4 (2 rounds of tiles, 4 of links) 51 -> 41 us, 12^3 x 4
+// (2, 2) 30.2 -> 27.8, 10^3 x 8 (3, 2) 30.6 -> 32.5 with defect coefficients, 16^3 x 2 (3, 2) 28.9 -> 29.4,
+// 64 x 64 x 2 x 2 (13, 4) 51 -> 82.  A force by itself also packs the records: 12x18x4x14 (6048) 33.6 -> 36.7,
+// 18x10x12x6 (6480) 43.5 -> 36.7, 16^4 166 -> 112.
+static bool gf_planes_pay(bool moves) {
+    const long sizeh = ctx().lat.sizeh;
+    long tiles = 0;
+    for (const GfPlan& q : gf_plans().p) tiles += q.tiles;
+    return (tiles + 511) / 512 <= (sizeh + 2047) / 2048 && (moves || sizeh > 6144);
+}
+
 // the plane kernel's buffers, or false: the per-link kernel then (its halo wraps at most once along a direction)
-bool gf_planes_ready() {
+bool gf_planes_ready(bool moves) {
     const Lattice& L = ctx().lat;
-    if (!g_gf_planes || !gf_size_ok()) return false;
+    if (!g_gf_planes || !gf_size_ok() || !g_tlsm) return false;
     // even extents: a wrap keeps the site's parity
     for (int k = 0; k < 4; k++)
         if (L.nd[k] < 2 || (L.nd[k] & 1)) return false;
     // 24-bit products of a coordinate and its stride
     if ((long)L.nd[0] * L.nd[1] * L.nd[2] >= (1L << 24) || L.nd[3] >= (1 << 24)) return false;
+    if (g_gf_planes == 1 && !gf_planes_pay(moves)) return false;
     const size_t links = (size_t)8 * L.sizeh;
     if (g_gf_rec.try_get(96 * links) && g_gf_part.try_get(3 * 64 * links)) return true;
     g_gf_rec.release();  // one without the other is of no use
@@ -1768,25 +1756,19 @@ bool gf_unpack(void* u) {
     return hip_ok(hipGetLastError(), "k_gf_unpack");
 }
 
-// the planes' force parts of the records' links (K planes from u); with stap, the staples as well
-bool gf_parts(const void* u, void* stap) {
-    const Lattice& L = ctx().lat;
+// the planes' force parts of the records' links (K planes from u): the planes are independent, one launch, two
+// blocks per CU (and at least a block for each XCD's share of the tiles)
+bool gf_parts(const void* u) {
     const GfPlans& plans = gf_plans();
-    // The planes are independent unless the staples are summed: one launch, two blocks per CU (and at least
-    // a block for each XCD's share of the tiles).
-    const int step = stap ? 1 : 6;
-    for (int p = 0; p < 6; p += step) {
-        long tiles = 0;
-        for (int k = p; k < p + step; k++) tiles += plans.p[k].tiles;
-        const unsigned nb = (unsigned)std::max(8L, std::min(tiles, 512L));
-        auto go = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, ctx().stream, (const double2*)g_gf_rec.p, gauge_ptrs(u),
-                               (double2*)stap, L.su3_bytes(), (double2*)g_gf_part.p, link_geom(), plans, p, p + step,
-                               g_tlsm ? 1 : 0, g_c_zero);
-        };
-        if (L.par_temp) go(k_gf_tile<true>);
-        else go(k_gf_tile<false>);
-    }
+    long tiles = 0;
+    for (const GfPlan& q : plans.p) tiles += q.tiles;
+    const unsigned nb = (unsigned)std::max(8L, std::min(tiles, 512L));
+    auto go = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3(nb), dim3(256), 0, ctx().stream, (const double2*)g_gf_rec.p, gauge_ptrs(u),
+                           (double2*)g_gf_part.p, link_geom(), plans, g_c_zero);
+    };
+    if (ctx().lat.par_temp) go(k_gf_tile<true>);
+    else go(k_gf_tile<false>);
     return hip_ok(hipGetLastError(), "k_gf_tile");
 }
 bool gf_ipdot(void* ipdot, void* mom, double fact) {
@@ -1803,7 +1785,7 @@ bool gf_move(void* mom, double fact, double delta) {
 bool launch_gauge_force(const void* u, void* stap, void* ipdot, void* mom, double fact) {
     const Lattice& L = ctx().lat;
     if (!gf_size_ok()) return fail("gauge force: lattice too large (sizeh %ld)", (long)L.sizeh);
-    if (gf_planes_ready()) return gf_pack(u) && gf_parts(u, stap) && gf_ipdot(ipdot, mom, fact);
+    if (!stap && gf_planes_ready(false)) return gf_pack(u) && gf_parts(u) && gf_ipdot(ipdot, mom, fact);
     // whole blocks per link array (the kernel takes the direction from the block)
     const int nb = 8 * (int)((L.sizeh + kGfLinks - 1) / kGfLinks);
     hipLaunchKernelGGL(k_gauge_force, dim3(nb), dim3(3 * kGfLinks), 0, ctx().stream, gauge_ptrs(u), (double2*)stap,
@@ -2020,7 +2002,7 @@ double calc_rettangolo_soloopenacc(const su3_soa* tconf_acc, su3_soa* local_plaq
 // library stream), with the fused momentum step when mom is not null
 int ostp_set_gauge_force_kernel(int planes) {
     const int prev = g_gf_planes;
-    g_gf_planes = planes ? 1 : 0;
+    g_gf_planes = planes == 2 ? 2 : planes ? 1 : 0;
     return prev;
 }
 

@@ -17,6 +17,7 @@ namespace {
 bool solves_end = true;
 int stop, iterations;        // (not 0) a CG converges in that many; launched
 std::string gone;            // kernels that were given memory that is no longer there
+int tiles, links;            // launches of the gauge force's plane and per-link kernels
 int with_qa, with_hops;      // launches that took a kept QA; that formed D_oe of solutions
 
 void* arg(void** args, int i) {
@@ -68,9 +69,12 @@ extern "C" void on_launch(const char* kernel, void** args) {
     } else if (is("k_sigma")) {
         used("k_sigma", arg(args, 1));
         used("k_sigma", arg(args, 2));
-    } else if (is("k_gf_tile")) {
+    } else if (is("k_gf_tile")) {  // records, links, parts
+        tiles++;
         used("k_gf_tile", arg(args, 0));
-        used("k_gf_tile", arg(args, 4));
+        used("k_gf_tile", arg(args, 2));
+    } else if (is("k_gauge_force")) {
+        links++;
     } else if (is("k_ms_verifyILi1E")) {
         // u[8], ph[8], x[8], m2[8], n, h
         const char* v = (const char*)args[0];
@@ -110,6 +114,7 @@ struct Fields {
         }
     }
     void gauge_force() {
+        ostp_set_gauge_force_kernel(2);  // whose work space this is about
         ostp_time_gauge_force((su3_soa*)u, nullptr, (tamat_soa*)ip, (thmat_soa*)mom, 0.1, 1);
     }
     void force() {
@@ -194,6 +199,27 @@ int main(int argc, char** argv) {
             for (size_t i = 0; i < kOrder * kVec; i++) zero = zero && !f.xs[i];
             printf("window %d : %s\n", w, zero ? "ok" : "old solutions");
         }
+    } else if (what == "gauge") {
+        // launches of the two kernels: a force with its staples, one without, the integrator's
+        ostp_init(atoi(argv[2]), atoi(argv[3]), atoi(argv[4]), atoi(argv[5]), 0);
+        ostp_set_stout(0.15, 2, 0.0, 0, 0, atoi(argv[6]));
+        ostp_set_gauge_force_kernel(atoi(argv[7]));
+        const size_t sh = ostp_sizeh();
+        su3_soa *u = (su3_soa*)ostp_malloc(8 * 144 * sh), *s = (su3_soa*)ostp_malloc(8 * 144 * sh);
+        tamat_soa* ip = (tamat_soa*)ostp_malloc(512 * sh);
+        thmat_soa* mom = (thmat_soa*)ostp_malloc(512 * sh);
+        md_param md = {};
+        md.no_md = 1, md.gauge_scale = 5, md.t = 1.0;
+        md_parameters = md;
+        initialize_md_global_variables(md);
+        auto count = [&](const char* name, auto call) {
+            tiles = links = 0;
+            call();
+            printf("%s : %d %d %s\n", name, tiles, links, verdict());
+        };
+        count("staples", [&] { calc_ipdot_gauge_soloopenacc(u, s, ip); });
+        count("force", [&] { ostp_time_gauge_force(u, nullptr, ip, nullptr, 0.0, 1); });
+        count("moves", [&] { multistep_2MN_gauge(u, s, ip, mom); });
     } else if (what == "short") {
         // CG solves that take few iterations: how many were queued
         ostp_init(16, 16, 16, 2 * strtol(argv[2], nullptr, 0), 0);  // half-sites: 4096 each

@@ -173,17 +173,17 @@ def test_staple_is_action_derivative(tlsm, par_temp, shape):
 @pytest.mark.parametrize("shape", [(8, 8, 8, 8), (4, 8, 4, 12), (8, 12, 4, 8)])
 @pytest.mark.parametrize("tlsm,par_temp", [(1, 0), (0, 0), (1, 1)])
 def test_plane_kernels_match_link_kernel(shape, tlsm, par_temp):
-    """The per-plane kernels (links of a tile in LDS; the force without
-    staples, as in the MD) against the per-link kernel: ipdot and the fused
-    momentum step mom -= i fact ipdot, over every tile shape (8 or 4 sites
-    along each direction) with and without the PAR_TEMP coefficients."""
+    """The per-plane kernel (links of a tile in LDS; the force without
+    staples, as in the MD) where it is chosen (1) and wherever it can be used
+    (2) against the per-link kernel (0): ipdot and the fused momentum step
+    mom -= i fact ipdot, with and without the PAR_TEMP coefficients."""
     f = Field(shape, bool(par_temp), 9)
     set_action(tlsm)
     init_lattice(f.shape, par_temp=f.pt)
     du = Dev(f.u)
     mom0 = np.random.default_rng(3).standard_normal(8 * 8 * f.sizeh)
     outs = []
-    for planes, with_staples in ((0, True), (1, True), (1, False)):
+    for planes, with_staples in ((0, True), (1, True), (1, False), (2, True), (2, False)):
         prev = lib.ostp_set_gauge_force_kernel(planes)
         dt, dm = Dev(nbytes=8 * 64 * f.sizeh), Dev(mom0)
         ds = Dev(nbytes=8 * f.per) if with_staples else None
@@ -194,20 +194,22 @@ def test_plane_kernels_match_link_kernel(shape, tlsm, par_temp):
         outs.append((dt.get(np.zeros(8 * 8 * f.sizeh)), dm.get(np.zeros(8 * 8 * f.sizeh)) - mom0,
                      staple_planes(f, ds.get(np.zeros(8 * f.per, dtype=np.uint8))) if ds else None))
     assert np.abs(outs[0][0]).max() > 0.1
-    for k in (1, 2):
+    for k in (1, 2, 3, 4):
         assert rel(outs[k][0], outs[0][0]) < 1e-13
         assert rel(outs[k][1], outs[0][1]) < 1e-13
-    assert rel(outs[1][2], outs[0][2]) < 1e-13
+        if outs[k][2] is not None:
+            assert rel(outs[k][2], outs[0][2]) < 1e-13
 
 
 @pytest.mark.parametrize("shape", [(2, 2, 2, 2), (4, 4, 4, 4), (6, 10, 14, 2), (18, 14, 10, 6), (22, 2, 26, 4),
                                    (32, 4, 16, 6), (8, 3, 4, 4)])
 @pytest.mark.parametrize("tlsm,par_temp", [(1, 0), (0, 0), (1, 1)])
 def test_plane_tiles_match_link_kernel(shape, tlsm, par_temp):
-    """The plane kernel on extents that its tiles divide and on those they
-    overhang, wrap onto themselves (extent 2) or leave to the per-link kernel
-    (an odd extent): the force with and without staples and a whole gauge
-    sub-integrator against the per-link kernel.  Both kernels round each link's
+    """The plane kernel (chosen, 1, and wherever it can be used, 2) on extents
+    that its tiles divide and on those they overhang, wrap onto themselves
+    (extent 2) or leave to the per-link kernel (an odd extent): the force with
+    and without staples and a whole gauge sub-integrator against the per-link
+    kernel.  Both kernels round each link's
     84-link sum differently, a few units of 2^-53 of its largest terms: 1e-13;
     the five steps of the integrator carry that along: 1e-12."""
     f = Field(shape, bool(par_temp), 9)
@@ -220,7 +222,7 @@ def test_plane_tiles_match_link_kernel(shape, tlsm, par_temp):
     C.memmove(C.addressof(ost.MdParam.in_dll(lib, "md_parameters")), C.addressof(md), C.sizeof(md))
     lib.initialize_md_global_variables(md)
     outs = []
-    for planes in (0, 1):
+    for planes in (0, 1, 2):
         prev = lib.ostp_set_gauge_force_kernel(planes)
         du, dt, dm, ds = Dev(f.u), Dev(nbytes=8 * n), Dev(mom0), Dev(nbytes=8 * f.per)
         zero = np.zeros(8 * f.per, dtype=np.uint8)
@@ -235,5 +237,6 @@ def test_plane_tiles_match_link_kernel(shape, tlsm, par_temp):
         ost.check(0, "gauge force")
         outs.append(got)
     assert np.abs(outs[0][0]).max() > 0.1
-    for k, (a, b) in enumerate(zip(*outs)):
-        assert rel(a, b) < (1e-13 if k < 4 else 1e-12), k
+    for got in outs[1:]:
+        for k, (a, b) in enumerate(zip(got, outs[0])):
+            assert rel(a, b) < (1e-13 if k < 4 else 1e-12), k

@@ -82,3 +82,22 @@ def test_short_solves_queue_few_iterations(run, tens, first):
         stop, queued = map(int, k.split())
         assert int(v) == stop
         assert queued <= (first if stop <= first else stop + 4), (stop, queued)
+
+
+@pytest.mark.parametrize("shape,tlsm,mode,force,moves", [
+    ((8, 8, 8, 8), 1, 1, False, True), ((10, 10, 10, 10), 1, 1, False, True), ((16, 16, 16, 4), 1, 1, True, True),
+    ((12, 18, 4, 14), 1, 1, False, True), ((16, 16, 16, 2), 1, 1, False, False), ((10, 10, 10, 8), 1, 1, False, False),
+    ((64, 64, 2, 2), 1, 1, False, False), ((64, 64, 2, 2), 1, 2, True, True), ((8, 3, 4, 4), 1, 2, False, False),
+    ((16, 16, 16, 8), 0, 1, False, False), ((16, 16, 16, 8), 0, 2, False, False), ((16, 16, 16, 8), 1, 0, False, False),
+])
+def test_gauge_force_kernels(run, shape, tlsm, mode, force, moves):
+    """Which kernel forms the gauge force: by planes where that is faster or,
+    asked for, possible; by links with the Wilson action, an odd extent, few
+    sites a tile, and always where the staples are asked for (the integrator's
+    last force)."""
+    got = run("gauge", *shape, tlsm, mode)
+    assert got["staples"] == "0 1 ok"
+    f, m = ([int(v) for v in got[k].split()[:2]] for k in ("force", "moves"))
+    assert all(v.endswith(" ok") for v in got.values())
+    assert (f[0] > 0, f[1] > 0) == (force, not force)
+    assert m == ([10, 1] if moves else [0, 11])
