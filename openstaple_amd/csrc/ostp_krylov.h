@@ -76,27 +76,7 @@ struct KrArgs {
     int n, tmajor, rev;
 };
 
-// sum of n partials by T threads (a wave; a block, for whom the thousands of a
-// large lattice are one round of loads), in the same order wherever it runs:
-// kr_part a thread's share, kr_wave the wave's total, kr_block the block's
-template <int T = 64>
-__device__ __forceinline__ double kr_part(const double* __restrict__ part, int n, int stride, int thread) {
-    double v = 0.0;
-    int i = thread;
-    for (; i + 7 * T < n; i += 8 * T) {
-        double t[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) t[q] = part[(long)(i + T * q) * stride];
-#pragma unroll
-        for (int q = 0; q < 8; q++) v += t[q];
-    }
-    double t[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) t[q] = i + T * q < n ? part[(long)(i + T * q) * stride] : 0.0;
-#pragma unroll
-    for (int q = 0; q < 8; q++) v += t[q];
-    return v;
-}
+// sums of partials (part_sum): kr_wave a wave's total, kr_block the block's
 __device__ __forceinline__ double kr_wave(double v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -126,7 +106,7 @@ __device__ __forceinline__ void kr_end(const KrArgs& a, int k, int lane, bool st
     SolverState* prev = a.st[k] + ((a.j - 1) & 1);
     // every load is issued before the first wait
     double sum = 0.0;
-    if (a.j > 1 && !total) sum = kr_part(a.partB[k], a.nB, 1, lane);
+    if (a.j > 1 && !total) sum = part_sum(a.partB[k], a.nB, 1, lane);
     const int status0 = prev->status;
     int status = status0, cg = prev->cg, restarted = prev->cg_restarted, maxiter = prev->maxiter;
     double g = 0.0, delta = prev->delta, lambda = prev->lambda;
@@ -514,7 +494,7 @@ __global__ __launch_bounds__(kBlock) void k_kr_p(KrArgs a) {
             pp[q][c] = p[e];
         }
     }
-    const double total = kr_block(a.j > 1 ? kr_part<kBlock>(a.partB[k], a.nB, 1, tid) : 0.0, lds);
+    const double total = kr_block(a.j > 1 ? part_sum<kBlock>(a.partB[k], a.nB, 1, tid) : 0.0, lds);
     if (tid < 64) kr_end(a, k, tid, store, &sh_gamma, &sh_run, sh_k, sh_on, &total);
     __syncthreads();
     if (store && a.ms && sh_on[kMaxShifts] && a.win[k]) kr_window(a.win[k], a.st[k][a.j & 1].order, sh_k, sh_on, tid, kBlock);
@@ -578,7 +558,7 @@ __global__ __launch_bounds__(kBlock) void k_kr_r(KrArgs a) {
             }
         }
     }
-    const double tot = kr_block(kr_part<kBlock>(a.partA[k], a.nA, a.sA, tid), lds);
+    const double tot = kr_block(part_sum<kBlock>(a.partA[k], a.nA, a.sA, tid), lds);
     if (tid < 64) {
         const double delta = st->delta;
         const int running = st->status == kRunning;
@@ -683,8 +663,8 @@ __global__ __launch_bounds__(kBlock) void k_mx_p(MxArgs a) {
             pp[q][c] = a.pf[e];
         }
     }
-    const double sumt = a.tail ? kr_block(kr_part<kBlock>(a.partT, a.nT, 2, tid), ldst) : 0.0;
-    const double sum = kr_block(a.j > 1 ? kr_part<kBlock>(a.partB, a.nB, 1, tid) : 0.0, lds);
+    const double sumt = a.tail ? kr_block(part_sum<kBlock>(a.partT, a.nT, 2, tid), ldst) : 0.0;
+    const double sum = kr_block(a.j > 1 ? part_sum<kBlock>(a.partB, a.nB, 1, tid) : 0.0, lds);
     if (tid < 64) {
         const SolverState* prev = a.st + ((a.j - 1) & 1);
         SolverState* next = a.st + (a.j & 1);
@@ -768,7 +748,7 @@ __global__ __launch_bounds__(kBlock) void k_mx_xr(MxArgs a) {
             sa[q][c] = a.sf[e];
         }
     }
-    const double tot = kr_block(kr_part<kBlock>(a.partA, a.nA, 2, tid), lds);
+    const double tot = kr_block(part_sum<kBlock>(a.partA, a.nA, 2, tid), lds);
     if (tid < 64) {
         const int go = st->status == kRunning && !st->hold, ru = st->ru;
         const double om = st->delta / tot;

@@ -39,3 +39,26 @@ def test_windows_do_not_depend_on_batch_ends(lines, form):
 
 def test_full_window_takes_no_step(lines):
     assert lines["full"] == "agree"
+
+
+def test_partial_sums_keep_their_order(tmp_path):
+    """part_sum adds a thread's partials one after the other, whatever their
+    number: bit for bit the plain loop."""
+    src = tmp_path / "part.cpp"
+    src.write_text(r"""
+#include "ostp_reduce.h"
+int main() {
+    std::vector<double> p(40000);
+    for (size_t i = 0; i < p.size(); i++) p[i] = sin(1.0 + i) * pow(10.0, (int)(i % 7) - 3);
+    for (int n : {0, 1, 63, 64, 255, 256, 257, 2047, 2048, 2049, 8192, 8197, 19999})
+        for (int stride : {1, 2})
+            for (int t = 0; t < 256; t++) {
+                double v = 0.0;
+                for (int i = t; i < n; i += 256) v += p[(size_t)i * stride];
+                if (ostp::part_sum<256>(p.data(), n, stride, t) != v) return 1;
+            }
+    return 0;
+}
+""")
+    build_host(src, tmp_path / "part")
+    subprocess.run([str(tmp_path / "part")], check=True)
