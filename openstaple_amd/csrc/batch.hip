@@ -348,7 +348,8 @@ __device__ __forceinline__ void chunk_partials(const double (&v)[NR], const bool
 // --------------------------------------- FP32/FP64 hops, several systems
 // Systems of a batch that share a gauge field (noise sources on one
 // configuration, the shifts of a rational solve) form chunks of up to
-// kMrSystems, taken NR at a time; a
+// kMrSystems, taken NR at a time (FP64: four or eight, whichever the autotuner
+// finds faster); a
 // chunk's workgroup computes the hops of all of them (the FP32 inner hops or
 // the FP64 ones): each link (two rows, the rebuilt third, its phase) is
 // loaded and prepared once per half-site and applied to the NR systems'
@@ -972,7 +973,8 @@ __global__ __launch_bounds__(kBlock) void kb_finalize(const BSys* __restrict__ s
 // the reliable updates are tuned separately
 struct Tile {
     int blk = 256;
-    int order = 1;   // bits 0-2 as in kb_dslash; bit 3: FP64 hops by chunks (kb_dslash_mr)
+    int order = 1;   // bits 0-2 as in kb_dslash; bit 3: hops by chunks (kb_dslash_mr); bit 4: by half
+                     // chunks in FP64
     float us = 0.f;
 };
 constexpr int kMrSystems = 8;  // systems per chunk of kb_dslash_mr
@@ -1057,12 +1059,20 @@ static void launch_role(const Tile& t, int nsys, int max_sizeh, int pred) {
                 hipLaunchKernelGGL(kern, dim3(tiles, g_batch.nchunks * (kMrSystems / nr)), dim3(t.blk), 0, S(),
                                    g_batch.dsys, ch, pred, o);
             };
-            // FP64: half chunks leave four waves a SIMD instead of two (twelve systems on
-            // 24^3 x 8, t-fastest: D_oe 48.6 -> 45.2 us, D_eo with the residual 59.1 -> 50.8)
-            constexpr int NR = ROLE >= kRoleF64Doe ? kMrSystems / 2 : kMrSystems;
-            if (t.blk == 64) go(kb_dslash_mr<ROLE, 64, NR>, NR);
-            else if (t.blk == 128) go(kb_dslash_mr<ROLE, 128, NR>, NR);
-            else go(kb_dslash_mr<ROLE, 256, NR>, NR);
+            // FP64: half chunks leave four waves a SIMD instead of two but load a link twice
+            // as often; which wins depends on the lattice and on how the systems fill the
+            // chunks, so the autotuner times both.  Best D_oe of whole against half chunks:
+            // 24^3 x 8 12 systems 49.2, 45.3 us, 16 systems 59.4, 66.1; 24^3 x 12 8 systems
+            // 51.5, 43.4, 10 systems 62.7, 72.1; 32^3 x 16 6 systems 105.8, 129.6; 16^4 16
+            // systems 39.3, 34.4; 32^4 19 systems 630.9, 702.8
+            auto size = [&](auto nr) {
+                constexpr int NR = decltype(nr)::value;
+                if (t.blk == 64) go(kb_dslash_mr<ROLE, 64, NR>, NR);
+                else if (t.blk == 128) go(kb_dslash_mr<ROLE, 128, NR>, NR);
+                else go(kb_dslash_mr<ROLE, 256, NR>, NR);
+            };
+            if (ROLE >= kRoleF64Doe && (t.order & 16)) size(std::integral_constant<int, kMrSystems / 2>{});
+            else size(std::integral_constant<int, kMrSystems>{});
             return;
         }
     }
@@ -1112,10 +1122,13 @@ static std::string signature(const std::vector<BSys>& v) {
 }
 
 // Time each candidate tile (64, 128 or 256 threads; t-fastest or contiguous
-// tiles; XCD-contiguous or hardware order; systems one after the other or
-// interleaved) on the batch's inner D_oe (FP32,
+// tiles; XCD-contiguous or hardware order; systems one after the other,
+// interleaved or by chunks) on the batch's inner D_oe (FP32,
 // or FP16 for the FP16 inner solver) and on its FP64 D_oe, three launches
-// each after one warm-up launch; keep the fastest of each.
+// each after one warm-up launch; keep the fastest of each.  The fastest FP64 tile
+// is then held against half chunks over both FP64 hops of a reliable update; they
+// have to win by 5%, as they lose where many systems of a batch have stopped (12
+// shifts refined on 24^4, even when all run: 13.0 ms with whole chunks, 13.3 half).
 static Tile g_forced_tile{0, 0, 0.f};  // blk 0: autotune
 
 static Tiles autotune(const std::string& sig, int nsys, int max_sizeh, bool half) {
@@ -1131,40 +1144,66 @@ static Tiles autotune(const std::string& sig, int nsys, int max_sizeh, bool half
     best.inner.us = best.f64.us = 1e30f;
     std::string rep = "batch " + sig + ":";
     if (!hip_ok(hipEventCreate(&e0), "event") || !hip_ok(hipEventCreate(&e1), "event")) return Tiles{};
-    static const char* const kOrder[16] = {
+    static const char* const kOrder[32] = {
         "contiguous", "t-fastest", "contiguous hw-order", "t-fastest hw-order",
         "contiguous interleaved", "t-fastest interleaved", "contiguous hw-order interleaved",
         "t-fastest hw-order interleaved", "chunks contiguous", "chunks t-fastest", "chunks contiguous hw-order",
         "chunks t-fastest hw-order", "chunks contiguous interleaved", "chunks t-fastest interleaved",
-        "chunks contiguous hw-order interleaved", "chunks t-fastest hw-order interleaved"};
+        "chunks contiguous hw-order interleaved", "chunks t-fastest hw-order interleaved",
+        "", "", "", "", "", "", "", "", "half chunks contiguous", "half chunks t-fastest",
+        "half chunks contiguous hw-order", "half chunks t-fastest hw-order", "half chunks contiguous interleaved",
+        "half chunks t-fastest interleaved", "half chunks contiguous hw-order interleaved",
+        "half chunks t-fastest hw-order interleaved"};
     for (int fam = 0; fam < 2; fam++) {
         rep += fam == 0 ? " inner D_oe:" : " fp64 D_oe:";
         Tile& b = fam == 0 ? best.inner : best.f64;
         const int norders = g_batch.shared ? 16 : 8;  // chunked hops only where systems share a field
+        auto timed = [&](Tile& keep, Tile c, const char* what, auto one) {
+            one();
+            (void)hipEventRecord(e0, S());
+            for (int r = 0; r < 3; r++) one();
+            (void)hipEventRecord(e1, S());
+            (void)hipEventSynchronize(e1);
+            float ms = 0.f;
+            (void)hipEventElapsedTime(&ms, e0, e1);
+            c.us = 1000.f * ms / 3;
+            char buf[96];
+            snprintf(buf, sizeof buf, " [%d thr, %s%s] %.1f us", c.blk, kOrder[c.order], what, c.us);
+            rep += buf;
+            if (c.us < keep.us) keep = c;
+        };
         for (int blk : {256, 128, 64})
             for (int order = 0; order < norders; order++) {
                 Tile c;
                 c.blk = blk;
                 c.order = order;
-                auto one = [&]() {
+                timed(b, c, "", [&]() {
                     if (fam == 1) launch_role<kRoleF64Doe>(c, nsys, max_sizeh, kAlways);
                     else if (half && g_sgn) launch_role<kRoleS16Doe>(c, nsys, max_sizeh, kAlways);
                     else if (half) launch_role<kRoleH16Doe>(c, nsys, max_sizeh, kAlways);
                     else launch_role<kRoleF32Doe>(c, nsys, max_sizeh, kAlways);
-                };
-                one();
-                (void)hipEventRecord(e0, S());
-                for (int r = 0; r < 3; r++) one();
-                (void)hipEventRecord(e1, S());
-                (void)hipEventSynchronize(e1);
-                float ms = 0.f;
-                (void)hipEventElapsedTime(&ms, e0, e1);
-                c.us = 1000.f * ms / 3;
-                char buf[96];
-                snprintf(buf, sizeof buf, " [%d thr, %s] %.1f us", c.blk, kOrder[c.order], c.us);
-                rep += buf;
-                if (c.us < b.us) b = c;
+                });
             }
+        if (fam == 1 && g_batch.shared) {
+            auto pair = [&](Tile& keep, const Tile& c) {
+                timed(keep, c, ", both hops", [&]() {
+                    launch_role<kRoleF64Doe>(c, nsys, max_sizeh, kAlways);
+                    if (half) launch_role<kRoleF64DeoResid>(c, nsys, max_sizeh, kAlways);
+                    else launch_role<kRoleF64Deo>(c, nsys, max_sizeh, kAlways);
+                });
+            };
+            Tile h;
+            b.us = h.us = 1e30f;
+            pair(b, Tile(b));
+            for (int blk : {256, 128, 64})
+                for (int order : {24, 25, 28, 29}) {
+                    Tile c;
+                    c.blk = blk;
+                    c.order = order;
+                    pair(h, c);
+                }
+            if (1.05f * h.us < b.us) b = h;
+        }
         char buf[96];
         snprintf(buf, sizeof buf, " -> %d thr %s;", b.blk, kOrder[b.order]);
         rep += buf;
@@ -1600,9 +1639,10 @@ int ostp_batched_half_solve(int nsys, const ostp_batch_system* sys, double res, 
 }
 
 int ostp_set_batch_tile(int blk, int order) {
-    if (blk != 0 && ((blk != 64 && blk != 128 && blk != 256) || order < 0 || order > 15)) {
-        fail("ostp_set_batch_tile: workgroup %d / order %d (64, 128 or 256 and 0..15, or 0 for the autotuner)", blk,
-             order);
+    if (blk != 0 &&
+        ((blk != 64 && blk != 128 && blk != 256) || order < 0 || order > 31 || (order & 24) == 16)) {
+        fail("ostp_set_batch_tile: workgroup %d / order %d (64, 128 or 256 and 0..15 or 24..31, or 0 for the "
+             "autotuner)", blk, order);
         return -1;
     }
     const int prev = g_forced_tile.blk ? g_forced_tile.blk * 16 + g_forced_tile.order : 0;

@@ -148,7 +148,7 @@ def test_tile_choices_agree(half):
     cg0, _ = run()
     try:
         for blk in (64, 128, 256):
-            for tfast in (0, 1, 8, 9):  # bit 3: hops of up to eight systems per thread
+            for tfast in (0, 1, 8, 9, 24, 25):  # bit 3: up to eight systems per thread; bit 4: four in FP64
                 first = None
                 for order in (tfast, tfast | 2, tfast | 4, tfast | 6):
                     assert lib.ostp_set_batch_tile(blk, order) >= 0
@@ -165,7 +165,8 @@ def test_tile_choices_agree(half):
                             assert np.array_equal(x1[k], first[1][k]), (blk, order, k)
     finally:
         lib.ostp_set_batch_tile(0, 0)
-    assert lib.ostp_set_batch_tile(96, 0) == -1
+    for blk, order in ((96, 0), (64, 16), (64, 32), (64, -1)):
+        assert lib.ostp_set_batch_tile(blk, order) == -1
     assert lib.ostp_last_error()
     lib.ostp_clear_error()
     assert lib.ostp_set_batched_graph_iterations(-1) == -1
