@@ -1174,6 +1174,8 @@ static Tiles autotune(const std::string& sig, int nsys, int max_sizeh, bool half
         };
         for (int blk : {256, 128, 64})
             for (int order = 0; order < norders; order++) {
+                // one system after the other in hardware order: not worth its time where chunks are tried as well
+                if (fam == 1 && norders == 16 && (order & 10) == 2) continue;
                 Tile c;
                 c.blk = blk;
                 c.order = order;
@@ -1195,13 +1197,12 @@ static Tiles autotune(const std::string& sig, int nsys, int max_sizeh, bool half
             Tile h;
             b.us = h.us = 1e30f;
             pair(b, Tile(b));
-            for (int blk : {256, 128, 64})
-                for (int order : {24, 25, 28, 29}) {
-                    Tile c;
-                    c.blk = blk;
-                    c.order = order;
-                    pair(h, c);
-                }
+            for (int order : {24, 28}) {
+                Tile c;
+                c.blk = b.blk;
+                c.order = order | (b.order & 1);
+                pair(h, c);
+            }
             if (1.05f * h.us < b.us) b = h;
         }
         char buf[96];
