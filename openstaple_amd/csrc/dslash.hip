@@ -160,11 +160,14 @@ __global__ __launch_bounds__(64 * kSplitWaves) void k_dslash_split(DslashArgs<R>
 // exchange through LDS costs more than the shorter chain gives; the line is that of
 // the fused solver iterations, so that a solver's sums have one order on either
 // side of it.  FP32 11.7 -> 7.8
-// at 2048, 25.7 -> 23.8 at 154440 and still 78.7 -> 74.5 at 524288 (half the
-// bytes a site).  Two or four waves a site lie between.
+// at 2048, 25.7 -> 23.8 at 154440, 78.7 -> 74.5 at 524288 (half the bytes a site)
+// and 243 -> 235 on 48^3 x 24 (1.3 million); then the gain goes: 361 -> 365 on
+// 64^3 x 14, 378 -> 393 on 128 x 32^3, 380 -> 373 on 64^3 x 16, 688 -> 697 on
+// 56^3 x 40, 826 -> 874 on 64^3 x 32.  Two or four waves a site lie between.
+constexpr long kHopSplitSizehF32 = 3L << 19;
 template <typename R>
 static bool dslash_split() {
-    return sizeof(R) == 4 || ctx().lat.sizeh <= kHopSplitSizeh;
+    return ctx().lat.sizeh <= (sizeof(R) == 4 ? kHopSplitSizehF32 : kHopSplitSizeh);
 }
 template <typename R>
 int dslash_blocks() {
@@ -176,16 +179,15 @@ template int dslash_blocks<float>();
 template <typename R, int EO, int MODE>
 static void go(const DslashArgs<R>& a) {
     const dim3 blocks(dslash_blocks<R>());
-    if constexpr (sizeof(R) == 8)
-        if (!dslash_split<R>()) {
-            if constexpr (MODE == kPlain || MODE == kMdagMDot)
-                if (a.sg) {
-                    hipLaunchKernelGGL((k_dslash<R, EO, MODE, true>), blocks, dim3(kBlock), 0, ctx().stream, a);
-                    return;
-                }
-            hipLaunchKernelGGL((k_dslash<R, EO, MODE>), blocks, dim3(kBlock), 0, ctx().stream, a);
-            return;
-        }
+    if (!dslash_split<R>()) {
+        if constexpr (sizeof(R) == 8 && (MODE == kPlain || MODE == kMdagMDot))
+            if (a.sg) {
+                hipLaunchKernelGGL((k_dslash<R, EO, MODE, true>), blocks, dim3(kBlock), 0, ctx().stream, a);
+                return;
+            }
+        hipLaunchKernelGGL((k_dslash<R, EO, MODE>), blocks, dim3(kBlock), 0, ctx().stream, a);
+        return;
+    }
     hipLaunchKernelGGL((k_dslash_split<R, EO, MODE>), blocks, dim3(64 * kSplitWaves), 0, ctx().stream, a);
 }
 

@@ -207,3 +207,28 @@ def test_hops_at_block_edges(shape):
     lib.acc_Doe_f(duf.p, doutf.p, dpsif.p, dpf.p)
     ost.check(0, "acc_Doe_f")
     assert rel(doutf.get(psif), o.doe_f(uf, psif, phf)) < TOL32
+
+
+@pytest.mark.parametrize("shape", [(64, 64, 64, 12), (64, 64, 64, 14)])
+def test_large_fp32_hops(shape):
+    """The FP32 hops up to 1.5 x 2^20 half-sites (split over waves) and above
+    (a thread a site) against the FP64 hops of the same fields."""
+    L = init_lattice(shape)
+    vb, gb, sh = L.vec3_bytes, 8 * L.su3_bytes, L.sizeh
+    u, uf, ph, phf = (Dev(nbytes=n) for n in (gb, gb // 2, 64 * sh, 32 * sh))
+    x, y, z = (Dev(nbytes=vb) for _ in range(3))
+    xf, yf, zf, tf = (Dev(nbytes=vb // 2) for _ in range(4))
+    lib.ostp_generate_Conf_cold(u.p, 0.7, 3)
+    lib.ostp_convert_double_to_float_gauge(u.p, uf.p)
+    lib.calc_u1_phases(ph.p, ost.BfParam(0, 0, 0, 0, 0, 0), 0.0, 0.0)
+    phf.put(ph.get(np.zeros(8 * sh)).astype(np.float32))
+    lib.ostp_generate_vec3_soa_gauss(x.p, 5, 1)
+    lib.convert_double_to_float_vec3_soa(x.p, xf.p)
+    fp = ost.ferm_param(0.05, ph.p, phf.p)
+    lib.fermion_matrix_multiplication_shifted(u.p, y.p, x.p, z.p, C.byref(fp), 0.013)
+    lib.fermion_matrix_multiplication_shifted_f(uf.p, yf.p, xf.p, tf.p, C.byref(fp), 0.013)
+    lib.acc_Doe_f(uf.p, zf.p, xf.p, phf.p)
+    ost.check(0, "hops")
+    like, likef = np.zeros(3 * sh, dtype=np.complex128), np.zeros(3 * sh, dtype=np.complex64)
+    for f, d in ((yf, y), (zf, z), (tf, z)):
+        assert rel(f.get(likef), d.get(like)) < TOL32
