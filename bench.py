@@ -781,7 +781,8 @@ def run_rhmc(ost, lib, args):
                       "of the shifts above the tolerance; heat bath and acceptance (1e-10) FP64 CG-M",
         }
     out["gauge_force"] = {
-        "kernel": "k_gauge_force (tree-level Symanzik staples + TA(U S))",
+        "kernel": "calc_ipdot_gauge without the staples kept: k_gf_pack + k_gf_tile + k_gf_ipdot "
+                  "(tree-level Symanzik staples + TA(U S); all its launches)",
         "us_per_launch": round(us_force, 1),
         "us_per_launch_with_momentum_step": round(us_force_mom, 1),
         "flops_per_link": GAUGE_FORCE_FLOPS_PER_LINK,
