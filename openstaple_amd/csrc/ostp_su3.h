@@ -43,7 +43,7 @@ __device__ __forceinline__ double2 cdet2_conj(double2 a, double2 b, double2 c, d
 // rebuild3row (single_types.h:45-50): row2 = conj(row0 x row1), 24 multiply-adds
 // (as differences of complex products it was 30, and the staple kernels
 // rebuild a row for nearly every product: stout smearing of two levels at
-// 48^3x12 1.90 -> 1.55 ms)
+// 48^3x12 1.92 -> 1.59 ms)
 __device__ __forceinline__ void rebuild3row(Su3& m) {
     m.c[2][0] = cdet2_conj(m.c[0][1], m.c[1][2], m.c[0][2], m.c[1][1]);
     m.c[2][1] = cdet2_conj(m.c[0][2], m.c[1][0], m.c[0][0], m.c[1][2]);

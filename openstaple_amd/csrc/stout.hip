@@ -618,8 +618,8 @@ __global__ __launch_bounds__(3 * kGfLinks, 2) void k_gauge_force(GaugePtrs G, do
 // the plan, 2900 for the term-by-term sides), 52% of the issue slots at the
 // 2.1 GHz the card holds; LDS and two blocks per CU leave two waves per SIMD.
 // 48^3x12: 1.85 ms per force, 2.4 ms with the records' and the force's passes
-// (term-by-term sides, six launches: 3.1 ms); gauge sub-integrator 38.8 -> 28
-// ms.  Tried and slower: summing the sides of both directions in two waves
+// (term-by-term sides, six launches: 3.1 ms); gauge sub-integrator, whose last
+// force goes by links, 39.0 -> 27.8 ms.  Tried and slower: summing the sides of both directions in two waves
 // that the second staple pass spares (more exchange through LDS, 2.0 ms).
 // Entry e (of six: rows 0, 1) of the LDS arrays' record r is pool[e kGfPool +
 // r]: an operand's six reads share one address with constant offsets, and
